@@ -466,7 +466,7 @@ namespace {
 template <class F>
 int guarded(hpq_ctx* c, F&& f) {
     // the caller may have changed the particle arrays since the last call
-    if (c) c->cl_plasma.valid = false;
+    if (c) c->ord_plasma.valid = false;
     try {
         f();
         return HPQ_OK;
@@ -537,7 +537,7 @@ void plasma_save(hpq_ctx* c, const hpq_plasma* p, PlasmaBuf& b) {
 }
 
 void plasma_restore(hpq_ctx* c, const PlasmaBuf& b, const hpq_plasma* p) {
-    c->cl_plasma.valid = false;
+    c->ord_plasma.valid = false;
     double* a[PLASMA_REALS];
     plasma_reals(p, a);
     for (int k = 0; k < PLASMA_REALS; ++k)
@@ -813,7 +813,7 @@ void hpq_destroy(hpq_ctx* c) {
     poisson_free(c);
     mg_free(c);
     bins_free(c);
-    cell_lists_free(c->cl_plasma);
+    plasma_order_free(c->ord_plasma);
     cell_lists_free(c->cl_beam);
     init_scratch_free(c);
     if (c->relb_rows) (void)hipFree(c->relb_rows);

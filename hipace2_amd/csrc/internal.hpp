@@ -169,10 +169,25 @@ struct Bins {
     bool reordered = false;      // the plasma was reordered since the step began
 };
 
-// Per-start-cell particle lists of the ordered deposition (gather.hip): list offsets over a
-// grid of base cells, the particles of every list by increasing index, and the per-particle
-// values the contributions need. valid/base/x/n name the plasma state the lists describe, so
-// the explicit deposition can reuse the lists of the current deposition on the same state.
+// Records, cells and cell bounding boxes of the plasma in index order (ordered.hip). valid,
+// base, x, n name the plasma state they describe, so the explicit deposition can reuse those of
+// the current deposition on the same state.
+struct PlasmaOrder {
+    double* rec = nullptr;
+    uint32_t* cell = nullptr;
+    int32_t* boxes = nullptr;
+    int32_t *count = nullptr, *list = nullptr;   // runs of particles listed per gather block
+    long rec_cap = 0, cell_cap = 0, boxes_cap = 0, count_cap = 0, list_cap = 0;
+    int pick = 0;                                // the set of counts in use
+    bool valid = false;
+    int base = -1;
+    const double* x = nullptr;
+    long n = 0;
+};
+
+// Per-start-cell particle lists of the beam's ordered deposition (gather.hip): list offsets
+// over a grid of base cells, the particles of every list by increasing index, and the
+// per-particle values the contributions need.
 struct CellLists {
     int bxlo = 0, bylo = 0, wx = 0, wy = 0;
     int T = 32, ntx = 1, nty = 1;
@@ -180,19 +195,12 @@ struct CellLists {
     long off_cap = 0, tmp_cap = 0, key_cap = 0, slot_cap = 0, unsorted_cap = 0, perm_cap = 0;
     double* rec = nullptr;
     long rec_cap = 0;
-    int32_t* ovf = nullptr;      // overflow lists of the staged gathers
-    long ovf_cap = 0;
-    bool explicit_ovf_clear = false;   // the explicit deposition's overflow count is zero
-    // the beam's per-cell contribution sequences: segment offsets per plane cell, their scan
-    // scratch, the contributions (3 arrays), the cells summed by a wavefront each
+    // the per-cell contribution sequences: segment offsets per plane cell, their scan scratch,
+    // the contributions (3 arrays), the cells summed by a wavefront each
     int32_t *seg = nullptr, *segtmp = nullptr, *longc = nullptr;
     long seg_cap = 0, segtmp_cap = 0, longc_cap = 0;
     double* contrib = nullptr;
     long contrib_cap = 0;
-    bool valid = false;
-    int base = -1;
-    const double* x = nullptr;
-    long n = 0;
 };
 
 // Scratch of the plasma injection: per-cell particle counts and their exclusive scan.
@@ -253,7 +261,7 @@ struct hpq_ctx {
     hpq::Poisson ps;
     hpq::MultiGrid mg;
     hpq::Bins bins;
-    hpq::CellLists cl_plasma;        // ordered deposition of the plasma (main stream)
+    hpq::PlasmaOrder ord_plasma;     // ordered deposition of the plasma (main stream)
     hpq::CellLists cl_beam;          // ordered deposition of the beam (either stream)
     hpq::InitScratch init;
     double* relb_rows = nullptr;     // row sums of ComputeRelBFieldError (2 * ny)
@@ -373,6 +381,7 @@ void deposit_current_ordered(hpq_ctx* c, const hpq_plasma* p, double* store, con
 void explicit_deposition_ordered(hpq_ctx* c, const hpq_plasma* p, double* store);
 void deposit_beam_ordered(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps,
                           const int32_t* select, int select_value);
+void plasma_order_free(PlasmaOrder& L);
 void cell_lists_free(CellLists& L);
 void sort_beam_slices(hpq_ctx* c, hpq_beam_state* b, int64_t* off_out);
 void deposit_vjp(hpq_ctx* c, const hpq_plasma* p, const double* adj, const int32_t* comps, hpq_plasma_adj* a);

@@ -299,7 +299,7 @@ void push_plasma_f32(hpq_ctx* c, const hpq_plasma* p, const double* store, doubl
 
 #ifndef HPQ_F32_TU
 void advance_plasma(hpq_ctx* c, const hpq_plasma* p, const double* store, bool temp_slice) {
-    c->cl_plasma.valid = false;   // positions change: the deposition lists are out of date
+    c->ord_plasma.valid = false;   // positions change: the deposition records are out of date
     if (p->n <= 0) return;
     const Layout& L = c->L;
     const double qmc = c->p.plasma_charge / (c->p.plasma_mass * 1.0);
@@ -466,7 +466,7 @@ int64_t plasma_count(hpq_ctx* c, const hpq_plasma_profile* prof) {
 }
 
 void init_plasma(hpq_ctx* c, const hpq_plasma_profile* prof, const hpq_plasma* p) {
-    c->cl_plasma.valid = false;
+    c->ord_plasma.valid = false;
     const Prof pr = make_prof(c, prof);
     const Geom& g = c->g;
     const long ncell = long(g.nx) * g.ny;
