@@ -66,6 +66,7 @@ struct DstPlan {
     bool fft = false;   // power-of-two FFT in LDS, else direct sum with a sine table
     double2* tw = nullptr;    // M/2 twiddles exp(-2 pi i k / M)
     double* sintab = nullptr; // 2N entries sin(pi m / N) (direct path)
+    double* mat = nullptr;    // n x n sine matrix (direct path, n <= 2048)
 };
 
 // Dirichlet Poisson solver on one slice (FFTPoissonSolverDirichlet*).

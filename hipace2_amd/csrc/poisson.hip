@@ -11,10 +11,11 @@
 // Row DST, power-of-two n+1: two real rows a, b are packed as a + i b, odd-extended to
 // length M = 2(n+1) and transformed with a radix-2 FFT held in LDS (M <= 4096,
 // 64 KiB). With F = FFT(a + i b), RODFT00(a)_{k-1} = -Im F_k and RODFT00(b)_{k-1} = Re F_k.
-// Other n: direct sum with an exactly reduced sine table, one row per workgroup.
+// Other n: direct sums over the sine matrix in tiles of rows and columns (n <= DST_MAT_MAX), or
+// with an exactly reduced sine table, one row per workgroup.
 #include <cmath>
-
 #include <type_traits>
+#include <utility>
 
 #include "internal.hpp"
 
@@ -224,6 +225,112 @@ __global__ __launch_bounds__(256) void k_dst_rows_direct(Rows in, Rows out, int 
     }
 }
 
+// entry (j, k) of the sine matrix, sin(pi (j + 1) (k + 1) / (n + 1)), from the reduced table
+__global__ __launch_bounds__(256) void k_sine_matrix(int n, const double* __restrict__ tab, double* __restrict__ mat) {
+    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= long(n) * n) return;
+    const long j = t / n, k = t - j * n;
+    mat[t] = tab[(j + 1) * (k + 1) % (2L * (n + 1))];
+}
+
+// The direct transform of a tile of 32 rows and 32 entries: each thread sums 2 x 2 outputs over
+// all j in order, as k_dst_rows_direct does for one (multiply and add rounded separately), with
+// the rows and the matrix staged through LDS 32 j at a time and the next 32 already loading.
+// TRANS: the output goes to [field][entry][row], the rows of the other direction's pass.
+// Bound by FP64 issue and LDS reads: four multiplies and four adds per j and wave take 39
+// cycles, its two 16-byte reads 9 of the CU's. At 384 x 384 (three fields) a pass takes 28.5 us
+// (14.7 us at 256 x 256); one row per workgroup with a table gather per term took 175 us, this
+// tile with each read next to its use 35 us, and 4 x 2 outputs per thread (half the wavefronts,
+// fewer than two per SIMD) 44 us.
+constexpr int DT_TILE = 32, DT_K = 32, DT_T = 256, DT_L = DT_TILE * DT_K / DT_T, JA = 4;
+template <bool TRANS>
+__global__ __launch_bounds__(DT_T) void k_dst_rows_tiled(Rows in, Rows out, int nrows, int n,
+                                                         const double* __restrict__ mat,
+                                                         const double* __restrict__ scale) {
+    __shared__ double2 a2[DT_K][DT_TILE / 2 + 1];
+    __shared__ double2 s2[DT_K][DT_TILE / 2];
+    const int tid = int(threadIdx.x);
+    const int r0 = int(blockIdx.y) * DT_TILE, k0 = int(blockIdx.x) * DT_TILE;
+    const int lx = tid % 32, ly = tid / 32;   // loads: j of a row, or entry of a matrix row
+    const double* row[DT_L];
+#pragma unroll
+    for (int q = 0; q < DT_L; ++q) {
+        const int r = r0 + ly + DT_T / 32 * q;
+        row[q] = r < nrows ? row_ptr(in, r) : nullptr;
+    }
+    double av[DT_L], sv[DT_L];
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int q = 0; q < DT_L; ++q) {
+            av[q] = row[q] && j0 + lx < n ? row[q][j0 + lx] : 0.0;
+            const int j = j0 + ly + DT_T / 32 * q;
+            sv[q] = j < n && k0 + lx < n ? mat[long(j) * n + k0 + lx] : 0.0;
+        }
+    };
+    const int tx = tid % 16, ty = tid / 16;   // sums: entries 2 tx, 2 tx + 1 of rows 2 ty, 2 ty + 1
+    double c[2][2] = {};
+    load(0);
+    for (int j0 = 0; j0 < n; j0 += DT_K) {
+#pragma unroll
+        for (int q = 0; q < DT_L; ++q) {
+            reinterpret_cast<double*>(a2[lx])[ly + DT_T / 32 * q] = av[q];
+            reinterpret_cast<double*>(s2[ly + DT_T / 32 * q])[lx] = sv[q];
+        }
+        __syncthreads();
+        if (j0 + DT_K < n) load(j0 + DT_K);
+        // LDS reads four j ahead of the sums; the fence keeps the compiler from moving each
+        // read next to its use, where it would wait for every one
+        double2 a[2][JA], s[2][JA];
+        auto read = [&](int b, int j) {
+#pragma unroll
+            for (int q = 0; q < JA; ++q) {
+                a[b][q] = a2[j + q][ty];
+                s[b][q] = s2[j + q][tx];
+            }
+        };
+        read(0, 0);
+#pragma unroll
+        for (int j = 0; j < DT_K; j += JA) {
+            const int b = (j / JA) & 1;
+            if (j + JA < DT_K) read(b ^ 1, j + JA);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < JA; ++q) {
+                c[0][0] += a[b][q].x * s[b][q].x;
+                c[0][1] += a[b][q].x * s[b][q].y;
+                c[1][0] += a[b][q].y * s[b][q].x;
+                c[1][1] += a[b][q].y * s[b][q].y;
+            }
+        }
+        __syncthreads();
+    }
+    // through LDS, so that lanes store consecutive addresses
+    double(*t)[DT_TILE + 1] = reinterpret_cast<double(*)[DT_TILE + 1]>(&a2[0][0]);
+    static_assert(sizeof(a2) >= sizeof(double) * DT_TILE * (DT_TILE + 1), "output tile");
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int r = r0 + 2 * ty + p, k = k0 + 2 * tx + q;
+            double o = 2.0 * c[p][q];
+            if (scale && r < nrows && k < n) o *= scale[long(r % in.rows_per_field) * n + k];
+            t[2 * ty + p][2 * tx + q] = o;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < DT_L; ++q) {
+        const int m = ly + DT_T / 32 * q;
+        const int r = r0 + (TRANS ? lx : m), k = k0 + (TRANS ? m : lx);
+        if (r >= nrows || k >= n) continue;
+        if (TRANS) {
+            const int f = r / in.rows_per_field;
+            out.base[f][long(k) * in.rows_per_field + (r - f * in.rows_per_field)] = t[lx][m];
+        } else {
+            row_ptr(out, r)[k] = t[m][lx];
+        }
+    }
+}
+
 // out[f][c][r] = in[f][r][c] for f in [0, nf), in: R x C rows
 __global__ __launch_bounds__(256) void k_transpose(const double* __restrict__ in, double* __restrict__ out, int R,
                                                    int C) {
@@ -241,10 +348,10 @@ __global__ __launch_bounds__(256) void k_transpose(const double* __restrict__ in
     }
 }
 
-// RODFT00 of nrows rows (times the eigenvalue rows when scale != null); sym: followed by
-// the inverse transform of the same rows (fused in LDS on the FFT path)
+// RODFT00 of nrows rows (times the eigenvalue rows when scale != null); sym (FFT path): followed
+// by the inverse transform of the same rows in LDS; trans (matrix path): the output transposed
 static void dst_rows(hpq_ctx* c, const DstPlan& P, const Rows& in, const Rows& out, int nrows, const double* scale,
-                     bool sym = false, const Shift& shift = Shift{}, bool add = false) {
+                     bool sym = false, const Shift& shift = Shift{}, bool add = false, bool trans = false) {
     TraceScope ts(c, HPQ_TRACE_DST);
     if (P.fft) {
         const size_t lds = size_t(P.M) * sizeof(double2);
@@ -256,13 +363,17 @@ static void dst_rows(hpq_ctx* c, const DstPlan& P, const Rows& in, const Rows& o
                                nrows, P.n, P.M, P.logM, P.tw, scale, shift, int(add));
     } else {
         if (shift.parts || add) throw HpqError(HPQ_E_UNSUPPORTED, "shifted DST solve: n + 1 must be a power of two");
-        const size_t lds = size_t(P.n) * sizeof(double);
-        hipLaunchKernelGGL(k_dst_rows_direct, dim3(nrows), dim3(256), lds, c->stream, in, out, P.n, P.sintab, scale);
-        if (sym) {
-            HPQ_HIP(hipGetLastError());
-            // the direct path writes in place row by row: transform out again into in
-            hipLaunchKernelGGL(k_dst_rows_direct, dim3(nrows), dim3(256), lds, c->stream, out, in, P.n, P.sintab,
-                               nullptr);
+        if (P.mat) {
+            const dim3 grid((P.n + DT_TILE - 1) / DT_TILE, (nrows + DT_TILE - 1) / DT_TILE);
+            if (trans)
+                hipLaunchKernelGGL(k_dst_rows_tiled<true>, grid, dim3(DT_T), 0, c->stream, in, out, nrows, P.n, P.mat,
+                                   scale);
+            else
+                hipLaunchKernelGGL(k_dst_rows_tiled<false>, grid, dim3(DT_T), 0, c->stream, in, out, nrows, P.n, P.mat,
+                                   scale);
+        } else {
+            hipLaunchKernelGGL(k_dst_rows_direct, dim3(nrows), dim3(256), size_t(P.n) * sizeof(double), c->stream, in,
+                               out, P.n, P.sintab, scale);
         }
     }
     HPQ_HIP(hipGetLastError());
@@ -277,6 +388,7 @@ static double sin_pi_frac(long m, long N) {
     return sgn * std::sin(M_PI * double(m) / double(N));
 }
 
+constexpr int DST_MAT_MAX = 2048;
 static void plan_init(DstPlan& P, int n) {
     P.n = n;
     P.N = n + 1;
@@ -295,6 +407,13 @@ static void plan_init(DstPlan& P, int n) {
         for (int m = 0; m < 2 * P.N; ++m) tab[m] = sin_pi_frac(m, P.N);
         HPQ_HIP(hipMalloc(&P.sintab, sizeof(double) * tab.size()));
         HPQ_HIP(hipMemcpy(P.sintab, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice));
+        // beyond 2048 the matrix (n^2 doubles, 32 MB there) would leave the caches and grow to
+        // gigabytes: those sizes keep the table
+        if (n <= DST_MAT_MAX) {
+            HPQ_HIP(hipMalloc(&P.mat, sizeof(double) * size_t(n) * n));
+            hipLaunchKernelGGL(k_sine_matrix, grid1d(long(n) * n, 256), dim3(256), 0, nullptr, n, P.sintab, P.mat);
+            HPQ_HIP(hipGetLastError());
+        }
     }
 }
 
@@ -328,7 +447,7 @@ void poisson_init(hpq_ctx* c) {
 
 void poisson_free(hpq_ctx* c) {
     Poisson& S = c->ps;
-    for (void* p : {(void*)S.px.tw, (void*)S.px.sintab, (void*)S.py.tw, (void*)S.py.sintab, (void*)S.eigT,
+    for (void* p : {(void*)S.px.tw, (void*)S.px.sintab, (void*)S.py.tw, (void*)S.py.sintab, (void*)S.px.mat, (void*)S.py.mat, (void*)S.eigT,
                     (void*)S.bufA, (void*)S.bufB, (void*)S.chi_part})
         if (p) (void)hipFree(p);
     dst_mfma_free(c);
@@ -350,24 +469,43 @@ static void solve_fft(hpq_ctx* c, int nf, double* const* lhs_planes, Shift shift
         R.rows_per_field = rpf;
         return R;
     };
-    // x pass on rows j
-    dst_rows(c, S.px, rows(S.bufA, nx, ny), rows(S.bufB, nx, ny), nf * ny, nullptr);
-    hipLaunchKernelGGL(k_transpose, dim3((nx + 31) / 32, (ny + 31) / 32, nf), dim3(32, 8), 0, c->stream, S.bufB,
-                       S.bufA, ny, nx);
-    // y pass, eigenvalue scaling, inverse y pass on rows i (one launch on the FFT path;
-    // the direct path leaves its result in bufA as well)
-    if (S.py.fft)
-        dst_rows(c, S.py, rows(S.bufA, ny, nx), rows(S.bufA, ny, nx), nf * nx, S.eigT, true, shift);
-    else
-        dst_rows(c, S.py, rows(S.bufA, ny, nx), rows(S.bufB, ny, nx), nf * nx, S.eigT, true, shift);
-    hipLaunchKernelGGL(k_transpose, dim3((ny + 31) / 32, (nx + 31) / 32, nf), dim3(32, 8), 0, c->stream, S.bufA,
-                       S.bufB, nx, ny);
+    auto transpose = [&](double* from, double* to, int R, int C) {
+        hipLaunchKernelGGL(k_transpose, dim3((C + 31) / 32, (R + 31) / 32, nf), dim3(32, 8), 0, c->stream, from, to, R, C);
+    };
+    const Shift none{};
+    // x pass on rows j: bufA -> rows i in P
+    double *P, *Q;
+    if (S.px.mat) {
+        dst_rows(c, S.px, rows(S.bufA, nx, ny), rows(S.bufB, ny, nx), nf * ny, nullptr, false, none, false, true);
+        P = S.bufB;
+        Q = S.bufA;
+    } else {
+        dst_rows(c, S.px, rows(S.bufA, nx, ny), rows(S.bufB, nx, ny), nf * ny, nullptr);
+        transpose(S.bufB, S.bufA, ny, nx);
+        P = S.bufA;
+        Q = S.bufB;
+    }
+    // y pass, eigenvalue scaling, inverse y pass on rows i in P (one launch on the FFT path),
+    // leaving rows j in Q
+    if (S.py.fft) {
+        dst_rows(c, S.py, rows(P, ny, nx), rows(P, ny, nx), nf * nx, S.eigT, true, shift);
+        transpose(P, Q, nx, ny);
+    } else {
+        dst_rows(c, S.py, rows(P, ny, nx), rows(Q, ny, nx), nf * nx, S.eigT, false, shift);
+        if (S.py.mat) {
+            dst_rows(c, S.py, rows(Q, ny, nx), rows(P, nx, ny), nf * nx, nullptr, false, none, false, true);
+            std::swap(P, Q);
+        } else {
+            dst_rows(c, S.py, rows(Q, ny, nx), rows(P, ny, nx), nf * nx, nullptr);
+            transpose(P, Q, nx, ny);
+        }
+    }
     // inverse x pass straight into the destination planes
     Rows out;
     for (int f = 0; f < 3; ++f) out.base[f] = lhs_planes[f < nf ? f : 0] + c->g.idx(0, 0);
     out.stride = c->g.ldx;
     out.rows_per_field = ny;
-    dst_rows(c, S.px, rows(S.bufB, nx, ny), out, nf * ny, nullptr, false, Shift{}, add);
+    dst_rows(c, S.px, rows(Q, nx, ny), out, nf * ny, nullptr, false, none, add);
 }
 
 // Solves nfields staged right-hand sides held in ps.bufA as [f][j][i] and writes the
