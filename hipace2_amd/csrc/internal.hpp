@@ -94,7 +94,8 @@ struct MGLevel {
     int ldx = 0, ldy = 0;
     long cs = 0;   // component stride
     double dx = 0, dy = 0;
-    double *acf = nullptr, *res = nullptr, *cor = nullptr, *rescor = nullptr;
+    double facx = 0, facy = 0;   // 1 / dx^2, 1 / dy^2
+    double *acf = nullptr, *c0i = nullptr, *res = nullptr, *cor = nullptr, *rescor = nullptr;
 };
 
 // Convergence state of one solve, kept on the device so V-cycles can be enqueued without
@@ -121,13 +122,14 @@ struct MultiGrid {
     int max_level = 0;
     int coarse_begin = 0;   // first level handled by the single-workgroup coarse kernel
     bool coarse_in_lds = false;
+    int coarse_kp = 1;      // points of a colour per thread on that level
     size_t coarse_lds_bytes = 0;
     int last_iters = 1;     // V-cycles of the previous solve: first batch size of the next
     bool last_zero = false; // the previous solve converged without a V-cycle
     double dx = 0, dy = 0;
     std::vector<MGLevel> lev;
-    alignas(16) unsigned char coarse_args[2048];   // kernel argument block of the coarse kernel
-    double* coarse_work = nullptr;   // coarse-level arrays when they do not fit in LDS
+    alignas(16) unsigned char coarse_args[256];   // kernel argument block of the coarse kernel
+    double* coarse_work = nullptr;   // acf-dependent arrays of the coarse levels, kept for a solve
     double* msol = nullptr;          // level-0 initial guess / odd iterates (copy path, 2 comps)
     double* mrhs = nullptr;          // level-0 right-hand side (copy path, 2 comps)
     MGCtl* d_ctl = nullptr;          // two control blocks, used alternately

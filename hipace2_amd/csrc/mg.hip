@@ -10,21 +10,21 @@
 // norm of the residual (:1330-1416). Every point update uses the reference's operation
 // order, so the iterates equal the CPU build's for equal inputs. The diagonal inverse
 // 1/c0 of a point depends only on acf and the point's position, so it is computed once
-// per launch (fine levels) or per V-cycle (coarse levels) instead of once per sweep.
+// per solve, in the first pass over a level, and kept.
 //
 // Mapping to the GPU: the sweeps (+ residual) of one level are one launch of an LDS-tiled
-// kernel: each workgroup loads its tile plus a halo of NSW + 2 points, runs the NSW
-// colour sweeps in LDS (points NSW or more away from the frozen outer ring see exactly
-// the values a global sweep gives them) and writes back the interior; the residual, its
-// restriction to the next level and its max norm come out of the same launch.
+// kernel: each workgroup loads its tile of one component plus a halo of NSW to NSW + 2
+// points, runs the NSW colour sweeps in LDS (points NSW or more away from the frozen outer
+// ring see exactly the values a global sweep gives them) and writes back the interior; the
+// residual, its restriction to the next level and its max norm come out of the same launch.
 // Prolongation is fused into the load of the up-sweep. On level 0 the up-sweep and the
 // final smoothing of the cycle are one launch of eight sweeps that leaves every
 // workgroup's residual max norm; a one-workgroup launch after it reduces them, evaluates
 // convergence and publishes the result to pinned host memory, which the host polls
-// instead of synchronising the stream. Levels from the first one of at most 33x33
-// points down run as one workgroup that does the coarse part of the V-cycle with barriers
-// between sweeps, its arrays in LDS; the levels of at most 64 points (and the bottom
-// solve) run in its first wavefront alone, without workgroup barriers. For odd n the
+// instead of synchronising the stream. Levels from the first one that fits (65x65 points
+// and the like) down run as one workgroup per component that does the coarse part of the
+// V-cycle with barriers between sweeps, its arrays in LDS; the levels of at most 64 points
+// of a colour run in its first wavefront alone, without workgroup barriers. For odd n the
 // level-0 arrays are the caller's planes themselves (the node-centred level-0 box with
 // its ghost ring has the slice store's guarded shape).
 #include <algorithm>
@@ -38,14 +38,7 @@ namespace hpq {
 
 namespace {
 
-constexpr int TX = 32, TY = 16;                // output tile of the fine-level kernel
-constexpr int NT = 256;                        // threads per workgroup
-constexpr int RW = TX + 2, RH = TY + 2;        // residual region: tile + 1 ring
-constexpr int COARSE_MAX_POINTS = 33 * 33;
-constexpr int CTX = 16, CTY = 32;              // coarse workgroup: CTX x CTY threads
-constexpr int COARSE_THREADS = CTX * CTY;
-constexpr size_t COARSE_LDS_MAX = 150 * 1024;
-constexpr int COARSE_MAX_LEVELS = 16;
+constexpr int NT = 512;                        // threads per workgroup
 
 __host__ __device__ __forceinline__ long at(const MGLevel& L, int i, int j) {
     return long(j - L.jlo + 1) * L.ldx + (i - L.ilo + 1);
@@ -67,6 +60,14 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by) {
 template <class LV>
 __device__ __forceinline__ bool in_valid(const LV& L, int i, int j) {
     return i >= L.vilo && i <= L.vihi && j >= L.vjlo && j <= L.vjhi;
+}
+// Barrier of a workgroup whose wavefronts exchange data through LDS alone: unlike
+// __syncthreads it does not wait for global loads, which stay in flight across the sweeps.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 __host__ __device__ __forceinline__ int cdiv2(int v) { return v >= 0 ? v / 2 : -((-v + 1) / 2); }
 
@@ -94,6 +95,16 @@ __device__ __forceinline__ double gs_point(const LV& L, int i, int j, PF P, doub
     return (rhs - l) * c0_inv;
 }
 
+// the same on a cell-centred level, with the one-sided stencil chosen by selects
+template <class LV>
+__device__ __forceinline__ double gs_edge(const LV& L, int i, int j, double w, double e, double b, double t, double rhs,
+                                          double c0_inv) {
+    const bool x0 = i == L.ilo, x1 = i == L.ihi, y0 = j == L.jlo, y1 = j == L.jhi;
+    double l = (x0 || x1 ? L.facx * (4. / 3.) : L.facx) * (x0 ? e : x1 ? w : w + e);
+    l += (y0 || y1 ? L.facy * (4. / 3.) : L.facy) * (y0 ? t : y1 ? b : b + t);
+    return (rhs - l) * c0_inv;
+}
+
 // laplacian + residual1 (HpMultiGrid.cpp:163-190). The box-edge branches only fire on
 // cell-centred levels: on node-centred ones the edge nodes are not valid points.
 template <bool CC, class LV, class PF>
@@ -109,17 +120,19 @@ __device__ __forceinline__ double residual1(const LV& L, int i, int j, PF P, dou
     return rhs + acf * P(0, 0) - r;
 }
 
-// fine_in + I(crse) at fine point (i, j) (interpcpy_cc / interpcpy_nd, :88-121);
-// c(a, b) reads the coarse correction
-template <bool CC, class CF>
-__device__ __forceinline__ double interp_add(int i, int j, double fine_in, CF c) {
-    const int ic = cdiv2(i), jc = cdiv2(j);
-    if (CC) return fine_in + c(ic, jc);
-    const bool io = (ic * 2 != i), jo = (jc * 2 != j);
-    if (io && jo) return fine_in + (c(ic, jc) + c(ic + 1, jc) + c(ic, jc + 1) + c(ic + 1, jc + 1)) * 0.25;
-    if (io) return fine_in + (c(ic, jc) + c(ic + 1, jc)) * 0.5;
-    if (jo) return fine_in + (c(ic, jc) + c(ic, jc + 1)) * 0.5;
-    return fine_in + c(ic, jc);
+// fine_in + I(crse) at fine point (i, j) (interpcpy_cc / interpcpy_nd, :88-121) from the
+// coarse values c00 .. c11 at (ic, jc), (ic + 1, jc), (ic, jc + 1), (ic + 1, jc + 1), ic = i / 2;
+// no branch: the sum and its factor (a power of two) are chosen by selects
+template <bool CC>
+__device__ __forceinline__ double interp_sum(int i, int j, double fine_in, double c00, double c10, double c01,
+                                             double c11) {
+    if (CC) return fine_in + c00;
+    const bool io = (i & 1) != 0, jo = (j & 1) != 0;
+    double t = c00;
+    t = io ? t + c10 : t;
+    t = jo ? t + c01 : t;
+    t = io && jo ? t + c11 : t;
+    return fine_in + t * (io && jo ? 0.25 : io || jo ? 0.5 : 1.0);
 }
 
 // restrict_cc / restrict_nd (:31-52) at coarse point (i, j); f(a, b) reads the fine array
@@ -286,113 +299,147 @@ __device__ bool fold_decide(const Fold& f, const MGCtl* gate, double* red) {
     return done;
 }
 
+// Tile of a k_smooth launch. A wavefront holds two swept rows of 32 points of one colour each,
+// a thread KP points of each colour NT / 32 rows apart, so the swept region is 64 x (16 KP)
+// points and the tile what is left inside it: after NSW sweeps a point is exact if
+// it lies NSW or more points inside the frozen ring, the residual needs one neighbour more and
+// the full weighting of node-centred levels the residual of one ring around the tile.
+template <int NSW, bool CC, bool RES, int KP>
+struct Tile {
+    static constexpr int HALO = NSW + (RES ? (CC ? 1 : 2) : 0);
+    static constexpr int SW = 64, SH = NT / 32 * KP;
+    static constexpr int LX = SW + 2, LY = SH + 2;
+    static constexpr int TX = LX - 2 * HALO, TY = LY - 2 * HALO;
+    static_assert(TX > 0 && TY > 0 && TX % 2 == 0 && TY % 2 == 0, "the tile holds whole coarse points");
+};
+
 // NSW red-black sweeps (colours 0,1,2,3,0,1,...) of one level, LDS-tiled, optionally
 // followed by the residual and its restriction to the coarse points this tile owns (res_c).
 // Start: zero (ZERO), phi_in + I(cor_c) (INTERP) or phi_in. Result -> phi_out.
 // NORMS: the workgroup's max |residual| over its tile and (RHSMAX) max |rhs| over its
 // points go to norms[2 b], norms[2 b + 1] for the convergence check that follows.
-// ACF: acf is restricted to the coarse points the tile owns as well (average_down_acoef,
-// :1641-1661), so the first pass over each level prepares the next level's coefficient.
+// FIRST, a solve's first pass over the level: 1/c0 of the tile's points is computed from acf
+// and kept for the later passes, and acf is restricted to the coarse points the tile owns
+// (average_down_acoef, :1641-1661), which prepares the next level's coefficient.
 // Every launch returns at once when the control block says the solve is finished (the
 // data loads are issued before that flag is tested, so its latency is hidden).
 //
-// Every thread owns up to KP swept points of each parity of (i + j) and keeps their rhs,
-// acf and 1/c0 in registers. A sweep of one colour touches one parity class only; the
-// thread reads all neighbours of its points first, then updates, then writes (points of
-// one colour never neighbour each other, so this is the order a global sweep has).
-template <int NSW, bool CC, bool ZERO, bool RES, bool INTERP, bool RHSMAX, bool NORMS, bool ACF>
-__global__ __launch_bounds__(NT) void k_smooth(MGLevel L, MGLevel C, double* __restrict__ phi_out,
+// The two components are independent systems with the same acf: each has workgroups of its
+// own. A thread owns KP points of each parity of (i + j) and keeps their rhs and 1/c0 in
+// registers. A sweep of one colour touches one parity class
+// only; the thread reads all neighbours of its points first, then updates, then writes
+// (points of one colour never neighbour each other, so this is the order a global sweep has).
+// Bound by latency on the small levels and by issue on the large ones: a sweep is one LDS
+// round trip, a chain of seven FP64 operations and a barrier. All points of a thread share
+// their LDS addresses up to a constant, the parity of i and that of j, so the sweeps and the
+// prolongation have no index arithmetic. Nothing is read under a condition: global indices
+// are clamped to the box and only the store of a swept point is predicated; a fence after
+// each group of reads keeps the compiler from waiting for them one by one. Measured, and before
+// with tiles of 32 x 16 points, both components in 256 threads and conditional reads: four sweeps
+// of a small level 4.6 us (8.7; an empty launch takes 2), eight sweeps of 255 x 255 points 7.8 us
+// (15.6), of 511 x 511 14.4 us (19.3), of 1023 x 1023 39 us (58; with KP = 4, 38).
+template <int NSW, bool CC, bool ZERO, bool RES, bool INTERP, bool RHSMAX, bool NORMS, bool FIRST, int KP>
+__global__ __launch_bounds__(NT, 4) void k_smooth(MGLevel L, MGLevel C, double* __restrict__ phi_out,
                                                const double* __restrict__ rhs, long rcs,
                                                const double* __restrict__ acf, const double* __restrict__ phi_in,
                                                const double* __restrict__ cor_c, double* __restrict__ res_c,
                                                const MGCtl* __restrict__ gate, double* __restrict__ norms,
                                                Fold fold) {
     static_assert(NSW % 2 == 0, "sweeps come in red-black pairs");
-    constexpr int HALO = NSW + 2;
-    constexpr int LX = TX + 2 * HALO, LY = TY + 2 * HALO;
-    constexpr int SW = LX - 2, SH = LY - 2;        // swept region (inside the frozen ring)
-    constexpr int HW = SW / 2;                     // points of one parity per swept row
-    constexpr int NPAR = HW * SH;                  // points of one parity
-    constexpr int KP = (NPAR + NT - 1) / NT;       // points of one parity per thread
-    constexpr int NLD = (LX * LY + NT - 1) / NT;   // start values loaded per thread
-    // LDS holds the two colours of the tile apart: point (lx, ly) lives in
-    // s[c][(base + lx + ly) & 1][ly][lx >> 1], so a colour sweep and its neighbour reads walk
-    // consecutive doubles across the lanes (no two-way bank conflict from stride-2 rows)
-    constexpr int LXH = LX / 2;
-    static_assert(LX % 2 == 0, "a tile row holds whole point pairs");
-    __shared__ double s[2][2][LY][LXH];
-    __shared__ double r[2][RH][RW];
-    __shared__ double red[2][NT / 64];
-    __shared__ double ra[ACF ? RH : 1][ACF ? RW : 1];
     static_assert(!NORMS || RES, "the norms come from the residual");
-    static_assert(!ACF || RES, "acf is restricted with the residual");
+    static_assert(!FIRST || RES, "acf is restricted with the residual");
+    using T = Tile<NSW, CC, RES, KP>;
+    constexpr int HALO = T::HALO, TX = T::TX, TY = T::TY, LX = T::LX, LY = T::LY;
+    constexpr int RS = NT / 32;                    // rows between a thread's points
+    // rows of the residual (the tile and, node-centred, one ring) among a thread's KP points
+    constexpr int RING = CC ? 0 : 1;
+    constexpr int QA = RES ? (HALO - RING - 1) / RS : (HALO - 1) / RS;
+    constexpr int QB = RES ? (HALO + TY + RING - 2) / RS + 1 : (HALO + TY - 2) / RS + 1;
+    // LDS holds the two colours of the tile apart: point (lx, ly) lives in
+    // s[(i + j) & 1][ly][lx >> 1], so a colour sweep and its neighbour reads walk consecutive
+    // doubles across the lanes
+    constexpr int LXH = LX / 2, PL = LY * LXH;
+    constexpr int CLX = INTERP ? LX / 2 + 2 : 1, CLY = INTERP ? LY / 2 + 2 : 1;
+    constexpr int NCL = (CLX * CLY + NT - 1) / NT;
+    __shared__ double s[2 * PL];
+    __shared__ double cc[CLX * CLY];               // the coarse correction under the tile
+    __shared__ double red[2][NT / 64];
     const int gate_done = (fold.mode == Fold::NONE) ? (gate ? gate->done : 0) : 0;
     int bx, by;
     xcd_tile(bx, by);
+    const int comp = bx & 1, tid = int(threadIdx.x);
+    bx >>= 1;
     const int ti0 = L.vilo + bx * TX - HALO;
     const int tj0 = L.vjlo + by * TY - HALO;
-    const int base = (ti0 + tj0) & 1;
-    auto S = [&](int c, int ly, int lx) -> double& { return s[c][(base + lx + ly) & 1][ly][lx >> 1]; };
-    const double facx = 1. / (L.dx * L.dx), facy = 1. / (L.dy * L.dy);
-    // owned points: [parity][q]; pl = lx | ly << 8, or -1 outside the valid box / region;
-    // acf stays in registers for the residual (ai), ci becomes 1/c0
-    double r0[2][KP], r1[2][KP], ci[2][KP], ai[2][RES ? KP : 1];
-    int pl[2][KP];
+    const double facx = L.facx, facy = L.facy;
+    // global offsets count from the first valid point of the region, clamped to the valid box
+    const int oi = max(ti0, L.vilo), oj = max(tj0, L.vjlo);
+    const long ko = at(L, oi, oj);
+    const double* const rhs_o = rhs + (comp ? rcs : 0) + ko;
+    const double* const phi_o = ZERO ? nullptr : phi_in + (comp ? L.cs : 0) + ko;
+    const double* const acf_o = acf + ko;
+    double* const out_o = phi_out + (comp ? L.cs : 0) + ko;
+    double* const c0i_o = L.c0i + ko;
+    const int omax = (L.vjhi - oj) * L.ldx;
+    auto ld = [](const double* b, int k) {
+        return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(b) + unsigned(k) * 8u);
+    };
+    // owned points: column lx[par], rows ly + RS q; ks is the index of q = 0 in its colour's
+    // plane, kw that of its west neighbour in the other one
+    const int ly = 1 + (tid >> 5);
+    const int row0 = __mul24(tj0 + ly - oj, L.ldx), rstep = RS * L.ldx;
+    int lx[2], ks[2], kw[2], col[2];
+    bool vi[2], vj[KP];
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
+        lx[par] = 1 + 2 * (tid & 31) + ((par + ti0 + tj0 + ly + 1) & 1);
+        ks[par] = ly * LXH + (lx[par] >> 1);
+        kw[par] = ly * LXH + ((lx[par] - 1) >> 1);
+        const int i = ti0 + lx[par];
+        col[par] = min(max(i, oi), L.vihi) - oi;
+        vi[par] = i >= L.vilo && i <= L.vihi;
+    }
+    double r0[2][KP], ci[2][KP], v[2][KP];
 #pragma unroll
-        for (int q = 0; q < KP; ++q) {
-            const int e = threadIdx.x + q * NT;
-            pl[par][q] = -1;
-            r0[par][q] = r1[par][q] = ci[par][q] = 0.0;
-            if (RES) ai[par][q] = 0.0;
-            if (e < NPAR) {
-                const int ly = 1 + e / HW;
-                const int lx = 1 + 2 * (e - (ly - 1) * HW) + ((par + base + ly + 1) & 1);
-                const int i = ti0 + lx, j = tj0 + ly;
-                if (in_valid(L, i, j)) {
-                    const long k = at(L, i, j);
-                    pl[par][q] = lx | (ly << 8);
-                    r0[par][q] = rhs[k];
-                    r1[par][q] = rhs[k + rcs];
-                    ci[par][q] = acf[k];   // acf for now, 1/c0 below
-                    if (RES) ai[par][q] = ci[par][q];
-                }
-            }
+    for (int q = 0; q < KP; ++q) {
+        const int j = tj0 + ly + RS * q;
+        vj[q] = j >= L.vjlo && j <= L.vjhi;
+        const int row = min(max(row0 + q * rstep, 0), omax);
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const int k = row + col[par];
+            r0[par][q] = ld(rhs_o, k);
+            ci[par][q] = FIRST ? ld(acf_o, k) : ld(c0i_o, k);
+            v[par][q] = ZERO ? 0.0 : ld(phi_o, k);
         }
     }
-    // start values: phi_in (and the coarse correction under the tile) into registers with
-    // all loads in flight at once, then into LDS; the prolongation reads the coarse tile
-    // from LDS
-    constexpr int CLX = INTERP ? LX / 2 + 2 : 1, CLY = INTERP ? LY / 2 + 2 : 1;
-    constexpr int NCL = INTERP ? (CLX * CLY + NT - 1) / NT : 1;
-    __shared__ double cc[2][CLY][CLX];
+    // the frozen ring without its corners: threads [0, 64) its first row, [64, 128) the last,
+    // the next LY - 2 the first column, the next the last
+    constexpr int NRING = 2 * T::SW + 2 * (LY - 2), KRING = (NRING + NT - 1) / NT;
+    double vr[KRING];
+    auto ring = [&](int q, int& x, int& y) {
+        const int e = tid + q * NT;
+        const int f = e - 2 * T::SW;
+        x = e < 2 * T::SW ? 1 + (e & 63) : f < LY - 2 ? 0 : LX - 1;
+        y = e < T::SW ? 0 : e < 2 * T::SW ? LY - 1 : 1 + (f < LY - 2 ? f : min(f - (LY - 2), LY - 3));
+    };
+#pragma unroll
+    for (int q = 0; q < KRING; ++q) {
+        int x, y;
+        ring(q, x, y);
+        vr[q] = ZERO ? 0.0
+                     : ld(phi_o, min(max(__mul24(tj0 + y - oj, L.ldx), 0), omax) +
+                                     (min(max(ti0 + x, oi), L.vihi) - oi));
+    }
     const int ic0 = cdiv2(ti0), jc0 = cdiv2(tj0);
-    double v0[NLD], v1[NLD], cv0[NCL], cv1[NCL];
-#pragma unroll
-    for (int it = 0; it < NLD; ++it) {
-        const int e = threadIdx.x + it * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        const int i = ti0 + lx, j = tj0 + ly;
-        v0[it] = v1[it] = 0.0;
-        if (!ZERO && e < LX * LY && in_valid(L, i, j)) {
-            const long k = at(L, i, j);
-            v0[it] = phi_in[k];
-            v1[it] = phi_in[k + L.cs];
-        }
-    }
+    double cv[NCL];
     if (INTERP) {
+        const double* const cor_k = cor_c + (comp ? C.cs : 0);
 #pragma unroll
         for (int it = 0; it < NCL; ++it) {
-            const int e = threadIdx.x + it * NT;
+            const int e = min(tid + it * NT, CLX * CLY - 1);
             const int cy = e / CLX, cx = e - cy * CLX;
-            const int ic = ic0 + cx, jc = jc0 + cy;
-            cv0[it] = cv1[it] = 0.0;
-            if (e < CLX * CLY && ic >= C.ilo - 1 && ic <= C.ihi + 1 && jc >= C.jlo - 1 && jc <= C.jhi + 1) {
-                const long k = at(C, ic, jc);
-                cv0[it] = cor_c[k];
-                cv1[it] = cor_c[k + C.cs];
-            }
+            cv[it] = cor_k[at(C, min(max(ic0 + cx, C.ilo - 1), C.ihi + 1), min(max(jc0 + cy, C.jlo - 1), C.jhi + 1))];
         }
     }
     if (gate_done) return;
@@ -400,151 +447,222 @@ __global__ __launch_bounds__(NT) void k_smooth(MGLevel L, MGLevel C, double* __r
     if (fold.mode != Fold::NONE && fold_decide(fold, nullptr, &red[0][0])) return;
     if (INTERP) {
 #pragma unroll
-        for (int it = 0; it < NCL; ++it) {
-            const int e = threadIdx.x + it * NT;
-            if (e < CLX * CLY) {
-                const int cy = e / CLX, cx = e - cy * CLX;
-                cc[0][cy][cx] = cv0[it];
-                cc[1][cy][cx] = cv1[it];
-            }
-        }
-        __syncthreads();
-    }
+        for (int it = 0; it < NCL; ++it) cc[min(tid + it * NT, CLX * CLY - 1)] = cv[it];
+        lds_barrier();
 #pragma unroll
-    for (int it = 0; it < NLD; ++it) {
-        const int e = threadIdx.x + it * NT;
-        if (e < LX * LY) {
-            const int ly = e / LX, lx = e - ly * LX;
-            double a0 = v0[it], a1 = v1[it];
-            if (INTERP && in_valid(L, ti0 + lx, tj0 + ly)) {
-                auto c0 = [&](int a, int b) { return cc[0][b - jc0][a - ic0]; };
-                auto c1 = [&](int a, int b) { return cc[1][b - jc0][a - ic0]; };
-                a0 = interp_add<CC>(ti0 + lx, tj0 + ly, a0, c0);
-                a1 = interp_add<CC>(ti0 + lx, tj0 + ly, a1, c1);
-            }
-            S(0, ly, lx) = a0;
-            S(1, ly, lx) = a1;
+        for (int q = 0; q < KRING; ++q) {
+            int x, y;
+            ring(q, x, y);
+            const int i = ti0 + x, j = tj0 + y;
+            const double* const p = cc + (cdiv2(j) - jc0) * CLX + (cdiv2(i) - ic0);
+            const double c00 = p[0], c10 = CC ? 0.0 : p[1], c01 = CC ? 0.0 : p[CLX], c11 = CC ? 0.0 : p[CLX + 1];
+            vr[q] = interp_sum<CC>(i, j, vr[q], c00, c10, c01, c11);
         }
     }
     double rmax = 0.0;
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
+        if (INTERP) {
+            const int i = ti0 + lx[par], j = tj0 + ly;
+            const double* const p = cc + (cdiv2(j) - jc0) * CLX + (cdiv2(i) - ic0);
+            // node-centred: i and j are both even or both odd for colour 0 (the coarse point
+            // or four of them), one of them is odd for colour 1 (two along that direction)
+            const bool jo = (j & 1) != 0;
+            const int p1 = par == 0 || !jo ? 1 : CLX;
+            double c[4][KP];
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                const double* const pq = p + q * (RS / 2) * CLX;
+                c[0][q] = pq[0];
+                if (!CC) c[1][q] = pq[p1];
+                if (!CC && par == 0) {
+                    c[2][q] = pq[CLX];
+                    c[3][q] = pq[CLX + 1];
+                }
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                if (CC) v[par][q] += c[0][q];
+                else if (par == 1) v[par][q] += (c[0][q] + c[1][q]) * 0.5;
+                else {
+                    const double four = (c[0][q] + c[1][q] + c[2][q] + c[3][q]) * 0.25;
+                    v[par][q] += jo ? four : c[0][q];
+                }
+            }
+        }
 #pragma unroll
         for (int q = 0; q < KP; ++q) {
-            if (pl[par][q] < 0) continue;
-            const int lx = pl[par][q] & 255, ly = pl[par][q] >> 8;
-            ci[par][q] = c0_inverse<CC>(L, ti0 + lx, tj0 + ly, ci[par][q], facx, facy);
-            if (RHSMAX) rmax = fmax(rmax, fmax(fabs(r0[par][q]), fabs(r1[par][q])));
+            s[par * PL + ks[par] + q * RS * LXH] = vi[par] && vj[q] ? v[par][q] : 0.0;
+            if (RHSMAX) rmax = fmax(rmax, fabs(r0[par][q]));
+            if (FIRST) {
+                ci[par][q] = c0_inverse<CC>(L, ti0 + lx[par], tj0 + ly + RS * q, ci[par][q], facx, facy);
+                const int y = ly + RS * q;
+                const bool out = lx[par] >= HALO && lx[par] < HALO + TX && y >= HALO && y < HALO + TY;
+                if (comp == 0 && out && vi[par] && vj[q]) c0i_o[row0 + q * rstep + col[par]] = ci[par][q];
+            }
         }
+        asm volatile("" ::: "memory");   // one colour at a time, for the registers
     }
-    __syncthreads();
-    // one colour: reads, then updates, then writes, in batches of up to KB points
-    constexpr int KB = KP > 2 ? (KP + 1) / 2 : KP;
+#pragma unroll
+    for (int q = 0; q < KRING; ++q) {
+        int x, y;
+        ring(q, x, y);
+        if (tid + q * NT < NRING)
+            s[((ti0 + tj0 + x + y) & 1) * PL + y * LXH + (x >> 1)] = in_valid(L, ti0 + x, tj0 + y) ? vr[q] : 0.0;
+    }
+    lds_barrier();
+    // cell-centred tiles at the edge of the box have points with a one-sided stencil
+    const bool edge = CC && (ti0 + 1 <= L.ilo || ti0 + T::SW >= L.ihi || tj0 + 1 <= L.jlo || tj0 + T::SH >= L.jhi);
+    // one colour: reads, then updates, then writes
     auto sweep = [&](auto PARC) {
         constexpr int par = decltype(PARC)::value;
-        // a point of colour par has (base + lx + ly) & 1 == par; its neighbours the other one
-        constexpr int np = 1 - par;
+        // a point of colour par has (i + j) & 1 == par; its neighbours the other one
+        const double* const sn = s + (1 - par) * PL;
+        double w[KP], e[KP], b[KP], t[KP], u[KP];
 #pragma unroll
-        for (int q0 = 0; q0 < KP; q0 += KB) {
-            double w0[KB], e0[KB], s0[KB], n0[KB], w1[KB], e1[KB], s1[KB], n1[KB];
+        for (int q = 0; q < KP; ++q) {
+            w[q] = sn[kw[par] + q * RS * LXH];
+            e[q] = sn[kw[par] + q * RS * LXH + 1];
+            b[q] = sn[ks[par] + (q * RS - 1) * LXH];
+            t[q] = sn[ks[par] + (q * RS + 1) * LXH];
+        }
+        asm volatile("" ::: "memory");
+        if (CC && edge) {
 #pragma unroll
-            for (int b = 0; b < KB; ++b) {
-                const int q = q0 + b;
-                if (q >= KP || pl[par][q] < 0) continue;
-                const int lx = pl[par][q] & 255, ly = pl[par][q] >> 8;
-                const int xw = (lx - 1) >> 1, xe = (lx + 1) >> 1, xc = lx >> 1;
-                w0[b] = s[0][np][ly][xw]; e0[b] = s[0][np][ly][xe]; s0[b] = s[0][np][ly - 1][xc]; n0[b] = s[0][np][ly + 1][xc];
-                w1[b] = s[1][np][ly][xw]; e1[b] = s[1][np][ly][xe]; s1[b] = s[1][np][ly - 1][xc]; n1[b] = s[1][np][ly + 1][xc];
-            }
-            double u0[KB], u1[KB];
+            for (int q = 0; q < KP; ++q)
+                u[q] = gs_edge(L, ti0 + lx[par], tj0 + ly + RS * q, w[q], e[q], b[q], t[q], r0[par][q], ci[par][q]);
+        } else {
 #pragma unroll
-            for (int b = 0; b < KB; ++b) {
-                const int q = q0 + b;
-                if (q >= KP || pl[par][q] < 0) continue;
-                const int lx = pl[par][q] & 255, ly = pl[par][q] >> 8;
-                const int i = ti0 + lx, j = tj0 + ly;
-                auto P0 = [&](int di, int dj) { return di < 0 ? w0[b] : di > 0 ? e0[b] : dj < 0 ? s0[b] : n0[b]; };
-                auto P1 = [&](int di, int dj) { return di < 0 ? w1[b] : di > 0 ? e1[b] : dj < 0 ? s1[b] : n1[b]; };
-                u0[b] = gs_point<CC>(L, i, j, P0, r0[par][q], ci[par][q], facx, facy);
-                u1[b] = gs_point<CC>(L, i, j, P1, r1[par][q], ci[par][q], facx, facy);
-            }
-#pragma unroll
-            for (int b = 0; b < KB; ++b) {
-                const int q = q0 + b;
-                if (q >= KP || pl[par][q] < 0) continue;
-                const int lx = pl[par][q] & 255, ly = pl[par][q] >> 8;
-                s[0][par][ly][lx >> 1] = u0[b];
-                s[1][par][ly][lx >> 1] = u1[b];
+            for (int q = 0; q < KP; ++q) {
+                double l = facx * (w[q] + e[q]);
+                l += facy * (b[q] + t[q]);
+                u[q] = (r0[par][q] - l) * ci[par][q];
             }
         }
-        __syncthreads();
+        // all updates before the first predicated store, or each would be moved under its own
+#pragma unroll
+        for (int q = 0; q < KP; ++q) asm volatile("" : "+v"(u[q]));
+#pragma unroll
+        for (int q = 0; q < KP; ++q)
+            if (vi[par] && vj[q]) s[par * PL + ks[par] + q * RS * LXH] = u[q];
+        lds_barrier();
     };
     // colour c updates the points with (i + j + c) even, i.e. parity c & 1
-    for (int c2 = 0; c2 < NSW; c2 += 2) {
+#pragma unroll 1
+    for (int c2 = 0; c2 < NSW - 2; c2 += 2) {
         sweep(std::integral_constant<int, 0>{});
         sweep(std::integral_constant<int, 1>{});
     }
+    // acf of the residual's points, in flight during the last two sweeps
+    double ar[2][RES ? QB - QA : 1];
+    if (RES) {
+#pragma unroll
+        for (int q = QA; q < QB; ++q) {
+            const int row = min(max(row0 + q * rstep, 0), omax);
+            ar[0][q - QA] = ld(acf_o, row + col[0]);
+            ar[1][q - QA] = ld(acf_o, row + col[1]);
+        }
+    }
+    sweep(std::integral_constant<int, 0>{});
+    sweep(std::integral_constant<int, 1>{});
     double m = 0.0;
+    double z[2][QB - QA], g[2][RES ? QB - QA : 1];
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
+        const double* const sn = s + (1 - par) * PL;
+        double w[QB - QA], e[QB - QA], b[QB - QA], t[QB - QA];
 #pragma unroll
-        for (int q = 0; q < KP; ++q) {
-            if (pl[par][q] < 0) continue;
-            const int lx = pl[par][q] & 255, ly = pl[par][q] >> 8;
-            const bool out = lx >= HALO && lx < HALO + TX && ly >= HALO && ly < HALO + TY;
+        for (int q = QA; q < QB; ++q) {
+            z[par][q - QA] = s[par * PL + ks[par] + q * RS * LXH];
             if (RES) {
-                const bool ring = lx >= HALO - 1 && lx <= HALO + TX && ly >= HALO - 1 && ly <= HALO + TY;
-                if (ring) {
-                    const int i = ti0 + lx, j = tj0 + ly;
-                    const double a = ai[par][RES ? q : 0];
-                    // the point has colour par, its four neighbours the other one
-                    auto P0 = [&](int di, int dj) {
-                        return (di | dj) ? s[0][1 - par][ly + dj][(lx + di) >> 1] : s[0][par][ly][lx >> 1];
-                    };
-                    auto P1 = [&](int di, int dj) {
-                        return (di | dj) ? s[1][1 - par][ly + dj][(lx + di) >> 1] : s[1][par][ly][lx >> 1];
-                    };
-                    const double g0 = residual1<CC>(L, i, j, P0, r0[par][q], a, facx, facy);
-                    const double g1 = residual1<CC>(L, i, j, P1, r1[par][q], a, facx, facy);
-                    if (out) m = fmax(m, fmax(fabs(g0), fabs(g1)));
-                    r[0][ly - HALO + 1][lx - HALO + 1] = g0;
-                    r[1][ly - HALO + 1][lx - HALO + 1] = g1;
-                    if (ACF) ra[ly - HALO + 1][lx - HALO + 1] = a;
-                }
+                w[q - QA] = sn[kw[par] + q * RS * LXH];
+                e[q - QA] = sn[kw[par] + q * RS * LXH + 1];
+                b[q - QA] = sn[ks[par] + (q * RS - 1) * LXH];
+                t[q - QA] = sn[ks[par] + (q * RS + 1) * LXH];
             }
-            if (out) {
-                const long k = at(L, ti0 + lx, tj0 + ly);
-                phi_out[k] = s[0][par][ly][lx >> 1];
-                phi_out[k + L.cs] = s[1][par][ly][lx >> 1];
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int q = QA; q < QB; ++q) asm volatile("" : "+v"(z[par][q - QA]));
+#pragma unroll
+        for (int q = QA; q < QB; ++q) {
+            const int n = q - QA, y = ly + RS * q;
+            const bool val = vi[par] && vj[q];
+            const bool out = val && lx[par] >= HALO && lx[par] < HALO + TX && y >= HALO && y < HALO + TY;
+            if (out) out_o[row0 + q * rstep + col[par]] = z[par][n];
+            if (RES) {
+                auto P = [&](int di, int dj) {
+                    return di < 0 ? w[n] : di > 0 ? e[n] : dj < 0 ? b[n] : dj > 0 ? t[n] : z[par][n];
+                };
+                const double x = CC && edge
+                                     ? residual1<CC>(L, ti0 + lx[par], tj0 + y, P, r0[par][q], ar[par][n], facx, facy)
+                                     : residual1<false>(L, 0, 0, P, r0[par][q], ar[par][n], facx, facy);
+                if (out) m = fmax(m, fabs(x));
+                // points outside the valid box hold zero residual
+                g[par][n] = val ? x : 0.0;
             }
         }
     }
     if (RES) {
-        // ring points outside the valid box hold zero residual
-        for (int e = threadIdx.x; e < RW * RH; e += NT) {
-            const int ry = e / RW, rx = e - ry * RW;
-            if (!in_valid(L, ti0 + HALO - 1 + rx, tj0 + HALO - 1 + ry)) {
-                r[0][ry][rx] = 0.0;
-                r[1][ry][rx] = 0.0;
-                if (ACF) ra[ry][rx] = 0.0;
+        // the residual takes the place of the iterate
+        lds_barrier();
+#pragma unroll
+        for (int par = 0; par < 2; ++par)
+#pragma unroll
+            for (int q = QA; q < QB; ++q) s[par * PL + ks[par] + q * RS * LXH] = g[par][q - QA];
+        lds_barrier();
+        // coarse points whose centre fine point 2*ic lies in this tile: TX/2 x TY/2 of them
+        static_assert(TX / 2 <= 32, "one lane per coarse point of a row");
+        const int ic = cdiv2(ti0 + HALO + 1) + (tid & 31);
+        auto restricted = [&](int jc) {
+            // the four diagonal neighbours have the centre's parity, 0, the others parity 1
+            const int cx = 2 * ic - ti0, cy = 2 * jc - tj0;
+            const double* const p0 = s + cy * LXH;
+            const double* const p1 = p0 + PL;
+            const int xw = (cx - 1) >> 1, xc = cx >> 1, xe = (cx + 1) >> 1;
+            double f[9];
+            f[4] = p0[xc];
+            f[5] = p1[xe];
+            f[7] = p1[LXH + xc];
+            f[8] = p0[LXH + xe];
+            if (!CC) {
+                f[0] = p0[xw - LXH];
+                f[1] = p1[xc - LXH];
+                f[2] = p0[xe - LXH];
+                f[3] = p1[xw];
+                f[6] = p0[xw + LXH];
             }
+            asm volatile("" ::: "memory");
+            auto F = [&](int a, int b) { return f[(b - 2 * jc + 1) * 3 + (a - 2 * ic) + 1]; };
+            return restrict_from<CC>(F, ic, jc);
+        };
+        const int jc_0 = cdiv2(tj0 + HALO + 1) + (tid >> 5);
+        const bool own = (tid & 31) < TX / 2 && ic >= C.vilo && ic <= C.vihi;
+#pragma unroll
+        for (int q = 0; q < TY / 2; q += RS) {
+            const int jc = jc_0 + q;
+            if (own && q + (tid >> 5) < TY / 2 && jc >= C.vjlo && jc <= C.vjhi)
+                res_c[at(C, ic, jc) + (comp ? C.cs : 0)] = restricted(jc);
         }
-        __syncthreads();
-        // coarse points whose centre fine point 2*ic lies in this tile
-        const int ox0 = ti0 + HALO, oy0 = tj0 + HALO;
-        const int ic0 = cdiv2(ox0 + 1), jc0 = cdiv2(oy0 + 1);
-        for (int t = threadIdx.x; t < (TX / 2 + 1) * (TY / 2 + 1); t += NT) {
-            const int ic = ic0 + t % (TX / 2 + 1), jc = jc0 + t / (TX / 2 + 1);
-            if (2 * ic < ox0 || 2 * ic >= ox0 + TX || 2 * jc < oy0 || 2 * jc >= oy0 + TY) continue;
-            if (!in_valid(C, ic, jc)) continue;
-            // fine residual at (fi, fj) lives in r[.][fj - oy0 + 1][fi - ox0 + 1]
-            auto f0 = [&](int fi, int fj) { return r[0][fj - oy0 + 1][fi - ox0 + 1]; };
-            auto f1 = [&](int fi, int fj) { return r[1][fj - oy0 + 1][fi - ox0 + 1]; };
-            res_c[at(C, ic, jc)] = restrict_from<CC>(f0, ic, jc);
-            res_c[at(C, ic, jc) + C.cs] = restrict_from<CC>(f1, ic, jc);
-            if (ACF) {
-                auto fa = [&](int fi, int fj) { return ra[fj - oy0 + 1][fi - ox0 + 1]; };
-                C.acf[at(C, ic, jc)] = restrict_from<CC>(fa, ic, jc);
+        if (FIRST) {
+            lds_barrier();
+            if (comp == 0) {
+                // then acf that of the residual
+#pragma unroll
+                for (int par = 0; par < 2; ++par)
+#pragma unroll
+                    for (int q = QA; q < QB; ++q)
+                        s[par * PL + ks[par] + q * RS * LXH] = vi[par] && vj[q] ? ar[par][q - QA] : 0.0;
+            }
+            lds_barrier();
+            if (comp == 0) {
+#pragma unroll
+                for (int q = 0; q < TY / 2; q += RS) {
+                    const int jc = jc_0 + q;
+                    if (own && q + (tid >> 5) < TY / 2 && jc >= C.vjlo && jc <= C.vjhi)
+                        C.acf[at(C, ic, jc)] = restricted(jc);
+                }
             }
         }
     }
@@ -559,14 +677,14 @@ __global__ __launch_bounds__(NT) void k_smooth(MGLevel L, MGLevel C, double* __r
         }
         __syncthreads();
         if (threadIdx.x == 0) {
-            double mm = red[0][0], rr = red[1][0];
+            double mm = red[0][0], rm = red[1][0];
             for (int w = 1; w < NT / 64; ++w) {
                 mm = fmax(mm, red[0][w]);
-                rr = fmax(rr, red[1][w]);
+                rm = fmax(rm, red[1][w]);
             }
-            const unsigned b = by * gridDim.x + bx;
+            const unsigned b = by * gridDim.x + 2 * bx + comp;
             norms[2 * b] = mm;
-            norms[2 * b + 1] = rr;
+            norms[2 * b + 1] = rm;
         }
     }
 }
@@ -574,177 +692,526 @@ __global__ __launch_bounds__(NT) void k_smooth(MGLevel L, MGLevel C, double* __r
 // ---------------------------------------------------------------------------------
 // coarse levels in one workgroup
 // ---------------------------------------------------------------------------------
-// Geometry of one coarse level and the offsets of its arrays in the work array (LDS, or
-// global memory when the levels do not fit). Every array covers the level box plus one
-// ghost ring, x fastest, as MGLevel's arrays do. The two components are independent
-// systems with the same acf, so each has a workgroup of its own: the work array holds one
-// component (a second one follows it when the arrays live in global memory).
-struct CLev {
-    int ilo, ihi, jlo, jhi, vilo, vihi, vjlo, vjhi, ldx, cs;
-    int acf, c0i, res, cor, rescor;
+// The coarse part of the V-cycle is a chain of some fifty dependent steps, bound by the length
+// of each: an LDS round trip, seven FP64 operations and a barrier. So a thread owns at most two
+// points of each colour of a level and knows their LDS addresses; its neighbours' reads are in
+// flight together; rhs and 1/c0 sit in registers during a level's sweeps; and the levels of at
+// most 64 points of a colour run on wavefront 0 alone, without barriers (LDS operations of one
+// wavefront execute in order, so a fence for the compiler is enough).
+// LDS of a level: phi and sc (acf, from the residual on the residual) with the colours apart,
+// [(i + j) & 1][y][x >> 1] over the box and one ghost ring; ci and r (1/c0, rhs) by owner,
+// [colour][thread]. The top level's ci, r and acf stay in registers. Below it, sc and ci depend
+// only on acf: a solve's first V-cycle averages acf down and leaves a copy of these arrays
+// (blob) in global memory for the later ones, which load it during the top level's sweeps. The
+// levels' geometry is computed, not read: loads from the argument block would be one more
+// round trip per level.
+constexpr int FT = 1024;                        // threads of the kernel
+constexpr int FKP = 2;                          // points of a colour per thread, top level
+constexpr int FNB = 4;                          // blob values per thread in flight
+constexpr size_t FLDS_MAX = 150 * 1024;
+
+// A level's box starts at point 0; its valid points at V = 0 (cell-centred) or 1.
+template <bool CC>
+struct FLev {
+    static constexpr int V = CC ? 0 : 1;
+    int nvx, nvy;            // valid points
+    int hw, np;              // points of one colour: hw per row, np in all
+    int nt;                  // threads that own points (whole wavefronts)
+    int pitch, plane;        // doubles per row and per colour
+    int sc, ci, bend;        // LDS offsets: the part kept in the blob, from 0
+    int phi, r, pend;        // the rest, from the blob's size
     double facx, facy;
-};
-struct CArgs {
-    int nlev;           // levels cb .. max_level
-    int nblock;         // levels [0, nblock) run on the whole workgroup, the rest on wave 0
-    int bottom_sweeps;
-    int work_doubles;
-    CLev lv[COARSE_MAX_LEVELS];
-    const double* acf;  // level cb in global memory
-    const double* res;
-    double* cor;
-    long gcs;
-};
-
-__device__ __forceinline__ int lat(const CLev& L, int i, int j) { return (j - L.jlo + 1) * L.ldx + (i - L.ilo + 1); }
-
-// Thread layouts of the coarse kernel. Block: thread (tx, ty) of CTX x CTY visits the
-// valid points (vilo + tx + CTX a, vjlo + ty + CTY b); a colour sweep gives each thread
-// two columns of CTX. Wave: the 64 lanes of wavefront 0 walk the valid points in order;
-// LDS traffic of one wavefront is ordered, so a wait for the LDS counter (plus a compiler
-// barrier) separates phases.
-struct BlockMode {
-    template <class F>
-    static __device__ __forceinline__ void valid(const CLev& L, F f) {
-        const int tx = threadIdx.x % CTX, ty = threadIdx.x / CTX;
-        for (int j = L.vjlo + ty; j <= L.vjhi; j += CTY)
-            for (int i = L.vilo + tx; i <= L.vihi; i += CTX) f(i, j);
+    // the level below arrays that end at b and p (the top level has phi alone)
+    __host__ __device__ __forceinline__ FLev(int nvx_, int nvy_, double fx, double fy, int b, int p, bool top)
+        : nvx(nvx_), nvy(nvy_), facx(fx), facy(fy) {
+        hw = (nvx + 1) / 2;
+        np = hw * nvy;
+        nt = np >= FT ? FT : (np + 63) & ~63;
+        pitch = (nvx + 2 * V + 3) / 2;
+        plane = pitch * (nvy + 2 * V + 2);
+        sc = b;
+        ci = sc + 2 * plane;
+        bend = top ? b : ci + 2 * nt;
+        phi = p;
+        r = phi + 2 * plane;
+        pend = top ? r : r + 2 * nt;
     }
-    template <class F>
-    static __device__ __forceinline__ void color(const CLev& L, int c, F f) {
-        const int tx = threadIdx.x % CTX, ty = threadIdx.x / CTX;
-        for (int j = L.vjlo + ty; j <= L.vjhi; j += CTY) {
-            const int i0 = L.vilo + ((L.vilo + j + c) & 1) + 2 * tx;
-            for (int i = i0; i <= L.vihi; i += 2 * CTX) f(i, j);
+    // the next coarser level, and the next finer one; spacings double exactly
+    __host__ __device__ __forceinline__ FLev coarser() const {
+        return FLev(CC ? nvx / 2 : (nvx - 1) / 2, CC ? nvy / 2 : (nvy - 1) / 2, 0.25 * facx, 0.25 * facy, bend, pend,
+                    false);
+    }
+    __device__ __forceinline__ FLev finer() const {
+        FLev f(CC ? 2 * nvx : 2 * nvx + 1, CC ? 2 * nvy : 2 * nvy + 1, 4.0 * facx, 4.0 * facy, 0, 0, false);
+        const int b = sc - f.bend, p = phi - f.pend;
+        f.sc += b; f.ci += b; f.bend += b;
+        f.phi += p; f.r += p; f.pend += p;
+        return f;
+    }
+};
+struct FArgs {
+    int nlev, nblock;    // levels [0, nblock) run on the whole workgroup
+    int bottom_sweeps;
+    int first;           // a solve's first V-cycle
+    int nblob;           // doubles of the blob
+    int tsc;             // LDS offset of the top level's sc
+    int gcs, ldx;        // level cb in global memory
+    int nvx, nvy;
+    double facx, facy;
+    const double *acf, *res;
+    double *c0i, *cor, *gblob;
+};
+
+// the points of a level that a thread owns: valid point (2 h + b, row) has colour
+// (b + row) & 1, so b = row & 1 for colour 0. at = (box row + 1) pitch + h addresses the
+// colour planes: node-centred, both colours' points lie at at + 1 and their west neighbours at
+// at + b; cell-centred, the points at at + b and the west neighbours at at.
+template <bool CC, int KP>
+struct Own {
+    static constexpr int V = CC ? 0 : 1;
+    int h[KP], row[KP], at[KP];
+    bool v[2][KP];
+    bool any;   // this wavefront owns points
+    __device__ __forceinline__ Own(const FLev<CC>& L) {
+        any = __builtin_amdgcn_readfirstlane(int(threadIdx.x)) < L.nt;
+        const float rhw = __frcp_rn(float(L.hw));   // e / hw for e < FKP * FT: see row
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+            const int e0 = int(threadIdx.x) + q * L.nt, e = min(e0, L.np - 1);
+            // (e + 1/2) / hw is 1 / (2 hw) or more from an integer, its error below 1e-3 / hw
+            row[q] = int((float(e) + 0.5f) * rhw);
+            h[q] = e - row[q] * L.hw;
+            at[q] = (row[q] + 1 + V) * L.pitch + h[q];
+            v[0][q] = e0 < L.np && 2 * h[q] + (row[q] & 1) < L.nvx;
+            v[1][q] = e0 < L.np && 2 * h[q] + 1 - (row[q] & 1) < L.nvx;
         }
     }
-    static __device__ __forceinline__ void sync() { __syncthreads(); }
+    __device__ __forceinline__ int b(int par, int q) const { return (par + row[q]) & 1; }
+    __device__ __forceinline__ int ks(int par, int q) const { return CC ? at[q] + b(par, q) : at[q] + 1; }
+    __device__ __forceinline__ int kw(int par, int q) const { return CC ? at[q] : at[q] + b(par, q); }
+    // coordinates, inside the box also for a point that is not valid
+    __device__ __forceinline__ int i(const FLev<CC>& L, int par, int q) const {
+        return V + min(2 * h[q] + b(par, q), L.nvx - 1);
+    }
+    __device__ __forceinline__ int j(int q) const { return V + row[q]; }
 };
-struct WaveMode {
-    template <class F>
-    static __device__ __forceinline__ void valid(const CLev& L, F f) {
-        const int nvx = L.vihi - L.vilo + 1, n = nvx * (L.vjhi - L.vjlo + 1);
-        for (int e = threadIdx.x; e < n; e += 64) f(L.vilo + e % nvx, L.vjlo + e / nvx);
-    }
-    template <class F>
-    static __device__ __forceinline__ void color(const CLev& L, int c, F f) {
-        valid(L, [&](int i, int j) {
-            if (((i + j + c) & 1) == 0) f(i, j);
-        });
-    }
-    static __device__ __forceinline__ void sync() {
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+
+// the cell-centred box for the functions that look at its edges
+template <bool CC>
+struct FBox {
+    int ilo, ihi, jlo, jhi;
+    double facx, facy;
+    __device__ __forceinline__ FBox(const FLev<CC>& L)
+        : ilo(0), ihi(L.nvx - 1), jlo(0), jhi(L.nvy - 1), facx(L.facx), facy(L.facy) {}
+};
+
+template <bool WAVE>
+__device__ __forceinline__ void f_sync() {
+    if (WAVE) {
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();
+    } else {
+        lds_barrier();
     }
-};
-
-template <class Mode, bool CC>
-__device__ __forceinline__ void c_sweep(double* w, const CLev& L, int color) {
-    Mode::color(L, color, [&](int i, int j) {
-        const int k = lat(L, i, j);
-        const double* p = w + L.cor;
-        auto P = [&](int a, int b) { return p[k + b * L.ldx + a]; };
-        w[L.cor + k] = gs_point<CC>(L, i, j, P, w[L.res + k], w[L.c0i + k], L.facx, L.facy);
-    });
-    Mode::sync();
 }
 
-// down-sweep step of level L: four sweeps from zero, residual, restriction into C.res
-template <class Mode, bool CC>
-__device__ void c_down(double* w, const CLev& L, const CLev& C) {
-    for (int color = 0; color < 4; ++color) c_sweep<Mode, CC>(w, L, color);
-    Mode::valid(L, [&](int i, int j) {
-        const int k = lat(L, i, j);
-        const double* p = w + L.cor;
-        auto P = [&](int di, int dj) { return p[k + dj * L.ldx + di]; };
-        w[L.rescor + k] = residual1<CC>(L, i, j, P, w[L.res + k], w[L.acf + k], L.facx, L.facy);
-    });
-    Mode::sync();
-    Mode::valid(C, [&](int i, int j) {
-        auto fa = [&](int a, int b) { return w[L.rescor + lat(L, a, b)]; };
-        w[C.res + lat(C, i, j)] = restrict_from<CC>(fa, i, j);
-    });
-    Mode::sync();
+// one sweep of colour PAR
+template <bool CC, int KP, bool WAVE, int PAR>
+__device__ __forceinline__ void f_sweep(double* phi, const FLev<CC>& L, const Own<CC, KP>& o, const double (&r)[2][KP],
+                                        const double (&ci)[2][KP]) {
+    if (o.any) {
+        double w[KP], e[KP], b[KP], t[KP], u[KP];
+        const double* const pn = phi + (1 - PAR) * L.plane;
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+            const int ks = o.ks(PAR, q), kw = o.kw(PAR, q);
+            w[q] = pn[kw];
+            e[q] = pn[kw + 1];
+            b[q] = pn[ks - L.pitch];
+            t[q] = pn[ks + L.pitch];
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+            if (CC) {
+                u[q] = gs_edge(FBox<CC>(L), o.i(L, PAR, q), o.j(q), w[q], e[q], b[q], t[q], r[PAR][q], ci[PAR][q]);
+            } else {
+                double l = L.facx * (w[q] + e[q]);
+                l += L.facy * (b[q] + t[q]);
+                u[q] = (r[PAR][q] - l) * ci[PAR][q];
+            }
+            asm volatile("" : "+v"(u[q]));
+        }
+#pragma unroll
+        for (int q = 0; q < KP; ++q)
+            if (o.v[PAR][q]) phi[PAR * L.plane + o.ks(PAR, q)] = u[q];
+    }
+    f_sync<WAVE>();
 }
 
-// up-sweep step of level L: cor += I(C.cor) in place (each point reads only itself on this
-// level), then four sweeps
-template <class Mode, bool CC>
-__device__ void c_up(double* w, const CLev& L, const CLev& C) {
-    Mode::valid(L, [&](int i, int j) {
-        const int k = lat(L, i, j);
-        auto c = [&](int a, int b) { return w[C.cor + lat(C, a, b)]; };
-        w[L.cor + k] = interp_add<CC>(i, j, w[L.cor + k], c);
-    });
-    Mode::sync();
-    for (int color = 0; color < 4; ++color) c_sweep<Mode, CC>(w, L, color);
+// n sweeps, n even; ZERO: from phi = 0, whose neighbour sums are zero. The loop has one copy
+// of each colour's sweep: the kernel runs through its code once, and fetching it counts.
+template <bool CC, int KP, bool WAVE, bool ZERO>
+__device__ __forceinline__ void f_sweeps(double* w, const FLev<CC>& L, const Own<CC, KP>& o, const double (&r)[2][KP],
+                                         const double (&ci)[2][KP], int n) {
+    double* const phi = w + L.phi;
+    if (ZERO) {
+#pragma unroll
+        for (int q = 0; q < KP; ++q)
+            if (o.v[0][q]) phi[o.ks(0, q)] = r[0][q] * ci[0][q];
+        f_sync<WAVE>();
+    } else {
+        f_sweep<CC, KP, WAVE, 0>(phi, L, o, r, ci);
+    }
+#pragma unroll 1
+    for (;;) {
+        f_sweep<CC, KP, WAVE, 1>(phi, L, o, r, ci);
+        if ((n -= 2) <= 0) break;
+        f_sweep<CC, KP, WAVE, 0>(phi, L, o, r, ci);
+    }
+}
+
+// sc = residual; acf comes from sc, or from registers (REG)
+template <bool CC, int KP, bool WAVE, bool REG>
+__device__ __forceinline__ void f_residual(double* w, const FLev<CC>& L, int sc, const Own<CC, KP>& o,
+                                           const double (&r)[2][KP], double (&a)[2][KP]) {
+    if (o.any) {
+        double z[2][KP], x0[2][KP], x1[2][KP], y0[2][KP], y1[2][KP], g[2][KP];
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const double* const p = w + L.phi + par * L.plane;
+            const double* const pn = w + L.phi + (1 - par) * L.plane;
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                const int ks = o.ks(par, q), kw = o.kw(par, q);
+                z[par][q] = p[ks];
+                x0[par][q] = pn[kw];
+                x1[par][q] = pn[kw + 1];
+                y0[par][q] = pn[ks - L.pitch];
+                y1[par][q] = pn[ks + L.pitch];
+                if (!REG) a[par][q] = w[sc + par * L.plane + ks];
+            }
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int par = 0; par < 2; ++par)
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                auto P = [&](int di, int dj) {
+                    return di < 0   ? x0[par][q]
+                           : di > 0 ? x1[par][q]
+                           : dj < 0 ? y0[par][q]
+                           : dj > 0 ? y1[par][q]
+                                    : z[par][q];
+                };
+                g[par][q] =
+                    residual1<CC>(FBox<CC>(L), o.i(L, par, q), o.j(q), P, r[par][q], a[par][q], L.facx, L.facy);
+                asm volatile("" : "+v"(g[par][q]));
+            }
+#pragma unroll
+        for (int par = 0; par < 2; ++par)
+#pragma unroll
+            for (int q = 0; q < KP; ++q)
+                if (o.v[par][q]) w[sc + par * L.plane + o.ks(par, q)] = g[par][q];
+    }
+    f_sync<WAVE>();
+}
+
+// sc of level F restricted to point (i, j) of the next level: the fine centre (2 i, 2 j) and
+// its diagonal neighbours have colour 0, the others colour 1
+template <bool CC>
+__device__ __forceinline__ double f_restrict(const double* w, const FLev<CC>& F, int sc, int i, int j) {
+    const int P = F.pitch;
+    const double* const p0 = w + sc + (2 * j + 1) * P + i;
+    const double* const p1 = p0 + F.plane;
+    double f[9] = {};
+    f[4] = p0[0];
+    f[5] = p1[1];
+    f[7] = p1[P];
+    f[8] = p0[P + 1];
+    if (!CC) {
+        f[0] = p0[-P];
+        f[1] = p1[-P];
+        f[2] = p0[1 - P];
+        f[3] = p1[0];
+        f[6] = p0[P];
+    }
+    asm volatile("" ::: "memory");
+    auto A = [&](int a, int b) { return f[(b - 2 * j + 1) * 3 + (a - 2 * i) + 1]; };
+    return restrict_from<CC>(A, i, j);
+}
+
+// phi of level L += I(phi of level C)
+template <bool CC, int KP, bool WAVE>
+__device__ __forceinline__ void f_interp(double* w, const FLev<CC>& L, const FLev<CC>& C, const Own<CC, KP>& o) {
+    if (o.any) {
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            double c[4][KP], x[KP];
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                // node-centred: point (1 + 2 h + b, 1 + row) lies at or right after coarse (h + b,
+                // (row + 1) / 2); both odd or both even (colour 0), or odd along one direction
+                const int ic = CC ? o.h[q] : o.h[q] + o.b(par, q), jc = CC ? o.row[q] >> 1 : (o.row[q] + 1) >> 1;
+                const int pc = ((ic + jc) & 1) * C.plane, pd = C.plane - pc;
+                const double* const p = w + C.phi + (jc + 1) * C.pitch + ((ic + 1) >> 1);
+                const int e = 1 - (ic & 1);   // to the east neighbour's place in its row
+                c[0][q] = p[pc];
+                if (!CC && par == 0) {
+                    c[1][q] = p[pd + e];
+                    c[2][q] = p[pd + C.pitch];
+                    c[3][q] = p[pc + C.pitch + e];
+                }
+                if (!CC && par == 1) c[1][q] = p[pd + ((o.row[q] & 1) ? e : C.pitch)];
+                x[q] = w[L.phi + par * L.plane + o.ks(par, q)];
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                if (CC) {
+                    x[q] += c[0][q];
+                } else if (par == 1) {
+                    x[q] += (c[0][q] + c[1][q]) * 0.5;
+                } else {
+                    const double four = (c[0][q] + c[1][q] + c[2][q] + c[3][q]) * 0.25;
+                    x[q] += (o.row[q] & 1) ? c[0][q] : four;
+                }
+                asm volatile("" : "+v"(x[q]));
+            }
+#pragma unroll
+            for (int q = 0; q < KP; ++q)
+                if (o.v[par][q]) w[L.phi + par * L.plane + o.ks(par, q)] = x[q];
+        }
+    }
+    f_sync<WAVE>();
+}
+
+// level L below the top, fine level F with its residual at sc: rhs from that, sweeps from
+// zero; then, on all but the bottom level, the residual
+template <bool CC, bool WAVE>
+__device__ __forceinline__ void f_down(double* w, const FLev<CC>& F, int sc, const FLev<CC>& L, int sweeps,
+                                       bool bottom) {
+    const Own<CC, 1> o(L);
+    double r[2][1] = {}, ci[2][1] = {}, a[2][1];
+    if (o.any) {
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const int slot = par * L.nt + int(threadIdx.x);
+            ci[par][0] = w[L.ci + slot];
+            r[par][0] = f_restrict<CC>(w, F, sc, o.i(L, par, 0), o.j(0));
+            w[L.r + slot] = r[par][0];
+        }
+    }
+    f_sweeps<CC, 1, WAVE, true>(w, L, o, r, ci, sweeps);
+    if (!bottom) f_residual<CC, 1, WAVE, false>(w, L, L.sc, o, r, a);
+}
+
+template <bool CC, bool WAVE>
+__device__ __forceinline__ void f_up(double* w, const FLev<CC>& L, const FLev<CC>& C) {
+    const Own<CC, 1> o(L);
+    double r[2][1] = {}, ci[2][1] = {};
+    if (o.any) {
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const int slot = par * L.nt + int(threadIdx.x);
+            ci[par][0] = w[L.ci + slot];
+            r[par][0] = w[L.r + slot];
+        }
+    }
+    f_interp<CC, 1, WAVE>(w, L, C, o);
+    f_sweeps<CC, 1, WAVE, false>(w, L, o, r, ci, 4);
+}
+
+// x of the lane OFF lanes away within a row of 16 lanes, zero beyond it
+template <int OFF>
+__device__ __forceinline__ double row_lane(double x) {
+    constexpr int ctrl = OFF < 0 ? 0x110 - OFF : 0x100 + OFF;   // row_shr, row_shl
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// The bottom level of at most 3 x 3 valid points (all grids of 2^k - 1 points), node-centred, in
+// registers: point (col, row) on lane 4 row + col, whose neighbours are 1 and 4 lanes away and
+// whose border lanes hold zero. A sweep is 8 lane moves and 7 FP64 operations, 90 cycles instead
+// of 290 through LDS.
+__device__ __forceinline__ void f_bottom3(double* w, const FLev<false>& F, int sc, const FLev<false>& L, int sweeps) {
+    const int lane = int(threadIdx.x), col = lane & 3, row = lane >> 2;
+    const bool own = col < L.nvx && row < L.nvy;
+    const int par = (col + row) & 1, c = min(col, L.nvx - 1), d = min(row, L.nvy - 1);
+    const double ci = w[L.ci + ((c + d) & 1) * L.nt + d * L.hw + (c >> 1)];
+    const double r = f_restrict<false>(w, F, sc, 1 + c, 1 + d);
+    double x = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < sweeps; ++k) {
+        double l = L.facx * (row_lane<-1>(x) + row_lane<1>(x));
+        l += L.facy * (row_lane<-4>(x) + row_lane<4>(x));
+        const double u = (r - l) * ci;
+        x = own && par == (k & 1) ? u : x;
+    }
+    if (own) w[L.phi + par * L.plane + (row + 2) * L.pitch + (col >> 1) + 1] = x;
+    f_sync<true>();
+}
+
+// acf of level L from level F, whose acf is at sc, and its 1/c0 (average_down_acoef, :1641-1661)
+template <bool CC>
+__device__ __forceinline__ void f_average(double* w, const FLev<CC>& F, int sc, const FLev<CC>& L) {
+    const Own<CC, 1> o(L);
+    if (o.any) {
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const int i = o.i(L, par, 0);
+            const double a = f_restrict<CC>(w, F, sc, i, o.j(0));
+            w[L.ci + par * L.nt + int(threadIdx.x)] = c0_inverse<CC>(FBox<CC>(L), i, o.j(0), a, L.facx, L.facy);
+            if (o.v[par][0]) w[L.sc + par * L.plane + o.ks(par, 0)] = a;
+        }
+    }
+    __syncthreads();
 }
 
 // Levels [cb, maxl] of one V-cycle for component blockIdx.x: down-sweep with residual
 // restriction, bottom solve (CPU branch of MultiGrid::bottomsolve, :1583-1593), up-sweep.
-// acf and res of level cb are loaded; acf of the coarser levels is averaged down here;
-// cor of level cb is written back for the finer up-sweep.
-template <bool CC, bool IN_LDS>
-__global__ __launch_bounds__(COARSE_THREADS) void k_coarse(const CArgs A, double* __restrict__ gwork,
-                                                           const MGCtl* __restrict__ ctl) {
-    constexpr int NB = 8;   // loads in flight per thread
-    extern __shared__ double sm[];
-    const int comp = blockIdx.x;
-    double* w = IN_LDS ? sm : gwork + long(comp) * A.work_doubles;
-    const int nl = A.nlev;
-    const CLev& T = A.lv[0];
-    const int done = ctl ? ctl->done : 0;
-    const double* gres = A.res + long(comp) * A.gcs;
-    // acf, res of level cb: up to NB loads per thread in flight at once
-    const int nload = 2 * T.cs;
-    for (int b0 = 0; b0 < nload; b0 += NB * COARSE_THREADS) {
-        double v[NB];
+// KP: points of one colour per thread on level cb. acf and rhs of level cb come from global
+// memory, its correction goes back there.
+// Measured: 17.5 us from 65 x 65 points down (node-centred), 21.5 us from 64 x 64 (cell-centred).
+// Before, with the arrays in LDS alone and 512 threads, 23.5 us from 33 x 33 and 36 us from
+// 32 x 32 points, and two more launches of 8.7 us for the level above. Loading its 150 KB takes
+// 3 us; a level's step costs 300 cycles a sweep on the small levels and 780, the LDS bandwidth,
+// on the top one.
+template <bool CC, int KP>
+__global__ __launch_bounds__(FT) void k_coarse_lds(const FArgs A, const MGCtl* __restrict__ ctl) {
+    extern __shared__ double w[];
+    const int comp = blockIdx.x, nl = A.nlev, nb = A.nblock;
+    const FLev<CC> T(A.nvx, A.nvy, A.facx, A.facy, 0, A.nblob, true);
+    const int done = ctl->done;
+    const Own<CC, KP> o(T);
+    double r[2][KP], ci[2][KP], a[2][KP], bl[FNB];
+    int k[2][KP];
+    const double* const gres = A.res + long(comp) * A.gcs;
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            const int t = b0 + q * COARSE_THREADS + threadIdx.x;
-            v[q] = 0.0;
-            if (t < nload) v[q] = t < T.cs ? A.acf[t] : gres[t - T.cs];
-        }
-        if (done) return;
+    for (int par = 0; par < 2; ++par)
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            const int t = b0 + q * COARSE_THREADS + threadIdx.x;
-            if (t < nload) w[t < T.cs ? T.acf + t : T.res + (t - T.cs)] = v[q];
+        for (int q = 0; q < KP; ++q) {
+            k[par][q] = (o.j(q) + 1) * A.ldx + o.i(T, par, q) + 1;
+            r[par][q] = gres[k[par][q]];
+            ci[par][q] = A.first ? A.acf[k[par][q]] : A.c0i[k[par][q]];
         }
+    // what the sweeps do not need comes in during them
+#pragma unroll
+    for (int par = 0; par < 2; ++par)
+#pragma unroll
+        for (int q = 0; q < KP; ++q) a[par][q] = A.acf[k[par][q]];
+    if (!A.first && nl > 1) {
+#pragma unroll
+        for (int q = 0; q < FNB; ++q) bl[q] = A.gblob[min(q * FT + int(threadIdx.x), A.nblob - 1)];
     }
-    for (int l = 0; l < nl; ++l) {
-        const CLev& L = A.lv[l];
-        for (int t = threadIdx.x; t < L.cs; t += COARSE_THREADS) w[L.cor + t] = 0.0;
-    }
-    __syncthreads();
-    // average_down_acoef (:1641-1661) and the diagonal inverses
-    for (int l = 0; l < nl; ++l) {
-        const CLev& L = A.lv[l];
-        BlockMode::valid(L, [&](int i, int j) {
-            const int k = lat(L, i, j);
-            w[L.c0i + k] = c0_inverse<CC>(L, i, j, w[L.acf + k], L.facx, L.facy);
-        });
-        if (l + 1 < nl) {
-            const CLev& C = A.lv[l + 1];
-            BlockMode::valid(C, [&](int i, int j) {
-                auto fa = [&](int a, int b) { return w[L.acf + lat(L, a, b)]; };
-                w[C.acf + lat(C, i, j)] = restrict_from<CC>(fa, i, j);
-            });
+    if (done) return;
+    for (int t = 2 * int(threadIdx.x); t < A.tsc - A.nblob; t += 2 * FT)
+        *reinterpret_cast<double2*>(w + A.nblob + t) = make_double2(0.0, 0.0);
+    if (A.first) {
+#pragma unroll
+        for (int par = 0; par < 2; ++par)
+#pragma unroll
+            for (int q = 0; q < KP; ++q) {
+                ci[par][q] = c0_inverse<CC>(FBox<CC>(T), o.i(T, par, q), o.j(q), ci[par][q], T.facx, T.facy);
+                if (comp == 0 && o.v[par][q]) A.c0i[k[par][q]] = ci[par][q];
+                if (o.v[par][q]) w[A.tsc + par * T.plane + o.ks(par, q)] = a[par][q];
+            }
+        for (int t = threadIdx.x; t < A.nblob; t += FT) w[t] = 0.0;
+        __syncthreads();
+        FLev<CC> F = T;
+        for (int l = 1, sc = A.tsc; l < nl; ++l) {
+            const FLev<CC> L = F.coarser();
+            f_average<CC>(w, F, sc, L);
+            F = L;
+            sc = L.sc;
         }
+        if (comp == 0)
+            for (int t = threadIdx.x; t < A.nblob; t += FT) A.gblob[t] = w[t];
+    }
+    lds_barrier();
+    f_sweeps<CC, KP, false, true>(w, T, o, r, ci, nl == 1 ? A.bottom_sweeps : 4);
+    if (nl > 1) {
+        if (!A.first) {
+#pragma unroll
+            for (int q = 0; q < FNB; ++q) w[min(q * FT + int(threadIdx.x), A.nblob - 1)] = bl[q];
+            for (int t = FNB * FT + int(threadIdx.x); t < A.nblob; t += FT) w[t] = A.gblob[t];
+        }
+        f_residual<CC, KP, false, true>(w, T, A.tsc, o, r, a);
+        FLev<CC> F = T;
+        int sc = A.tsc;
+        for (int l = 1; l < nb; ++l) {
+            const FLev<CC> L = F.coarser();
+            f_down<CC, false>(w, F, sc, L, l == nl - 1 ? A.bottom_sweeps : 4, l == nl - 1);
+            F = L;
+            sc = L.sc;
+        }
+        if (__builtin_amdgcn_readfirstlane(int(threadIdx.x)) < 64) {
+            for (int l = nb; l < nl; ++l) {
+                const FLev<CC> L = F.coarser();
+                const bool bottom = l == nl - 1;
+                if constexpr (!CC) {
+                    if (bottom && L.nvx <= 3 && L.nvy <= 3) {
+                        f_bottom3(w, F, sc, L, A.bottom_sweeps);
+                        F = L;
+                        break;
+                    }
+                }
+                f_down<CC, true>(w, F, sc, L, bottom ? A.bottom_sweeps : 4, bottom);
+                F = L;
+                sc = L.sc;
+            }
+            for (int l = nl - 2; l >= nb; --l) {
+                const FLev<CC> L = F.finer();
+                f_up<CC, true>(w, L, F);
+                F = L;
+            }
+        } else if (nb < nl) {
+            F = F.coarser();
+        }
+        lds_barrier();
+        for (int l = min(nb, nl - 1) - 1; l >= 1; --l) {
+            const FLev<CC> L = F.finer();
+            f_up<CC, false>(w, L, F);
+            F = L;
+        }
+        f_interp<CC, KP, false>(w, T, F, o);
+        f_sweeps<CC, KP, false, false>(w, T, o, r, ci, 4);
+    }
+    double* const gcor = A.cor + long(comp) * A.gcs;
+#pragma unroll
+    for (int par = 0; par < 2; ++par)
+#pragma unroll
+        for (int q = 0; q < KP; ++q)
+            if (o.v[par][q]) gcor[k[par][q]] = w[T.phi + par * T.plane + o.ks(par, q)];
+}
+
+// Bottom solve of a bottom level that is too large for k_coarse_lds (a grid that hardly
+// coarsens): the same sweeps on the level's global arrays, one workgroup per component.
+template <bool CC>
+__global__ __launch_bounds__(FT) void k_bottom(MGLevel L, int sweeps, const MGCtl* __restrict__ ctl) {
+    if (ctl->done) return;
+    const long ck = blockIdx.x ? L.cs : 0;
+    double* const phi = L.cor + ck;
+    const int hw = (L.vihi - L.vilo + 2) / 2, np = hw * (L.vjhi - L.vjlo + 1);
+    for (int sw = 0; sw < sweeps; ++sw) {
+        for (int e = threadIdx.x; e < np; e += FT) {
+            const int j = L.vjlo + e / hw, i = L.vilo + 2 * (e % hw) + ((sw + L.vilo + j) & 1);
+            if (i > L.vihi) continue;
+            const long k = at(L, i, j);
+            const double ci = c0_inverse<CC>(L, i, j, L.acf[k], L.facx, L.facy);
+            const double rhs = L.res[k + ck];
+            auto P = [&](int a, int b) { return sw == 0 ? 0.0 : phi[k + b * L.ldx + a]; };
+            phi[k] = gs_point<CC>(L, i, j, P, rhs, ci, L.facx, L.facy);
+        }
+        // the other colour starts from zero as well
+        if (sw == 0)
+            for (int e = threadIdx.x; e < np; e += FT) {
+                const int j = L.vjlo + e / hw, i = L.vilo + 2 * (e % hw) + ((1 + L.vilo + j) & 1);
+                if (i <= L.vihi) phi[at(L, i, j)] = 0.0;
+            }
         __syncthreads();
     }
-    const int nb = A.nblock;
-    for (int l = 0; l < nb && l + 1 < nl; ++l) c_down<BlockMode, CC>(w, A.lv[l], A.lv[l + 1]);
-    if (threadIdx.x < 64) {
-        for (int l = nb; l + 1 < nl; ++l) c_down<WaveMode, CC>(w, A.lv[l], A.lv[l + 1]);
-        // bottom solve from zero (the bottom level is always a wavefront level)
-        for (int sw = 0; sw < A.bottom_sweeps; ++sw) c_sweep<WaveMode, CC>(w, A.lv[nl - 1], sw);
-        for (int l = nl - 2; l >= nb; --l) c_up<WaveMode, CC>(w, A.lv[l], A.lv[l + 1]);
-    }
-    __syncthreads();
-    for (int l = min(nb, nl - 1) - 1; l >= 0; --l) c_up<BlockMode, CC>(w, A.lv[l], A.lv[l + 1]);
-    double* gcor = A.cor + long(comp) * A.gcs;
-    for (int t = threadIdx.x; t < T.cs; t += COARSE_THREADS) gcor[t] = w[T.cor + t];
 }
 
 // level-0 load (copy path): acf, sol and rhs (2 comps) over the whole box
@@ -794,51 +1261,50 @@ bool coarsenable(bool cc, int lo, int hi, int min_width) {
     return (cdiv2(lo) * 2 == lo) && (cdiv2(hi) * 2 == hi);
 }
 
-// the single-workgroup description of levels cb..max_level
-void coarse_args(MultiGrid& M) {
-    CArgs& A = *reinterpret_cast<CArgs*>(M.coarse_args);
-    std::memset(&A, 0, sizeof(CArgs));
-    const int cb = M.coarse_begin;
-    A.nlev = M.max_level - cb + 1;
-    int off = 0;
-    for (int l = cb; l <= M.max_level; ++l) {
-        const MGLevel& G = M.lev[l];
-        CLev& L = A.lv[l - cb];
-        L.ilo = G.ilo; L.ihi = G.ihi; L.jlo = G.jlo; L.jhi = G.jhi;
-        L.vilo = G.vilo; L.vihi = G.vihi; L.vjlo = G.vjlo; L.vjhi = G.vjhi;
-        L.ldx = G.ldx;
-        L.cs = int(G.cs);
-        L.acf = off; off += L.cs;
-        L.c0i = off; off += L.cs;
-        L.res = off; off += L.cs;
-        L.cor = off; off += L.cs;
-        L.rescor = off; off += L.cs;
-        L.facx = 1. / (G.dx * G.dx);
-        L.facy = 1. / (G.dy * G.dy);
-    }
-    A.work_doubles = off;
-    // levels of more than 64 valid points run on the whole workgroup; the bottom level
-    // always on one wavefront
-    A.nblock = 0;
-    while (A.nblock < A.nlev - 1) {
-        const CLev& L = A.lv[A.nblock];
-        if ((L.vihi - L.vilo + 1) * (L.vjhi - L.vjlo + 1) <= 64) break;
-        ++A.nblock;
-    }
-    const MGLevel& B = M.lev[M.max_level];
+int bottom_sweeps(const MGLevel& B) {
     const int len = std::max(B.ihi - B.ilo + 1, B.jhi - B.jlo + 1);
-    A.bottom_sweeps = std::max(16, (len + 1) / 2 * 2);
-    const MGLevel& T = M.lev[cb];
-    A.acf = T.acf;
-    A.res = T.res;
-    A.cor = T.cor;
-    A.gcs = T.cs;
+    return std::max(16, (len + 1) / 2 * 2);
+}
+
+// the description of levels cb..max_level for k_coarse_lds, or false where they do not fit: a
+// thread would own more than FKP points of a colour, or the arrays exceed the LDS
+template <bool CC>
+bool coarse_lds_args(MultiGrid& M, int cb) {
+    const MGLevel& G = M.lev[cb];
+    FArgs A{};
+    A.nlev = M.max_level - cb + 1;
+    A.nvx = G.vihi - G.vilo + 1;
+    A.nvy = G.vjhi - G.vjlo + 1;
+    if (A.nvx > 2 * FKP * FT || A.nvy > FKP * FT) return false;
+    A.facx = G.facx;
+    A.facy = G.facy;
+    const FLev<CC> T(A.nvx, A.nvy, G.facx, G.facy, 0, 0, true);
+    FLev<CC> L = T;
+    for (int l = 0; l < A.nlev; ++l) {
+        if (l) L = L.coarser();
+        if (L.np > L.nt * (l == 0 ? FKP : 1)) return false;
+        if (l == 0 || L.nt > 64) A.nblock = l + 1;
+    }
+    A.nblob = (L.bend + 1) & ~1;
+    A.tsc = (A.nblob + L.pend + 1) & ~1;
+    M.coarse_lds_bytes = sizeof(double) * size_t(A.tsc + 2 * T.plane);
+    if (M.coarse_lds_bytes > FLDS_MAX) return false;
+    M.coarse_kp = T.np <= FT ? 1 : 2;
+    A.bottom_sweeps = bottom_sweeps(M.lev[M.max_level]);
+    A.gcs = int(G.cs);
+    A.ldx = G.ldx;
+    A.acf = G.acf;
+    A.res = G.res;
+    A.c0i = G.c0i;
+    A.cor = G.cor;
+    std::memcpy(M.coarse_args, &A, sizeof(A));
+    return true;
 }
 
 }  // namespace
 
 void mg_init(hpq_ctx* c) {
-    static_assert(sizeof(CArgs) <= sizeof(MultiGrid::coarse_args), "coarse argument block too small");
+    static_assert(sizeof(FArgs) <= sizeof(MultiGrid::coarse_args), "coarse argument block too small");
     MultiGrid& M = c->mg;
     const int nx = c->g.nx, ny = c->g.ny;
     if (nx % 2 != ny % 2) throw HpqError(HPQ_E_UNSUPPORTED, "hpmg: nx and ny must have the same parity");
@@ -876,8 +1342,11 @@ void mg_init(hpq_ctx* c) {
         L.cs = long(L.ldx) * L.ldy;
         L.dx = M.dx * double(1 << l);
         L.dy = M.dy * double(1 << l);
+        L.facx = 1. / (L.dx * L.dx);
+        L.facy = 1. / (L.dy * L.dy);
         const size_t b1 = sizeof(double) * L.cs;
         HPQ_HIP(hipMalloc(&L.acf, b1));
+        HPQ_HIP(hipMalloc(&L.c0i, b1));
         HPQ_HIP(hipMalloc(&L.res, 2 * b1));
         HPQ_HIP(hipMalloc(&L.cor, 2 * b1));
         HPQ_HIP(hipMalloc(&L.rescor, 2 * b1));
@@ -886,18 +1355,18 @@ void mg_init(hpq_ctx* c) {
         HPQ_HIP(hipMemset(L.cor, 0, 2 * b1));
         HPQ_HIP(hipMemset(L.rescor, 0, 2 * b1));
     }
+    // from the first level that k_coarse_lds can take, or the bottom level alone from global memory
     M.coarse_begin = M.max_level;
-    for (int l = 1; l <= M.max_level; ++l) {
-        const MGLevel& L = M.lev[l];
-        if ((L.ihi - L.ilo + 1) * (L.jhi - L.jlo + 1) <= COARSE_MAX_POINTS) { M.coarse_begin = l; break; }
+    M.coarse_in_lds = false;
+    for (int l = 1; l <= M.max_level && !M.coarse_in_lds; ++l) {
+        M.coarse_in_lds = M.cc ? coarse_lds_args<true>(M, l) : coarse_lds_args<false>(M, l);
+        if (M.coarse_in_lds) M.coarse_begin = l;
     }
-    if (M.max_level - M.coarse_begin + 1 > COARSE_MAX_LEVELS)
-        throw HpqError(HPQ_E_UNSUPPORTED, "hpmg: too many coarse levels");
-    coarse_args(M);
-    const CArgs& A = *reinterpret_cast<const CArgs*>(M.coarse_args);
-    M.coarse_lds_bytes = sizeof(double) * size_t(A.work_doubles);
-    M.coarse_in_lds = M.coarse_lds_bytes <= COARSE_LDS_MAX;
-    if (!M.coarse_in_lds) HPQ_HIP(hipMalloc(&M.coarse_work, 2 * M.coarse_lds_bytes));
+    if (M.coarse_in_lds) {
+        FArgs& A = *reinterpret_cast<FArgs*>(M.coarse_args);
+        HPQ_HIP(hipMalloc(&M.coarse_work, sizeof(double) * size_t(std::max(1, A.nblob))));
+        A.gblob = M.coarse_work;
+    }
     const size_t b0 = sizeof(double) * 2 * M.lev[0].cs;
     HPQ_HIP(hipMalloc(&M.msol, b0));
     HPQ_HIP(hipMalloc(&M.mrhs, b0));
@@ -907,15 +1376,18 @@ void mg_init(hpq_ctx* c) {
     HPQ_HIP(hipMemset(M.d_ctl, 0, 2 * sizeof(MGCtl)));
     {
         const MGLevel& L0 = M.lev[0];
-        const long nblk = long((L0.vihi - L0.vilo + 1 + TX - 1) / TX) * ((L0.vjhi - L0.vjlo + 1 + TY - 1) / TY);
+        // the tiles of level-0 launches have 8 x 4 points or more, for each component
+        const long nblk = 2 * long((L0.vihi - L0.vilo + 8) / 8) * ((L0.vjhi - L0.vjlo + 4) / 4);
         HPQ_HIP(hipMalloc(&M.d_norms, sizeof(double) * 2 * nblk));
     }
     HPQ_HIP(hipHostMalloc(&M.h_mirror, sizeof(MGMirror), hipHostMallocMapped | hipHostMallocCoherent));
     M.h_mirror->word = 0;
     HPQ_HIP(hipHostGetDevicePointer((void**)&M.d_mirror, M.h_mirror, 0));
     if (M.coarse_in_lds) {
-        const void* f = M.cc ? (const void*)k_coarse<true, true> : (const void*)k_coarse<false, true>;
-        HPQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(M.coarse_lds_bytes)));
+        const void* fs[2][2] = {{(const void*)k_coarse_lds<false, 1>, (const void*)k_coarse_lds<false, 2>},
+                                {(const void*)k_coarse_lds<true, 1>, (const void*)k_coarse_lds<true, 2>}};
+        HPQ_HIP(hipFuncSetAttribute(fs[M.cc][M.coarse_kp - 1], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    int(M.coarse_lds_bytes)));
     }
 }
 
@@ -936,7 +1408,7 @@ void mg_free(hpq_ctx* c) {
     MultiGrid& M = c->mg;
     if (M.hist) (void)hipFree(M.hist);
     for (auto& L : M.lev)
-        for (void* p : {(void*)L.acf, (void*)L.res, (void*)L.cor, (void*)L.rescor})
+        for (void* p : {(void*)L.acf, (void*)L.c0i, (void*)L.res, (void*)L.cor, (void*)L.rescor})
             if (p) (void)hipFree(p);
     if (M.coarse_work) (void)hipFree(M.coarse_work);
     if (M.msol) (void)hipFree(M.msol);
@@ -949,10 +1421,6 @@ void mg_free(hpq_ctx* c) {
 
 namespace {
 
-int level0_blocks(const MGLevel& L) {
-    return ((L.vihi - L.vilo + 1 + TX - 1) / TX) * ((L.vjhi - L.vjlo + 1 + TY - 1) / TY);
-}
-
 // the caller's view of one solve: level-0 rhs, acf and the two iterate buffers
 struct Solve {
     const double* rhs0;   // comp stride rcs
@@ -962,20 +1430,42 @@ struct Solve {
     MGCtl* ctl;
     MGCtl* other;
     double tol_rel, tol_abs;
+    int nblk;             // workgroups of the last level-0 launch (entries of d_norms)
 };
 
-template <int NSW, bool ZERO, bool RES, bool INTERP, bool RHSMAX = false, bool NORMS = false, bool ACF = false>
-void smooth(hpq_ctx* c, const MGLevel& L, const MGLevel& C, double* phi_out, const double* rhs, long rcs,
-            const double* acf, const double* phi_in, const double* cor_c, double* res_c, const MGCtl* gate,
-            double* norms = nullptr, const Fold& fold = Fold{}) {
+template <int NSW, bool CC, bool RES, int KP>
+dim3 smooth_grid(const MGLevel& L) {
+    using T = Tile<NSW, CC, RES, KP>;
+    return dim3(2 * ((L.vihi - L.vilo + T::TX) / T::TX), (L.vjhi - L.vjlo + T::TY) / T::TY);
+}
+
+// Returns the number of workgroups (entries of norms).
+template <int NSW, bool ZERO, bool RES, bool INTERP, bool RHSMAX = false, bool NORMS = false, bool FIRST = false>
+int smooth(hpq_ctx* c, const MGLevel& L, const MGLevel& C, double* phi_out, const double* rhs, long rcs,
+           const double* acf, const double* phi_in, const double* cor_c, double* res_c, const MGCtl* gate,
+           double* norms = nullptr, const Fold& fold = Fold{}) {
     TraceScope ts(c, HPQ_TRACE_MG_SMOOTH);
-    const dim3 grid((L.vihi - L.vilo + 1 + TX - 1) / TX, (L.vjhi - L.vjlo + 1 + TY - 1) / TY);
-    if (L.cc)
-        hipLaunchKernelGGL((k_smooth<NSW, true, ZERO, RES, INTERP, RHSMAX, NORMS, ACF>), grid, dim3(NT), 0, c->stream, L,
-                           C, phi_out, rhs, rcs, acf, phi_in, cor_c, res_c, gate, norms, fold);
-    else
-        hipLaunchKernelGGL((k_smooth<NSW, false, ZERO, RES, INTERP, RHSMAX, NORMS, ACF>), grid, dim3(NT), 0, c->stream,
-                           L, C, phi_out, rhs, rcs, acf, phi_in, cor_c, res_c, gate, norms, fold);
+    auto launch = [&](auto CCC, auto KPC) {
+        constexpr bool CC = decltype(CCC)::value;
+        constexpr int KP = decltype(KPC)::value;
+        const dim3 grid = smooth_grid<NSW, CC, RES, KP>(L);
+        hipLaunchKernelGGL((k_smooth<NSW, CC, ZERO, RES, INTERP, RHSMAX, NORMS, FIRST, KP>), grid, dim3(NT), 0,
+                           c->stream, L, C, phi_out, rhs, rcs, acf, phi_in, cor_c, res_c, gate, norms, fold);
+        return int(grid.x * grid.y);
+    };
+    // The smaller tile while all its workgroups are resident (four to a CU at one point of a
+    // colour per thread, two at two): 4.6 against 5.6 us for four sweeps of 127 x 127 points (78
+    // or 30 workgroups), 7.8 against 9.5 us for eight of 255 x 255 (228 or 108). Beyond that the
+    // larger one, which recomputes less of its surroundings: 9.0 against 16.0 us for four sweeps
+    // of 511 x 511 (480 or 1720 workgroups), 14.4 against 18.7 us for eight (432 or 888).
+    constexpr int KP = NSW == 8 ? 2 : 1;
+    constexpr unsigned resident = 256 * (NSW == 8 ? 2 : 4);
+    auto pick = [&](auto CCC) {
+        const dim3 g = smooth_grid<NSW, decltype(CCC)::value, RES, KP>(L);
+        return g.x * g.y <= resident ? launch(CCC, std::integral_constant<int, KP>{})
+                                     : launch(CCC, std::integral_constant<int, KP + 1>{});
+    };
+    return L.cc ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 // MultiGrid::vcycle (:1430-1512), V-cycle number m of the solve. Level 0's residual and
@@ -985,7 +1475,7 @@ void smooth(hpq_ctx* c, const MGLevel& L, const MGLevel& C, double* phi_out, con
 // buf[m & 1] and ends in buf[(m + 1) & 1]. fold: the convergence target (m = 0) or the end
 // of cycle m - 1 is evaluated by the cycle's first launch (level 1 down); check: the cycle
 // ends with a k_check launch that publishes its result to the host.
-void vcycle(hpq_ctx* c, const Solve& S, int m, int maxiter, bool fold, bool check) {
+void vcycle(hpq_ctx* c, Solve& S, int m, int maxiter, bool fold, bool check) {
     MultiGrid& M = c->mg;
     MGCtl* ctl = S.ctl;
     const int cb = M.coarse_begin;
@@ -997,7 +1487,7 @@ void vcycle(hpq_ctx* c, const Solve& S, int m, int maxiter, bool fold, bool chec
             f.mode = m == 0 ? Fold::TARGET : Fold::CHECK;
             f.m = m;
             f.maxiter = maxiter;
-            f.nblk = level0_blocks(S.L0);
+            f.nblk = S.nblk;
             f.tol_rel = S.tol_rel;
             f.tol_abs = S.tol_abs;
             f.norms = M.d_norms;
@@ -1012,21 +1502,18 @@ void vcycle(hpq_ctx* c, const Solve& S, int m, int maxiter, bool fold, bool chec
     }
     {
         TraceScope ts(c, HPQ_TRACE_MG_COARSE);
-        const CArgs& A = *reinterpret_cast<const CArgs*>(M.coarse_args);
         if (M.coarse_in_lds) {
-            if (M.cc)
-                hipLaunchKernelGGL((k_coarse<true, true>), dim3(2), dim3(COARSE_THREADS), M.coarse_lds_bytes,
-                                   c->stream, A, nullptr, ctl);
-            else
-                hipLaunchKernelGGL((k_coarse<false, true>), dim3(2), dim3(COARSE_THREADS), M.coarse_lds_bytes,
-                                   c->stream, A, nullptr, ctl);
+            FArgs& A = *reinterpret_cast<FArgs*>(M.coarse_args);
+            A.first = m == 0;
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(2), dim3(FT), M.coarse_lds_bytes, c->stream, A, ctl);
+            };
+            if (M.cc) M.coarse_kp == 1 ? launch(k_coarse_lds<true, 1>) : launch(k_coarse_lds<true, 2>);
+            else M.coarse_kp == 1 ? launch(k_coarse_lds<false, 1>) : launch(k_coarse_lds<false, 2>);
         } else {
-            if (M.cc)
-                hipLaunchKernelGGL((k_coarse<true, false>), dim3(2), dim3(COARSE_THREADS), 0, c->stream, A,
-                                   M.coarse_work, ctl);
-            else
-                hipLaunchKernelGGL((k_coarse<false, false>), dim3(2), dim3(COARSE_THREADS), 0, c->stream, A,
-                                   M.coarse_work, ctl);
+            const MGLevel& B = M.lev[cb];
+            hipLaunchKernelGGL(M.cc ? k_bottom<true> : k_bottom<false>, dim3(2), dim3(FT), 0, c->stream, B,
+                               bottom_sweeps(B), ctl);
         }
     }
     // Up-sweep: the result of level l >= 1 goes to rescor[l] (dead after the restriction),
@@ -1043,10 +1530,10 @@ void vcycle(hpq_ctx* c, const Solve& S, int m, int maxiter, bool fold, bool chec
     // intermediate after four sweeps is not needed.
     MGLevel& L1 = M.lev[1];
     const double* corc = (cb == 1) ? L1.cor : L1.rescor;
-    smooth<8, false, true, true, false, true>(c, S.L0, L1, S.buf[(m + 1) & 1], S.rhs0, S.rcs, S.L0.acf, S.buf[m & 1],
-                                              corc, L1.res, ctl, M.d_norms);
+    S.nblk = smooth<8, false, true, true, false, true>(c, S.L0, L1, S.buf[(m + 1) & 1], S.rhs0, S.rcs, S.L0.acf,
+                                                       S.buf[m & 1], corc, L1.res, ctl, M.d_norms);
     if (check) {
-        const Check chk{ctl, S.other, M.d_mirror, M.d_norms, level0_blocks(S.L0), ++M.seq, maxiter, 0.0, 0.0};
+        const Check chk{ctl, S.other, M.d_mirror, M.d_norms, S.nblk, ++M.seq, maxiter, 0.0, 0.0};
         hipLaunchKernelGGL(k_check, dim3(1), dim3(NT), 0, c->stream, chk);
     }
 }
@@ -1116,8 +1603,8 @@ int mg_solve1(hpq_ctx* c, double* sol, const double* rhs, const double* acf, lon
     // first V-cycle's down-sweep, the coarse ones inside k_coarse
     // initial smoothing from the guess (buf[1]) into buf[0], the iterate after zero cycles;
     // k_target then sets the convergence target from its residual and rhs max norms
-    smooth<4, false, true, false, true, true, true>(c, S.L0, L1, S.buf[0], S.rhs0, S.rcs, S.L0.acf, S.buf[1], nullptr,
-                                                    L1.res, nullptr, M.d_norms);
+    S.nblk = smooth<4, false, true, false, true, true, true>(c, S.L0, L1, S.buf[0], S.rhs0, S.rcs, S.L0.acf, S.buf[1],
+                                                             nullptr, L1.res, nullptr, M.d_norms);
     S.tol_rel = tol_rel;
     S.tol_abs = tol_abs;
     // the convergence bookkeeping rides on the first launch of the next V-cycle when there
@@ -1128,7 +1615,7 @@ int mg_solve1(hpq_ctx* c, double* sol, const double* rhs, const double* acf, lon
     const bool probe = M.last_zero && maxiter > 0;
     if (!can_fold || probe) {
         const int seq = probe ? ++M.seq : 0;
-        const Check chk0{S.ctl, S.other, M.d_mirror, M.d_norms, level0_blocks(S.L0), seq, maxiter, tol_rel, tol_abs};
+        const Check chk0{S.ctl, S.other, M.d_mirror, M.d_norms, S.nblk, seq, maxiter, tol_rel, tol_abs};
         hipLaunchKernelGGL(k_target, dim3(1), dim3(NT), 0, c->stream, chk0);
     }
     HPQ_HIP(hipGetLastError());
