@@ -585,6 +585,15 @@ void deposit_beam(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const
     deposit_beam_select(c, b, slice, store, comps, nullptr, 0);
 }
 
+// Builds a slice's ordered contributions once for repeated beam_sequences_add; false where there
+// is nothing to build (no particles, atomic deposition), and deposit_beam does it all.
+bool prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice) {
+    if (!b || slice < 0 || slice >= c->g.nz || !b->off || b->off[slice + 1] <= b->off[slice]) return false;
+    if (c->p.deposition != HPQ_DEPOSIT_ORDERED) return false;
+    beam_sequences(c, b, slice, nullptr, 0);
+    return true;
+}
+
 // only the particles whose select entry equals select_value deposit (select NULL: all)
 void deposit_beam_select(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps,
                          const int32_t* select, int select_value) {
@@ -595,7 +604,8 @@ void deposit_beam_select(hpq_ctx* c, const hpq_beam* b, int slice, double* store
     if ((comps[0] >= 0) != (comps[1] >= 0))
         throw HpqError(HPQ_E_INVALID, "deposit_current_slice: jx and jy go together");
     if (c->p.deposition == HPQ_DEPOSIT_ORDERED) {
-        deposit_beam_ordered(c, b, slice, store, comps, select, select_value);
+        beam_sequences(c, b, slice, select, select_value);
+        beam_sequences_add(c, store, comps);
         return;
     }
     TraceScope ts(c, HPQ_TRACE_BEAM_DEPOSIT);

@@ -1,11 +1,14 @@
-// Slice-store bookkeeping kernels: fill/copy/add/linear combination of planes
-// (Fields::setVal/duplicate/add, MultiFab::LinComb; src/fields/Fields.H:143-287),
+// Slice-store bookkeeping kernels: fill/copy/add of planes
+// (Fields::setVal/duplicate/add; src/fields/Fields.H:143-287),
 // Sx/Sy from the beam (Hipace::InitializeSxSyWithBeam, src/Hipace.cpp:745-790),
 // the relative B-field error of the predictor-corrector loop
-// (Fields::ComputeRelBFieldError, src/fields/Fields.cpp:1229-1286) and the per-slice
+// (Fields::ComputeRelBFieldError, src/fields/Fields.cpp:1229-1286), its guess and its mixing
+// (InitialBfieldGuess, MixAndShiftBfields, :1150-1226), and the per-slice
 // field diagnostics (sum |F| over valid cells, tests/checksum/backend/openpmd_backend.py).
 // Up to 16 planes are handled per launch so a slice-store update is one kernel; the end of
 // a slice (diagnostics, ShiftSlices and the next slice's InitializeSlices) is one pass.
+#include <algorithm>
+#include <chrono>
 #include <vector>
 
 #include "internal.hpp"
@@ -155,12 +158,6 @@ __global__ __launch_bounds__(256) void k_diag_finalize(double* __restrict__ part
     }
 }
 
-__global__ void k_lincomb(double* __restrict__ store, long plane, int dst, double a, int sa, double b, int sb) {
-    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= plane) return;
-    store[long(dst) * plane + t] = a * store[long(sa) * plane + t] + b * store[long(sb) * plane + t];
-}
-
 __global__ void k_sxsy(Geom g, const double* __restrict__ jzb, const double* __restrict__ pjx,
                        const double* __restrict__ pjy, const double* __restrict__ njx, const double* __restrict__ njy,
                        double* __restrict__ Sx, double* __restrict__ Sy) {
@@ -214,17 +211,76 @@ __global__ __launch_bounds__(256) void k_relb_rows(Geom g, const double* __restr
     }
 }
 
-__global__ __launch_bounds__(64) void k_relb_total(int ny, const double* __restrict__ rows, double* __restrict__ out) {
+// the relative error from the row sums, on every lane of a wavefront
+__device__ __forceinline__ double relb_total(int ny, const double* __restrict__ rows) {
     double a = 0.0, b = 0.0;
-    for (int j = threadIdx.x; j < ny; j += 64) {
+    for (int j = threadIdx.x & 63; j < ny; j += 64) {
         a += rows[j];
         b += rows[ny + j];
     }
     a = butterfly64(a);
     b = butterfly64(b);
-    if (threadIdx.x == 0) {
-        out[0] = a;
-        out[1] = b;
+    return a > 0. ? b / a : 0.;
+}
+
+__device__ __forceinline__ void publish(PCMirror* m, double err, unsigned long long seq) {
+    m->err = err;
+    __hip_atomic_store(&m->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(64) void k_relb_total(int ny, const double* __restrict__ rows, PCMirror* mirror,
+                                                   unsigned long long seq) {
+    const double err = relb_total(ny, rows);
+    if (threadIdx.x == 0) publish(mirror, err, seq);
+}
+
+// planes of the predictor-corrector loop, x and y
+struct PCPlanes {
+    int B[2], prev[2], iter[2], pcprev[2], next_j[2];
+};
+
+// Before the loop: InitialBfieldGuess (Fields.cpp:1150-1171), B_iter = 0 and B_prev_iter = B
+// (Hipace.cpp:956-967), one pass.
+__global__ __launch_bounds__(256) void k_pc_guess(double* __restrict__ store, long plane, PCPlanes P, double a, double b) {
+    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= plane) return;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+        const double B = a * store[long(P.prev[d]) * plane + t] + b * store[long(P.pcprev[d]) * plane + t];
+        store[long(P.B[d]) * plane + t] = B;
+        store[long(P.iter[d]) * plane + t] = 0.0;
+        store[long(P.pcprev[d]) * plane + t] = B;
+    }
+}
+
+// After an iteration's Poisson solve: the error from the row sums, its publication to the host,
+// MixAndShiftBfields (Fields.cpp:1174-1226) with the weights that follow from it and from the
+// iteration before, and the next slice's currents cleared for the next iteration. err[it & 1]
+// keeps the error; every workgroup sums the rows for itself, in one order. One launch for what
+// took eight (four linear combinations, a copy, a fill, the total and a copy to the host, which
+// waited for them): at 63 x 63 these were 18 of an iteration's 125 us, and bound by latency; it takes 4.
+constexpr int PC_BLOCKS = 1024;
+__global__ __launch_bounds__(256) void k_pc_mix(double* __restrict__ store, long plane, PCPlanes P, int ny,
+                                                const double* __restrict__ rows, double* __restrict__ err, int it,
+                                                double mix1, double mix, PCMirror* mirror, unsigned long long seq) {
+    const double e = relb_total(ny, rows);
+    const double ep = it == 1 ? e : err[(it - 1) & 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        err[it & 1] = e;
+        publish(mirror, e, seq);
+    }
+    const bool any = e != 0. || ep != 0.;
+    const double wi = any ? ep / (e + ep) : 0.5, wp = any ? e / (e + ep) : 0.5;
+    for (long t = long(blockIdx.x) * blockDim.x + threadIdx.x; t < plane; t += long(gridDim.x) * blockDim.x) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const double bi = store[long(P.iter[d]) * plane + t];
+            const double p = wi * bi + wp * store[long(P.pcprev[d]) * plane + t];
+            const long kb = long(P.B[d]) * plane + t;
+            store[kb] = mix1 * store[kb] + mix * p;
+            store[long(P.pcprev[d]) * plane + t] = bi;
+            store[long(P.next_j[d]) * plane + t] = 0.0;
+        }
     }
 }
 
@@ -261,12 +317,6 @@ void plane_add(hpq_ctx* c, double* store, const int* dst, const int* src, int nc
         }
     if (s.n == 0) return;
     hipLaunchKernelGGL(k_add, grid1d(c->g.plane, 256), dim3(256), 0, c->stream, store, c->g.plane, s);
-    HPQ_HIP(hipGetLastError());
-}
-
-void plane_lincomb(hpq_ctx* c, double* store, int dst, double a, int sa, double b, int sb) {
-    hipLaunchKernelGGL(k_lincomb, grid1d(c->g.plane, 256), dim3(256), 0, c->stream, store, c->g.plane, dst, a, sa, b,
-                       sb);
     HPQ_HIP(hipGetLastError());
 }
 
@@ -372,7 +422,9 @@ void diag_finalize(hpq_ctx* c) {
     c->diag_pending = false;
 }
 
-double rel_b_error(hpq_ctx* c, const double* store, int bx, int by, int bxi, int byi) {
+namespace {
+
+void relb_rows(hpq_ctx* c, const double* store, int bx, int by, int bxi, int byi) {
     const Geom& g = c->g;
     if (c->relb_cap < 2L * g.ny) {
         if (c->relb_rows) HPQ_HIP(hipFree(c->relb_rows));
@@ -383,12 +435,50 @@ double rel_b_error(hpq_ctx* c, const double* store, int bx, int by, int bxi, int
     hipLaunchKernelGGL(k_relb_rows, dim3((g.ny + 3) / 4), dim3(256), 0, c->stream, g, store + long(bx) * g.plane,
                        store + long(by) * g.plane, store + long(bxi) * g.plane, store + long(byi) * g.plane,
                        c->relb_rows);
-    hipLaunchKernelGGL(k_relb_total, dim3(1), dim3(64), 0, c->stream, g.ny, c->relb_rows, c->d_red);
+}
+
+// waits until the device has published sequence number c->pc_seq
+double wait_error(hpq_ctx* c) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (long spin = 0; __atomic_load_n(&c->h_pc->seq, __ATOMIC_ACQUIRE) != c->pc_seq; ++spin)
+        if ((spin & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::seconds(30)) {
+            // the device has not reported: let the stream drain, then look once more
+            HPQ_HIP(hipStreamSynchronize(c->stream));
+            if (__atomic_load_n(&c->h_pc->seq, __ATOMIC_ACQUIRE) != c->pc_seq)
+                throw HpqError(HPQ_E_HIP, "predictor-corrector: the device did not report the field error");
+            break;
+        }
+    return c->h_pc->err;
+}
+
+PCPlanes pc_planes(const Layout& L) {
+    return PCPlanes{{L.Bx, L.By}, {L.prev_Bx, L.prev_By}, {L.pciter_Bx, L.pciter_By}, {L.pcprev_Bx, L.pcprev_By},
+                    {L.next_jx, L.next_jy}};
+}
+
+}  // namespace
+
+double rel_b_error(hpq_ctx* c, const double* store, int bx, int by, int bxi, int byi) {
+    relb_rows(c, store, bx, by, bxi, byi);
+    hipLaunchKernelGGL(k_relb_total, dim3(1), dim3(64), 0, c->stream, c->g.ny, c->relb_rows, c->d_pc, ++c->pc_seq);
     HPQ_HIP(hipGetLastError());
-    HPQ_HIP(hipMemcpyAsync(c->h_red, c->d_red, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HPQ_HIP(hipStreamSynchronize(c->stream));
-    const double nB = c->h_red[0], nD = c->h_red[1];
-    return (nB > 0.) ? nD / nB : 0.;
+    return wait_error(c);
+}
+
+void pc_guess(hpq_ctx* c, double* store, double m) {
+    hipLaunchKernelGGL(k_pc_guess, grid1d(c->g.plane, 256), dim3(256), 0, c->stream, store, c->g.plane,
+                       pc_planes(c->L), 1. + m, -m);
+    HPQ_HIP(hipGetLastError());
+}
+
+double pc_error_mix(hpq_ctx* c, double* store, int it, double mix) {
+    const Layout& L = c->L;
+    relb_rows(c, store, L.Bx, L.By, L.pciter_Bx, L.pciter_By);
+    const int nblk = int(std::min<long>(PC_BLOCKS, (c->g.plane + 255) / 256));
+    hipLaunchKernelGGL(k_pc_mix, dim3(nblk), dim3(256), 0, c->stream, store, c->g.plane, pc_planes(L), c->g.ny,
+                       c->relb_rows, c->pc_err, it, 1. - mix, mix, c->d_pc, ++c->pc_seq);
+    HPQ_HIP(hipGetLastError());
+    return wait_error(c);
 }
 
 }  // namespace hpq

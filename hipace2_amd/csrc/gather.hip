@@ -20,7 +20,10 @@
 //   order   each list sorted by particle index (rank by counting inside the list); at its
 //           list position the particle's record is written;
 //   pairs   every (particle, stencil offset) pair writes its contribution at its place in its
-//           cell's sequence; each cell then adds its sequence in order.
+//           cell's sequence;
+//   sum     each cell adds its sequence in order to the plane's value. The sequences hold jx, jy
+//           and jz and depend on the beam alone: the predictor-corrector loop, which deposits
+//           the same slice's beam in every iteration, builds them once.
 #include <climits>
 #include <cmath>
 
@@ -193,9 +196,11 @@ __global__ __launch_bounds__(256) void k_lists_order_beam(Geom g, hpq_beam b, lo
 // or one wavefront per cell where the sequence is long.
 constexpr int BEAM_LONG = 32;   // longer sequences: a wavefront per cell
 
-// sequence length of every plane cell: the entries of its window lists (thread per cell)
+// sequence length of every plane cell: the entries of its window lists (thread per cell);
+// cells with long sequences are listed in longc (count at longc[0])
 template <int O>
-__global__ __launch_bounds__(256) void k_beam_seg_count(Geom g, CLView cl, int32_t* __restrict__ seg) {
+__global__ __launch_bounds__(256) void k_beam_seg_count(Geom g, CLView cl, int32_t* __restrict__ seg,
+                                                        int32_t* __restrict__ longc) {
     constexpr int S = O + 1, DELTA = shape_delta<O>();
     const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t > g.plane) return;
@@ -212,6 +217,7 @@ __global__ __launch_bounds__(256) void k_beam_seg_count(Geom g, CLView cl, int32
         len += cl.off[r + col0 + S] - cl.off[r + col0];
     }
     seg[t] = len;
+    if (len > BEAM_LONG) longc[1 + atomicAdd(&longc[0], 1)] = int32_t(t);
 }
 
 // entries of perm[a, b) (increasing) below v
@@ -270,53 +276,50 @@ __global__ __launch_bounds__(256) void k_beam_pairs(Geom g, CLView cl, const int
     contrib[2 * m + out] = sx * sy * rec[2 * n + pos];
 }
 
-// the sums of cells with short sequences (thread per cell); longer ones are listed in longc
-// (count at longc[0]) for k_beam_sum_long. jx and jy go together, as in the deposit functor.
-__global__ __launch_bounds__(256) void k_beam_sum_short(Geom g, const int32_t* __restrict__ seg,
-                                                        const double* __restrict__ contrib, long m,
-                                                        double* __restrict__ store, int cjx, int cjy, int cjz,
-                                                        int32_t* __restrict__ longc) {
-    const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= g.plane) return;
-    const int a = seg[t], e = seg[t + 1];
-    if (a == e) return;
-    if (e - a > BEAM_LONG) {
-        longc[1 + atomicAdd(&longc[0], 1)] = int32_t(t);
+// Every cell's sum, added to the plane's value in sequence order; jx and jy go together, as in
+// the deposit functor. Workgroups below nshort: a thread per cell with a short sequence. The
+// rest: a wavefront per cell of longc; chunks of 64 contributions per component are read by the
+// whole wavefront into LDS (LCH chunks in flight), and lanes 0-2 add the jx, jy and jz chunks.
+// One launch for both: the predictor-corrector loop runs it in every iteration, where a launch
+// more costs 4 us of some 70.
+__global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restrict__ seg,
+                                                  const double* __restrict__ contrib, long m,
+                                                  double* __restrict__ store, int cjx, int cjy, int cjz,
+                                                  const int32_t* __restrict__ longc, int nshort) {
+    const long ps = g.plane;
+    if (int(blockIdx.x) < nshort) {
+        const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
+        if (t >= g.plane) return;
+        const int a = seg[t], e = seg[t + 1];
+        if (a == e || e - a > BEAM_LONG) return;
+        if (cjx >= 0) {
+            double ajx = store[cjx * ps + t], ajy = store[cjy * ps + t];
+            for (int h = a; h < e; ++h) {
+                ajx += contrib[h];
+                ajy += contrib[m + h];
+            }
+            store[cjx * ps + t] = ajx;
+            store[cjy * ps + t] = ajy;
+        }
+        if (cjz >= 0) {
+            double ajz = store[cjz * ps + t];
+            for (int h = a; h < e; ++h) ajz += contrib[2 * m + h];
+            store[cjz * ps + t] = ajz;
+        }
         return;
     }
-    const long ps = g.plane;
-    if (cjx >= 0) {
-        double ajx = store[cjx * ps + t], ajy = store[cjy * ps + t];
-        for (int h = a; h < e; ++h) {
-            ajx += contrib[h];
-            ajy += contrib[m + h];
-        }
-        store[cjx * ps + t] = ajx;
-        store[cjy * ps + t] = ajy;
-    }
-    if (cjz >= 0) {
-        double ajz = store[cjz * ps + t];
-        for (int h = a; h < e; ++h) ajz += contrib[2 * m + h];
-        store[cjz * ps + t] = ajz;
-    }
-}
-
-// the sums of the listed cells, a wavefront per cell: chunks of 64 contributions per component
-// are read by the whole wavefront into LDS (the next chunk already in flight), and lanes 0-2
-// add the jx, jy and jz chunks in sequence order
-__global__ __launch_bounds__(64) void k_beam_sum_long(Geom g, const int32_t* __restrict__ seg,
-                                                      const double* __restrict__ contrib, long m,
-                                                      double* __restrict__ store, int cjx, int cjy, int cjz,
-                                                      const int32_t* __restrict__ longc) {
-    // LCH chunks of 64 contributions in flight: each chunk is read by the whole wavefront while
-    // three lanes add the previous ones in sequence order
     constexpr int LCH = 4;
-    __shared__ double buf[3][64];
-    const int lane = int(threadIdx.x);
-    const long ps = g.plane;
+    __shared__ double buf_[4][3][64];
+    const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+    double(*buf)[64] = buf_[wave];
+    // a wavefront uses its own part of the LDS, whose operations execute in order
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
     const int comp = lane == 0 ? cjx : lane == 1 ? (cjx >= 0 ? cjy : -1) : lane == 2 ? cjz : -1;
     const int nl = longc[0];
-    for (int w = int(blockIdx.x); w < nl; w += int(gridDim.x)) {
+    for (int w = (int(blockIdx.x) - nshort) * 4 + wave; w < nl; w += (int(gridDim.x) - nshort) * 4) {
         const long t = longc[1 + w];
         const int a = seg[t], e = seg[t + 1];
         double acc = comp >= 0 ? store[comp * ps + t] : 0.0;
@@ -336,11 +339,11 @@ __global__ __launch_bounds__(64) void k_beam_sum_long(Geom g, const int32_t* __r
             for (int d = 0; d < LCH; ++d) {
                 const int hc = h0 + 64 * d;
                 if (hc >= e) break;
-                __syncthreads();
+                fence();
                 buf[0][lane] = v[d][0];
                 buf[1][lane] = v[d][1];
                 buf[2][lane] = v[d][2];
-                __syncthreads();
+                fence();
                 const int hn = hc + 64 * LCH + lane;
                 if (hn < e) {
                     v[d][0] = contrib[hn];
@@ -356,6 +359,7 @@ __global__ __launch_bounds__(64) void k_beam_sum_long(Geom g, const int32_t* __r
                         double q[16];
 #pragma unroll
                         for (int k = 0; k < 16; ++k) q[k] = row[u + k];
+                        asm volatile("" ::: "memory");
 #pragma unroll
                         for (int k = 0; k < 16; ++k) acc += q[k];
                     }
@@ -364,7 +368,6 @@ __global__ __launch_bounds__(64) void k_beam_sum_long(Geom g, const int32_t* __r
             }
         }
         if (comp >= 0) store[comp * ps + t] = acc;
-        __syncthreads();
     }
 }
 
@@ -428,15 +431,14 @@ void cell_lists_free(CellLists& L) {
     L = CellLists{};
 }
 
-// ::DepositCurrentSlice in the CPU build's order (particles of `slice` whose select entry
-// equals select_value; select NULL: all)
-void deposit_beam_ordered(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps,
-                          const int32_t* select, int select_value) {
+// The contribution sequences of ::DepositCurrentSlice in the CPU build's order (particles of
+// `slice` whose select entry equals select_value; select NULL: all), for beam_sequences_add
+// until the next call. The slice has particles.
+void beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value) {
     const Geom& g = c->g;
     CellLists& L = c->cl_beam;
     const long first = b->off[slice];
     const long count = b->off[slice + 1] - first;
-    if (count <= 0) return;
     const int S = c->p.depos_order + 1;
     if (count > INT32_MAX / (S * S)) throw HpqError(HPQ_E_INVALID, "ordered beam deposition: too many particles in a slice");
     lists_geometry(c, L);
@@ -446,6 +448,7 @@ void deposit_beam_ordered(hpq_ctx* c, const hpq_beam* b, int slice, double* stor
     grow(L.longc, L.longc_cap, g.plane + 1);
     const long m = long(S) * S * count;
     grow(L.contrib, L.contrib_cap, 3 * m);
+    L.m = m;
     TraceScope ts(c, HPQ_TRACE_BEAM_DEPOSIT);
     lists_clear(c->stream, L);
     dispatch_order(c->p.depos_order, [&](auto O) {
@@ -456,15 +459,23 @@ void deposit_beam_ordered(hpq_ctx* c, const hpq_beam* b, int slice, double* stor
         lists_scatter(c->stream, L, count);
         hipLaunchKernelGGL(k_lists_order_beam<o>, grid1d(count, 256), dim3(256), 0, c->stream, g, *b, first, count,
                            L.key, L.off, L.unsorted, L.perm, L.rec);
-        hipLaunchKernelGGL(k_beam_seg_count<o>, grid1d(g.plane + 1, 256), dim3(256), 0, c->stream, g, view(L), L.seg);
+        hipLaunchKernelGGL(k_beam_seg_count<o>, grid1d(g.plane + 1, 256), dim3(256), 0, c->stream, g, view(L), L.seg,
+                           L.longc);
         scan_exclusive(c->stream, L.seg, g.plane + 1, L.segtmp);
         hipLaunchKernelGGL(k_beam_pairs<o>, grid1d(m, 256), dim3(256), 0, c->stream, g, view(L), L.key, L.rec, count,
                            L.seg, L.contrib, m);
     });
-    hipLaunchKernelGGL(k_beam_sum_short, grid1d(g.plane, 256), dim3(256), 0, c->stream, g, L.seg, L.contrib, m, store,
-                       comps[0], comps[1], comps[2], L.longc);
-    hipLaunchKernelGGL(k_beam_sum_long, dim3(2048), dim3(64), 0, c->stream, g, L.seg, L.contrib, m, store, comps[0],
-                       comps[1], comps[2], L.longc);
+    HPQ_HIP(hipGetLastError());
+}
+
+// the sequences added to the planes comps (jx, jy, jz; -1: none)
+void beam_sequences_add(hpq_ctx* c, double* store, const int32_t* comps) {
+    const Geom& g = c->g;
+    const CellLists& L = c->cl_beam;
+    TraceScope ts(c, HPQ_TRACE_BEAM_DEPOSIT);
+    const int nshort = int((g.plane + 255) / 256);
+    hipLaunchKernelGGL(k_beam_sum, dim3(nshort + 512), dim3(256), 0, c->stream, g, L.seg, L.contrib, L.m, store,
+                       comps[0], comps[1], comps[2], L.longc, nshort);
     HPQ_HIP(hipGetLastError());
 }
 

@@ -154,29 +154,13 @@ public:
         poisson_solve_staged(c_, 2, lhs);
     }
     // Fields::InitialBfieldGuess, :1150-1171
+    // with the loop's first B_iter = 0 and B_prev_iter = B
     void InitialBfieldGuess(double err, double tol) {
-        const double m = std::exp(-0.5 * std::pow(err / (2.5 * tol), 2));
-        plane_lincomb(c_, s_, L_.Bx, 1. + m, L_.prev_Bx, -m, L_.pcprev_Bx);
-        plane_lincomb(c_, s_, L_.By, 1. + m, L_.prev_By, -m, L_.pcprev_By);
+        pc_guess(c_, s_, std::exp(-0.5 * std::pow(err / (2.5 * tol), 2)));
     }
-    // Fields::MixAndShiftBfields, :1174-1226
-    void MixAndShiftBfields(double err, double err_prev, double mix) {
-        double wi, wp;
-        if (err != 0. || err_prev != 0.) {
-            wi = err_prev / (err + err_prev);
-            wp = err / (err + err_prev);
-        } else {
-            wi = 0.5;
-            wp = 0.5;
-        }
-        plane_lincomb(c_, s_, L_.pcprev_Bx, wi, L_.pciter_Bx, wp, L_.pcprev_Bx);
-        plane_lincomb(c_, s_, L_.pcprev_By, wi, L_.pciter_By, wp, L_.pcprev_By);
-        plane_lincomb(c_, s_, L_.Bx, 1. - mix, L_.Bx, mix, L_.pcprev_Bx);
-        plane_lincomb(c_, s_, L_.By, 1. - mix, L_.By, mix, L_.pcprev_By);
-        const int d[] = {L_.pcprev_Bx, L_.pcprev_By};
-        const int s[] = {L_.pciter_Bx, L_.pciter_By};
-        plane_copy(c_, s_, d, s, 2);
-    }
+    // Fields::ComputeRelBFieldError between B and B_iter, then MixAndShiftBfields, :1174-1226, and
+    // the next slice's currents cleared
+    double MixAndShiftBfields(int it, double mix) { return pc_error_mix(c_, s_, it, mix); }
     // Fields::ComputeRelBFieldError, :1229-1286
     double ComputeRelBFieldError(int bx, int by, int bxi, int byi) { return rel_b_error(c_, s_, bx, by, bxi, byi); }
 
@@ -419,28 +403,21 @@ public:
     // Hipace::PredictorCorrectorLoopToSolveBxBy, :936-1031
     void PredictorCorrectorLoopToSolveBxBy(int islice) {
         const hpq_params& P = c_->p;
-        double err_prev = 1.0;
         double err = fields_.ComputeRelBFieldError(L_.prev_Bx, L_.prev_By, L_.pcprev_Bx, L_.pcprev_By);
         fields_.InitialBfieldGuess(err, P.pc_tol);
-        const int z[] = {L_.pciter_Bx, L_.pciter_By};
-        plane_fill(c_, s_, z, 2, 0.0);
-        const int d[] = {L_.pcprev_Bx, L_.pcprev_By};
-        const int s[] = {L_.Bx, L_.By};
-        plane_copy(c_, s_, d, s, 2);
+        // the next slice's beam deposits the same in every iteration
+        const int32_t beam[3] = {L_.next_jx, L_.next_jy, -1};
+        const bool sequences = P.do_beam_jx_jy && prepare_beam(c_, b_, islice - 1);
         int it = 0;
         err = 1.0;
         while (err > P.pc_tol && it < P.pc_maxiter) {
             ++it;
             advance_plasma(c_, p_, s_, true);
             DepositCurrent(c_, p_, s_, L_.next_jx, L_.next_jy, -1, -1, -1, -1);
-            if (P.do_beam_jx_jy) DepositCurrentSlice(c_, b_, islice - 1, s_, L_.next_jx, L_.next_jy, -1);
+            if (sequences) beam_sequences_add(c_, s_, beam);
+            else if (P.do_beam_jx_jy) deposit_beam(c_, b_, islice - 1, s_, beam);
             fields_.SolvePoissonBxBy();
-            err = fields_.ComputeRelBFieldError(L_.Bx, L_.By, L_.pciter_Bx, L_.pciter_By);
-            if (it == 1) err_prev = err;
-            fields_.MixAndShiftBfields(err, err_prev, P.pc_mix);
-            const int zz[] = {L_.next_jx, L_.next_jy};
-            plane_fill(c_, s_, zz, 2, 0.0);
-            err_prev = err;
+            err = fields_.MixAndShiftBfields(it, P.pc_mix);
         }
         c_->stats[2] += it;
     }
@@ -787,8 +764,10 @@ int hpq_create(const hpq_params* p, hpq_ctx** out) {
         bins_noalloc_setup(c->device);
         HPQ_HIP(hipMalloc(&c->d_count, sizeof(int) * 4));
         HPQ_HIP(hipHostMalloc(&c->h_count, sizeof(int) * 4, hipHostMallocDefault));
-        HPQ_HIP(hipMalloc(&c->d_red, sizeof(double) * 8));
-        HPQ_HIP(hipHostMalloc(&c->h_red, sizeof(double) * 8, hipHostMallocDefault));
+        HPQ_HIP(hipMalloc(&c->pc_err, sizeof(double) * 2));
+        HPQ_HIP(hipHostMalloc(&c->h_pc, sizeof(PCMirror), hipHostMallocMapped | hipHostMallocCoherent));
+        c->h_pc->seq = 0;
+        HPQ_HIP(hipHostGetDevicePointer((void**)&c->d_pc, c->h_pc, 0));
         HPQ_HIP(hipMemset(c->d_count, 0, sizeof(int) * 4));
         poisson_init(c);
         mg_init(c);
@@ -821,8 +800,8 @@ void hpq_destroy(hpq_ctx* c) {
     if (c->diag_comp_of) (void)hipFree(c->diag_comp_of);
     if (c->d_count) (void)hipFree(c->d_count);
     if (c->h_count) (void)hipHostFree(c->h_count);
-    if (c->d_red) (void)hipFree(c->d_red);
-    if (c->h_red) (void)hipHostFree(c->h_red);
+    if (c->pc_err) (void)hipFree(c->pc_err);
+    if (c->h_pc) (void)hipHostFree(c->h_pc);
     adjoint_free(c);
     beam_slip_free(c);
     insitu_free(c);

@@ -117,6 +117,13 @@ struct MGMirror {
     unsigned long long word;
 };
 
+// What it publishes after every predictor-corrector iteration: the relative B-field error,
+// valid once seq has the expected value.
+struct PCMirror {
+    double err;
+    unsigned long long seq;
+};
+
 struct MultiGrid {
     bool cc = true;
     int max_level = 0;
@@ -204,6 +211,7 @@ struct CellLists {
     long seg_cap = 0, segtmp_cap = 0, longc_cap = 0;
     double* contrib = nullptr;
     long contrib_cap = 0;
+    long m = 0;   // (particle, stencil offset) pairs: stride of the contribution arrays
 };
 
 // Scratch of the plasma injection: per-cell particle counts and their exclusive scan.
@@ -273,8 +281,10 @@ struct hpq_ctx {
     hpq::BeamSlip slip;
     int* d_count = nullptr;          // QSA counter
     int* h_count = nullptr;          // pinned
-    double* d_red = nullptr;         // reduction scratch (8 doubles)
-    double* h_red = nullptr;         // pinned
+    double* pc_err = nullptr;        // B-field error of odd and even predictor-corrector iterations
+    hpq::PCMirror* h_pc = nullptr;   // pinned coherent host memory, and its device address
+    hpq::PCMirror* d_pc = nullptr;
+    unsigned long long pc_seq = 0;
     double* checksums = nullptr;     // caller-owned device accumulator (may be null)
     double* diag_partial = nullptr;  // per-workgroup diagnostic sums not yet in checksums
     int* diag_comp_of = nullptr;
@@ -326,11 +336,11 @@ int mg_solve1(hpq_ctx* c, double* sol, const double* rhs, const double* acf, lon
 void deposit_current(hpq_ctx* c, const hpq_plasma* p, double* store, const int32_t* comps, bool ions);
 void explicit_deposition(hpq_ctx* c, const hpq_plasma* p, double* store);
 void deposit_beam(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps);
+bool prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice);
 void advance_plasma(hpq_ctx* c, const hpq_plasma* p, const double* store, bool temp_slice);
 void plane_fill(hpq_ctx* c, double* store, const int* comps, int ncomps, double v);
 void plane_copy(hpq_ctx* c, double* store, const int* dst, const int* src, int ncomps);
 void plane_add(hpq_ctx* c, double* store, const int* dst, const int* src, int ncomps);
-void plane_lincomb(hpq_ctx* c, double* store, int dst, double a, int sa, double b, int sb);
 void sxsy_from_beam(hpq_ctx* c, double* store);
 void captures(hpq_ctx* c, const double* store, int islice);
 void slice_end(hpq_ctx* c, double* store, int islice, const int* shift_dst, const int* shift_src, int nshift,
@@ -356,6 +366,8 @@ void salame_jxjy_from_b(hpq_ctx* c, double* store);
 void salame_sums(hpq_ctx* c, const double* store, double out[4]);
 void salame_multiply(hpq_ctx* c, const hpq_beam* b, int slice, double W);
 double rel_b_error(hpq_ctx* c, const double* store, int bx, int by, int bxi, int byi);
+void pc_guess(hpq_ctx* c, double* store, double m);
+double pc_error_mix(hpq_ctx* c, double* store, int it, double mix);
 void init_plasma(hpq_ctx* c, const hpq_plasma_profile* prof, const hpq_plasma* p);
 void init_scratch_free(hpq_ctx* c);
 int64_t plasma_count(hpq_ctx* c, const hpq_plasma_profile* prof);
@@ -382,8 +394,8 @@ void scan_exclusive(hipStream_t s, int32_t* a, long n, int32_t* tmp);
 long scan_tmp_size(long n);
 void deposit_current_ordered(hpq_ctx* c, const hpq_plasma* p, double* store, const int32_t* comps, bool ions);
 void explicit_deposition_ordered(hpq_ctx* c, const hpq_plasma* p, double* store);
-void deposit_beam_ordered(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps,
-                          const int32_t* select, int select_value);
+void beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value);
+void beam_sequences_add(hpq_ctx* c, double* store, const int32_t* comps);
 void plasma_order_free(PlasmaOrder& L);
 void cell_lists_free(CellLists& L);
 void sort_beam_slices(hpq_ctx* c, hpq_beam_state* b, int64_t* off_out);
