@@ -22,7 +22,8 @@ OBJDIR = os.path.join(HERE, "_build")
 SOURCES = ["poisson.hip", "mg.hip", "particles.hip", "deposit.hip", "bins.hip", "dst_mfma.hip", "adjoint.hip", "insitu.hip", "salame.hip", "fields.hip", "gather.hip", "ordered.hip", "particles_f32.hip", "deposit_f32.hip", "hipace.cpp"]
 # sources a translation unit includes besides the headers
 INCLUDES = {"particles_f32.hip": ["particles.hip"], "deposit_f32.hip": ["deposit.hip"]}
-HEADERS = ["internal.hpp", "shape.hpp", "push.hpp", "tangent.hpp", "ordered.hpp", os.path.join("..", "..", "include", "hpq.h")]
+HEADERS = ["internal.hpp", "shape.hpp", "push.hpp", "tangent.hpp", "barrier.hpp", "ordered.hpp",
+           os.path.join("..", "..", "include", "hpq.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("HPQ_ARCH", "gfx950")

@@ -32,6 +32,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "barrier.hpp"
 #include "internal.hpp"
 
 namespace hpq {
@@ -60,14 +61,6 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by) {
 template <class LV>
 __device__ __forceinline__ bool in_valid(const LV& L, int i, int j) {
     return i >= L.vilo && i <= L.vihi && j >= L.vjlo && j <= L.vjhi;
-}
-// Barrier of a workgroup whose wavefronts exchange data through LDS alone: unlike
-// __syncthreads it does not wait for global loads, which stay in flight across the sweeps.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
 }
 __host__ __device__ __forceinline__ int cdiv2(int v) { return v >= 0 ? v / 2 : -((-v + 1) / 2); }
 

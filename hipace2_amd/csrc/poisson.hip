@@ -1,5 +1,5 @@
-// Transverse Dirichlet Poisson solver on gfx950: batched DST-I along rows in LDS,
-// LDS-tiled transposes between the x and y passes, eigenvalue scaling fused into the
+// Transverse Dirichlet Poisson solver on gfx950: batched DST-I along rows in LDS that leave
+// their output transposed for the other direction's pass, eigenvalue scaling fused into the
 // middle pass. Solves up to three fields (Psi, Ez, Bz) per call so each launch has
 // 3 x n rows of work.
 //
@@ -13,10 +13,12 @@
 // 64 KiB). With F = FFT(a + i b), RODFT00(a)_{k-1} = -Im F_k and RODFT00(b)_{k-1} = Re F_k.
 // Other n: direct sums over the sine matrix in tiles of rows and columns (n <= DST_MAT_MAX), or
 // with an exactly reduced sine table, one row per workgroup.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <utility>
 
+#include "barrier.hpp"
 #include "internal.hpp"
 
 namespace hpq {
@@ -33,7 +35,10 @@ __device__ __forceinline__ double* row_ptr(const Rows& R, int r) {
     return R.base[f] + long(j) * R.stride;
 }
 
+// Threads of an FFT row workgroup: a 4-point butterfly each, up to 256 of them with NB each
+// beyond (M = 2048: 2, 4096: 4), so that short rows are not held up by idle wavefronts.
 constexpr int DST_T = 256;
+static int fft_threads(int M) { return std::min(DST_T, std::max(64, M / 4)); }
 
 // complex a * w
 __device__ __forceinline__ double2 cmul(double2 x, double2 w) {
@@ -52,61 +57,76 @@ __device__ __forceinline__ int sw(int i) {
 
 // In-place radix-2 DIT FFT of the bit-reversed sequence a[0..M): the stages are taken in
 // pairs (a 4-point butterfly per thread and one barrier per pair); the arithmetic is that
-// of the radix-2 stages. tw[k] = exp(-2 pi i k / M).
+// of the radix-2 stages. tw[k] = exp(-2 pi i k / M). Twiddles of a pair are loaded before the
+// barrier that ends the one before.
+template <int NB>
 __device__ void fft_lds(double2* a, int M, int logM, const double2* __restrict__ tw) {
+    const int T = int(blockDim.x);
+    double2 w1[NB], w2[NB], w3[NB];
+    auto load = [&](int s) {
+        // the last stage alone: butterflies b and b + M / 4
+        const bool last = s >= logM;
+        const int h = 1 << (s - 1), half = M >> 1;
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const int b = int(threadIdx.x) + q * T, k = b & (h - 1);
+            w1[q] = tw[last ? b & (half - 1) : k * (M >> s)];
+            w2[q] = tw[last ? (b + (M >> 2)) & (half - 1) : k * (M >> (s + 1))];
+            w3[q] = tw[last ? 0 : (k + h) * (M >> (s + 1))];
+        }
+    };
+    load(1);
     int s = 1;
     for (; s + 1 <= logM; s += 2) {
         const int h = 1 << (s - 1);
-        const int st1 = M >> s, st2 = M >> (s + 1);
-        for (int b = threadIdx.x; b < (M >> 2); b += DST_T) {
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const int b = int(threadIdx.x) + q * T;
+            if (NB == 1 && b >= (M >> 2)) continue;
             const int k = b & (h - 1);
             const int i0 = ((b >> (s - 1)) << (s + 1)) + k;
             const int i1 = i0 + h, i2 = i0 + 2 * h, i3 = i0 + 3 * h;
-            const double2 w1 = tw[k * st1], w2 = tw[k * st2], w3 = tw[(k + h) * st2];
             const double2 a0 = a[sw(i0)], a1 = a[sw(i1)], a2 = a[sw(i2)], a3 = a[sw(i3)];
-            const double2 v1 = cmul(a1, w1), v3 = cmul(a3, w1);
+            const double2 v1 = cmul(a1, w1[q]), v3 = cmul(a3, w1[q]);
             const double2 x0 = make_double2(a0.x + v1.x, a0.y + v1.y), x1 = make_double2(a0.x - v1.x, a0.y - v1.y);
             const double2 x2 = make_double2(a2.x + v3.x, a2.y + v3.y), x3 = make_double2(a2.x - v3.x, a2.y - v3.y);
-            const double2 u2 = cmul(x2, w2), u3 = cmul(x3, w3);
+            const double2 u2 = cmul(x2, w2[q]), u3 = cmul(x3, w3[q]);
             a[sw(i0)] = make_double2(x0.x + u2.x, x0.y + u2.y);
             a[sw(i2)] = make_double2(x0.x - u2.x, x0.y - u2.y);
             a[sw(i1)] = make_double2(x1.x + u3.x, x1.y + u3.y);
             a[sw(i3)] = make_double2(x1.x - u3.x, x1.y - u3.y);
         }
-        __syncthreads();
+        load(s + 2);
+        lds_barrier();
     }
     if (s == logM) {   // odd number of stages: the last one alone
-        const int half = 1 << (s - 1);
-        const int step = M >> s;
-        for (int b = threadIdx.x; b < (M >> 1); b += DST_T) {
-            const int k = b & (half - 1);
-            const int i0 = ((b >> (s - 1)) << s) + k;
-            const int i1 = i0 + half;
-            const double2 u = a[sw(i0)];
-            const double2 v = cmul(a[sw(i1)], tw[k * step]);
-            a[sw(i0)] = make_double2(u.x + v.x, u.y + v.y);
-            a[sw(i1)] = make_double2(u.x - v.x, u.y - v.y);
+        const int half = M >> 1;
+        auto two = [&](int b, double2 w) {
+            const double2 u = a[sw(b)];
+            const double2 v = cmul(a[sw(b + half)], w);
+            a[sw(b)] = make_double2(u.x + v.x, u.y + v.y);
+            a[sw(b + half)] = make_double2(u.x - v.x, u.y - v.y);
+        };
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+            const int b = int(threadIdx.x) + q * T;
+            if (NB == 1 && b >= (M >> 2)) continue;
+            two(b, w1[q]);
+            two(b + (M >> 2), w2[q]);
         }
-        __syncthreads();
+        lds_barrier();
     }
 }
 
-// Two rows per workgroup: a + i b odd-extended to length M, bit-reversed into LDS.
-// v(m) gives the pair of values at m in [1, n].
-template <class V>
-__device__ __forceinline__ void load_odd_extension(double2* a, int n, int M, int logM, V v) {
-    const int N = M >> 1;
-    for (int m = threadIdx.x; m < M; m += DST_T) {
-        double2 x = make_double2(0.0, 0.0);
-        if (m >= 1 && m <= n) {
-            x = v(m);
-        } else if (m > N) {
-            const double2 y = v(M - m);
-            x = make_double2(-y.x, -y.y);
-        }
-        a[sw(__brev(unsigned(m)) >> (32 - logM))] = x;
+// entry m of the odd extension and its image, bit-reversed into LDS; m = 0 sets the two zeros
+__device__ __forceinline__ void put_odd(double2* a, int m, int M, int logM, double2 x) {
+    auto at = [&](int k) -> double2& { return a[sw(__brev(unsigned(k)) >> (32 - logM))]; };
+    if (m == 0) {
+        at(0) = at(M >> 1) = make_double2(0.0, 0.0);
+    } else {
+        at(m) = x;
+        at(M - m) = make_double2(-x.x, -x.y);
     }
-    __syncthreads();
 }
 
 // Rows r0, r0 + 1: RODFT00 of each (with F = FFT of the packed odd extension,
@@ -123,80 +143,98 @@ struct Shift {
     double inv_count = 0.0, inv_f = 0.0;
 };
 
-template <bool SYM>
+//
+// TRANS: the output goes to [field][entry][row], the rows of the other direction's pass, 16
+// bytes of an entry's line per workgroup; the workgroups of one XCD hold neighbouring rows,
+// whose pieces meet in its L2. Bound by latency: a row pair is one chain of LDS stages. A solve
+// of three fields is three launches, 14.4 us at 63 x 63, 40 us at 511 x 511, 130 us at
+// 1023 x 1023; with two launches of transposes, twiddles loaded after each barrier and 256
+// threads for every length it was 22.7, 52.6 and 154 us.
+template <bool SYM, bool TRANS, int NB>
 __global__ __launch_bounds__(DST_T) void k_dst_rows_fft(Rows in, Rows out, int nrows, int n, int M, int logM,
                                                         const double2* __restrict__ tw,
                                                         const double* __restrict__ scale, Shift shift, int add) {
     extern __shared__ double2 a[];
     __shared__ double sigma_s;
+    const int T = int(blockDim.x), tid = int(threadIdx.x);
     double sh = 0.0;
     if (shift.parts) {
-        if (threadIdx.x < 64) {
+        if (tid < 64) {
             double t = 0.0;
-            for (int q = threadIdx.x; q < shift.n; q += 64) t += shift.parts[q];
+            for (int q = tid; q < shift.n; q += 64) t += shift.parts[q];
             for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
-            if (threadIdx.x == 0) sigma_s = t * shift.inv_count;
+            if (tid == 0) sigma_s = t * shift.inv_count;
         }
         __syncthreads();
         sh = sigma_s;
     }
     auto shifted = [&](double s) { return shift.parts ? s / (1.0 - sh * s * shift.inv_f) : s; };
-    const int r0 = 2 * blockIdx.x, r1 = r0 + 1;
+    // workgroups go to the eight XCDs in turn: each XCD takes an eighth of the row pairs
+    const int npair = int(gridDim.x), full = npair & ~7, id = int(blockIdx.x);
+    const int pair = id < full ? (id & 7) * (full >> 3) + (id >> 3) : id;
+    const int r0 = 2 * pair, r1 = r0 + 1;
     const bool has1 = r1 < nrows;
     const double* p0 = row_ptr(in, r0);
     const double* p1 = has1 ? row_ptr(in, r1) : p0;
-    load_odd_extension(a, n, M, logM, [&](int m) { return make_double2(p0[m - 1], has1 ? p1[m - 1] : 0.0); });
-    fft_lds(a, M, logM, tw);
     const double* s0 = scale ? scale + long(r0 % in.rows_per_field) * n : nullptr;
     const double* s1 = (scale && has1) ? scale + long(r1 % in.rows_per_field) * n : nullptr;
+    // entries m = tid + q T of [0, n]; n + 1 = M / 2 is a multiple of 32
+    double2 v[2 * NB];
+#pragma unroll
+    for (int q = 0; q < 2 * NB; ++q) {
+        const int m = tid + q * T, k = min(max(m - 1, 0), n - 1);
+        v[q] = make_double2(p0[k], has1 ? p1[k] : 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < 2 * NB; ++q)
+        if (tid + q * T <= n) put_odd(a, tid + q * T, M, logM, v[q]);
+    lds_barrier();
+    fft_lds<NB>(a, M, logM, tw);
+    // entry m of the transform of both rows: RODFT00(a)_{m-1} = -Im F_m, RODFT00(b)_{m-1} = Re F_m
+    auto result = [&](int m, const double* t0, const double* t1) {
+        const double2 F = a[sw(m)];
+        double2 o = make_double2(-F.y, F.x);
+        if (t0) o.x *= shifted(t0[m - 1]);
+        if (t1) o.y *= shifted(t1[m - 1]);
+        return o;
+    };
     if (SYM) {
-        // RODFT00 of the scaled rows: pack them again; F_m is read for m in [1, n] only,
-        // so the new sequence goes through registers (each thread M / DST_T entries)
-        constexpr int MAXQ = 4096 / DST_T;
-        double2 nv[MAXQ];
-        const int N = M >> 1;
+        // RODFT00 of the scaled rows: pack them again, through registers
 #pragma unroll
-        for (int q = 0; q < MAXQ; ++q) {
-            const int m = threadIdx.x + q * DST_T;
-            nv[q] = make_double2(0.0, 0.0);
-            if (m < M) {
-                const int src = (m >= 1 && m <= n) ? m : (m > N ? M - m : 0);
-                if (src) {
-                    const double2 F = a[sw(src)];
-                    double o0 = -F.y, o1 = F.x;
-                    if (s0) o0 *= shifted(s0[src - 1]);
-                    if (s1) o1 *= shifted(s1[src - 1]);
-                    if (!has1) o1 = 0.0;
-                    nv[q] = m <= n ? make_double2(o0, o1) : make_double2(-o0, -o1);
-                }
-            }
+        for (int q = 0; q < 2 * NB; ++q) {
+            const int m = tid + q * T;
+            v[q] = make_double2(0.0, 0.0);
+            if (m >= 1 && m <= n) v[q] = result(m, s0, s1);
+            if (!has1) v[q].y = 0.0;
         }
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
-        for (int q = 0; q < MAXQ; ++q) {
-            const int m = threadIdx.x + q * DST_T;
-            if (m < M) a[sw(__brev(unsigned(m)) >> (32 - logM))] = nv[q];
-        }
-        __syncthreads();
-        fft_lds(a, M, logM, tw);
+        for (int q = 0; q < 2 * NB; ++q)
+            if (tid + q * T <= n) put_odd(a, tid + q * T, M, logM, v[q]);
+        lds_barrier();
+        fft_lds<NB>(a, M, logM, tw);
         s0 = s1 = nullptr;
     }
-    double* q0 = row_ptr(out, r0);
-    double* q1 = has1 ? row_ptr(out, r1) : nullptr;
+    const int f0 = r0 / in.rows_per_field, f1 = r1 / in.rows_per_field;
+    const int j0 = r0 - f0 * in.rows_per_field, j1 = r1 - f1 * in.rows_per_field;
+    double* q0 = TRANS ? out.base[f0] + j0 : row_ptr(out, r0);
+    double* q1 = !has1 ? nullptr : TRANS ? out.base[f1] + j1 : row_ptr(out, r1);
     // entries m = k + 1 in [1, n], lanes on aligned runs of m
-    for (int m = threadIdx.x; m <= n; m += DST_T) {
-        if (m == 0) continue;
-        const int k = m - 1;
-        const double2 F = a[sw(m)];
-        double o0 = -F.y, o1 = F.x;
-        if (s0) o0 *= shifted(s0[k]);
-        if (s1) o1 *= shifted(s1[k]);
+#pragma unroll
+    for (int q = 0; q < 2 * NB; ++q) {
+        const int m = tid + q * T;
+        if (m < 1 || m > n) continue;
+        const double2 o = result(m, s0, s1);
+        const long k = TRANS ? long(m - 1) * in.rows_per_field : m - 1;
         if (add) {
-            q0[k] += o0;
-            if (has1) q1[k] += o1;
+            q0[k] += o.x;
+            if (has1) q1[k] += o.y;
+        } else if (TRANS && has1 && q1 == q0 + 1) {
+            struct alignas(8) Pair { double x, y; };
+            *reinterpret_cast<Pair*>(q0 + k) = Pair{o.x, o.y};
         } else {
-            q0[k] = o0;
-            if (has1) q1[k] = o1;
+            q0[k] = o.x;
+            if (has1) q1[k] = o.y;
         }
     }
 }
@@ -349,18 +387,26 @@ __global__ __launch_bounds__(256) void k_transpose(const double* __restrict__ in
 }
 
 // RODFT00 of nrows rows (times the eigenvalue rows when scale != null); sym (FFT path): followed
-// by the inverse transform of the same rows in LDS; trans (matrix path): the output transposed
+// by the inverse transform of the same rows in LDS; trans (FFT path, always with sym, and matrix
+// path): the output transposed
 static void dst_rows(hpq_ctx* c, const DstPlan& P, const Rows& in, const Rows& out, int nrows, const double* scale,
                      bool sym = false, const Shift& shift = Shift{}, bool add = false, bool trans = false) {
     TraceScope ts(c, HPQ_TRACE_DST);
     if (P.fft) {
         const size_t lds = size_t(P.M) * sizeof(double2);
-        if (sym)
-            hipLaunchKernelGGL(k_dst_rows_fft<true>, dim3((nrows + 1) / 2), dim3(DST_T), lds, c->stream, in, out,
-                               nrows, P.n, P.M, P.logM, P.tw, scale, shift, int(add));
-        else
-            hipLaunchKernelGGL(k_dst_rows_fft<false>, dim3((nrows + 1) / 2), dim3(DST_T), lds, c->stream, in, out,
-                               nrows, P.n, P.M, P.logM, P.tw, scale, shift, int(add));
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((nrows + 1) / 2), dim3(fft_threads(P.M)), lds, c->stream, in, out, nrows,
+                               P.n, P.M, P.logM, P.tw, scale, shift, int(add));
+        };
+        auto pick = [&](auto NB) {
+            constexpr int nb = decltype(NB)::value;
+            if (sym) launch(k_dst_rows_fft<true, true, nb>);
+            else if (trans) launch(k_dst_rows_fft<false, true, nb>);
+            else launch(k_dst_rows_fft<false, false, nb>);
+        };
+        if (P.M <= 1024) pick(std::integral_constant<int, 1>{});
+        else if (P.M == 2048) pick(std::integral_constant<int, 2>{});
+        else pick(std::integral_constant<int, 4>{});
     } else {
         if (shift.parts || add) throw HpqError(HPQ_E_UNSUPPORTED, "shifted DST solve: n + 1 must be a power of two");
         if (P.mat) {
@@ -475,7 +521,7 @@ static void solve_fft(hpq_ctx* c, int nf, double* const* lhs_planes, Shift shift
     const Shift none{};
     // x pass on rows j: bufA -> rows i in P
     double *P, *Q;
-    if (S.px.mat) {
+    if (S.px.fft || S.px.mat) {
         dst_rows(c, S.px, rows(S.bufA, nx, ny), rows(S.bufB, ny, nx), nf * ny, nullptr, false, none, false, true);
         P = S.bufB;
         Q = S.bufA;
@@ -488,8 +534,7 @@ static void solve_fft(hpq_ctx* c, int nf, double* const* lhs_planes, Shift shift
     // y pass, eigenvalue scaling, inverse y pass on rows i in P (one launch on the FFT path),
     // leaving rows j in Q
     if (S.py.fft) {
-        dst_rows(c, S.py, rows(P, ny, nx), rows(P, ny, nx), nf * nx, S.eigT, true, shift);
-        transpose(P, Q, nx, ny);
+        dst_rows(c, S.py, rows(P, ny, nx), rows(Q, nx, ny), nf * nx, S.eigT, true, shift, false, true);
     } else {
         dst_rows(c, S.py, rows(P, ny, nx), rows(Q, ny, nx), nf * nx, S.eigT, false, shift);
         if (S.py.mat) {
