@@ -324,14 +324,14 @@ __device__ PushOut<N> push_tan(const Geom& g, const hpq_plasma& p, long ip, cons
     constexpr int nsub = 4;
     const double sdz = dz / nsub;
     T ux = seed(p.ux_half_step[ip], 2), uy = seed(p.uy_half_step[ip], 3), psi = seed(p.psi_half_step[ip], 4);
-    const T cir(clight_inv), qmr(qmc);
+    const double cir = clight_inv, qmr = qmc;
     auto substep = [&]() {
         const T psi_inv = 1.0 / psi;
         T dux, duy, dpsi;
-        momentum_rhs<T, T>(ux, uy, psi_inv, G[0], G[1], G[2], G[3], G[4], G[5], cir, qmr, dux, duy, dpsi);
+        momentum_rhs(ux, uy, psi_inv, G[0], G[1], G[2], G[3], G[4], G[5], cir, qmr, dux, duy, dpsi);
         const Dual<T> uxd{ux, dux}, uyd{uy, duy}, pid{psi_inv, -psi_inv * psi_inv * dpsi};
         Dual<T> ddux(T(0.0)), dduy(T(0.0)), ddpsi(T(0.0));
-        momentum_rhs<Dual<T>, T>(uxd, uyd, pid, G[0], G[1], G[2], G[3], G[4], G[5], cir, qmr, ddux, dduy, ddpsi);
+        momentum_rhs(uxd, uyd, pid, G[0], G[1], G[2], G[3], G[4], G[5], cir, qmr, ddux, dduy, ddpsi);
         ux = ux + sdz * dux + 0.5 * sdz * sdz * ddux.e;
         uy = uy + sdz * duy + 0.5 * sdz * sdz * dduy.e;
         psi = psi + sdz * dpsi + 0.5 * sdz * sdz * ddpsi.e;

@@ -40,7 +40,99 @@ __device__ __forceinline__ bool enforce_bc(const BC& bc, double& x, double& y, d
     return false;
 }
 
+// Fields at a particle (src/particles/particles_utils/FieldGather.H:45-96, nodal): Psi
+// through the nodal derivative's W x W = (O + 2)^2 cells, the others through their O + 1 by O + 1
+// cells of it with a weight other than zero (the shape function is zero on the first or the
+// last column, and row). Every accumulator sums its cells in (iy, ix) order, as the reference's cell
+// loop does; what is left out added zeros.
+template <class R>
+struct Gathered {
+    R ExmBy = 0, EypBx = 0, Ez = 0, Bx = 0, By = 0, Bz = 0;
+};
+template <int O, class R>
+__device__ __forceinline__ Gathered<R> gather_fields(const Geom& g, const double* __restrict__ store, int cPsi, int cEz,
+                                                     int cBx, int cBy, int cBz, double xp, double yp) {
+    const double xm = (xp - g.xoff) * g.dxi, ym = (yp - g.yoff) * g.dyi;
+    const double* Psi = store + long(cPsi) * g.plane;
+    const double* Ez = store + long(cEz) * g.plane;
+    const double* Bx = store + long(cBx) * g.plane;
+    const double* By = store + long(cBy) * g.plane;
+    const double* Bz = store + long(cBz) * g.plane;
+    constexpr int W = O + 2, N = O + 1;
+    const R dxi = R(g.dxi), dyi = R(g.dyi);
+    Gathered<R> G;
+    DsfR<R> sx[W], sy[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+        sx[k] = dshape<1, O, R>(xm, k);
+        sy[k] = dshape<1, O, R>(ym, k);
+    }
+    if (in_store(g, sx[0].cell, sy[0].cell) && in_store(g, sx[W - 1].cell, sy[W - 1].cell)) {
+        // the whole stencil lies in the guarded plane: a field's loads are issued together
+        const long k0 = g.idx(sx[0].cell, sy[0].cell);
+        {
+            R v[W][W];
+#pragma unroll
+            for (int iy = 0; iy < W; ++iy)
+#pragma unroll
+                for (int ix = 0; ix < W; ++ix) v[iy][ix] = R(Psi[k0 + long(iy) * g.ldx + ix]);
+#pragma unroll
+            for (int iy = 0; iy < W; ++iy)
+#pragma unroll
+                for (int ix = 0; ix < W; ++ix) {
+                    G.ExmBy += (sx[ix].ds * sy[iy].s) * v[iy][ix] * dxi;
+                    G.EypBx += (sx[ix].s * sy[iy].ds) * v[iy][ix] * dyi;
+                }
+        }
+        // the first of the O + 1 columns and rows
+        const bool x1 = sx[W - 1].s != R(0), y1 = sy[W - 1].s != R(0);
+        R s[N][N];
+#pragma unroll
+        for (int iy = 0; iy < N; ++iy)
+#pragma unroll
+            for (int ix = 0; ix < N; ++ix)
+                s[iy][ix] = (x1 ? sx[ix + 1].s : sx[ix].s) * (y1 ? sy[iy + 1].s : sy[iy].s);
+        const long k1 = k0 + (x1 ? 1 : 0) + (y1 ? g.ldx : 0);
+        auto plain = [&](const double* F, R& acc) {
+            R v[N][N];
+#pragma unroll
+            for (int iy = 0; iy < N; ++iy)
+#pragma unroll
+                for (int ix = 0; ix < N; ++ix) v[iy][ix] = R(F[k1 + long(iy) * g.ldx + ix]);
+#pragma unroll
+            for (int iy = 0; iy < N; ++iy)
+#pragma unroll
+                for (int ix = 0; ix < N; ++ix) acc += s[iy][ix] * v[iy][ix];
+        };
+        plain(Ez, G.Ez);
+        plain(Bx, G.Bx);
+        plain(By, G.By);
+        plain(Bz, G.Bz);
+    } else {
+#pragma unroll 1
+        for (int iy = 0; iy < W; ++iy) {
+#pragma unroll 1
+            for (int ix = 0; ix < W; ++ix) {
+                const DsfR<R> X = dshape<1, O, R>(xm, ix), Y = dshape<1, O, R>(ym, iy);
+                if (!in_store(g, X.cell, Y.cell)) continue;
+                const long k = g.idx(X.cell, Y.cell);
+                G.ExmBy += (X.ds * Y.s) * R(Psi[k]) * dxi;
+                G.EypBx += (X.s * Y.ds) * R(Psi[k]) * dyi;
+                G.Ez += (X.s * Y.s) * R(Ez[k]);
+                G.Bx += (X.s * Y.s) * R(Bx[k]);
+                G.By += (X.s * Y.s) * R(By[k]);
+                G.Bz += (X.s * Y.s) * R(Bz[k]);
+            }
+        }
+    }
+    return G;
+}
+
 // AdvancePlasmaParticles, src/particles/pusher/PlasmaParticleAdvance.cpp:84-240 (leapfrog)
+// Bound by FP64 issue: 861 multiplies and adds per particle at order 2 (263 of them the gather,
+// 102 a sub-step), 33 us of 41.6 at 511 x 511, 2 x 2 particles per cell. With the whole nodal
+// stencil for every field and dual-number constants it was 1122 and 49 us. Fewer registers (five
+// or six wavefronts per SIMD instead of four) spill: 64 and 132 us.
 template <int O, class R>
 __global__ __launch_bounds__(256) void k_push_plasma(Geom g, hpq_plasma p, const double* __restrict__ store, int cPsi,
                                                      int cEz, int cBx, int cBy, int cBz, double qmc, BC bc,
@@ -51,92 +143,30 @@ __global__ __launch_bounds__(256) void k_push_plasma(Geom g, hpq_plasma p, const
     // the round-robin order: their window flushes contend less when neighbouring chunks sit
     // on different XCDs.
     const long ip = long(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
-    if (ip >= p.n || !p.valid[ip]) return;
+    if (ip >= p.n) return;
     const double clight = 1.0, clight_inv = 1.0 / 1.0;
     const double dz = g.dz / 1;
+    // the particle's values in flight together, those of the sub-steps during the gather
+    const int32_t valid = p.valid[ip];
     double xp = p.x_prev[ip], yp = p.y_prev[ip];
-    R ExmByp = 0, EypBxp = 0, Ezp = 0, Bxp = 0, Byp = 0, Bzp = 0;
-    {
-        const double xm = (xp - g.xoff) * g.dxi, ym = (yp - g.yoff) * g.dyi;
-        const double* Psi = store + long(cPsi) * g.plane;
-        const double* Ez = store + long(cEz) * g.plane;
-        const double* Bx = store + long(cBx) * g.plane;
-        const double* By = store + long(cBy) * g.plane;
-        const double* Bz = store + long(cBz) * g.plane;
-        constexpr int W = O + 2;
-        const R dxi = R(g.dxi), dyi = R(g.dyi);
-        DsfR<R> sx[W], sy[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-            sx[k] = dshape<1, O, R>(xm, k);
-            sy[k] = dshape<1, O, R>(ym, k);
-        }
-        auto accumulate = [&](const DsfR<R>& X, const DsfR<R>& Y, R ps, R ez, R bx, R by, R bz) {
-            ExmByp += (X.ds * Y.s) * ps * dxi;
-            EypBxp += (X.s * Y.ds) * ps * dyi;
-            Ezp += (X.s * Y.s) * ez;
-            Bxp += (X.s * Y.s) * bx;
-            Byp += (X.s * Y.s) * by;
-            Bzp += (X.s * Y.s) * bz;
-        };
-        if (in_store(g, sx[0].cell, sy[0].cell) && in_store(g, sx[W - 1].cell, sy[W - 1].cell)) {
-            // The whole stencil lies in the guarded plane: one field at a time, its W x W
-            // loads issued together. Every accumulator still sums its cells in (iy, ix)
-            // order, as the reference's cell loop does.
-            const long k0 = g.idx(sx[0].cell, sy[0].cell);
-            auto tile = [&](const double* F, R (&v)[W][W]) {
-#pragma unroll
-                for (int iy = 0; iy < W; ++iy)
-#pragma unroll
-                    for (int ix = 0; ix < W; ++ix) v[iy][ix] = R(F[k0 + long(iy) * g.ldx + ix]);
-            };
-            R v[W][W];
-            tile(Psi, v);
-#pragma unroll
-            for (int iy = 0; iy < W; ++iy)
-#pragma unroll
-                for (int ix = 0; ix < W; ++ix) {
-                    ExmByp += (sx[ix].ds * sy[iy].s) * v[iy][ix] * dxi;
-                    EypBxp += (sx[ix].s * sy[iy].ds) * v[iy][ix] * dyi;
-                }
-            auto plain = [&](const double* F, R& acc) {
-                tile(F, v);
-#pragma unroll
-                for (int iy = 0; iy < W; ++iy)
-#pragma unroll
-                    for (int ix = 0; ix < W; ++ix) acc += (sx[ix].s * sy[iy].s) * v[iy][ix];
-            };
-            plain(Ez, Ezp);
-            plain(Bx, Bxp);
-            plain(By, Byp);
-            plain(Bz, Bzp);
-        } else {
-#pragma unroll
-            for (int iy = 0; iy < W; ++iy) {
-#pragma unroll
-                for (int ix = 0; ix < W; ++ix) {
-                    const DsfR<R> X = sx[ix], Y = sy[iy];
-                    if (!in_store(g, X.cell, Y.cell)) continue;
-                    const long k = g.idx(X.cell, Y.cell);
-                    accumulate(X, Y, R(Psi[k]), R(Ez[k]), R(Bx[k]), R(By[k]), R(Bz[k]));
-                }
-            }
-        }
-    }
+    double ux = p.ux_half_step[ip], uy = p.uy_half_step[ip], psi = p.psi_half_step[ip];
+    if (!valid) return;
+    const Gathered<R> G = gather_fields<O, R>(g, store, cPsi, cEz, cBx, cBy, cBz, xp, yp);
+    const R ExmByp = G.ExmBy, EypBxp = G.EypBx, Ezp = G.Ez, Bzp = G.Bz;
+    R Bxp = G.Bx, Byp = G.By;
     Bxp *= R(clight);
     Byp *= R(clight);
     constexpr int nsub = 4;
     const double sdz = dz / nsub;
-    // the (FP64) state; the increments are computed in R
-    double ux = p.ux_half_step[ip], uy = p.uy_half_step[ip], psi = p.psi_half_step[ip];
+    // the state (ux, uy, psi) is FP64; the increments are computed in R
     const R sdr = R(sdz), cir = R(clight_inv), qmr = R(qmc);
     auto substep = [&]() {
         const R psi_inv = R(1.0) / R(psi);
         R dux, duy, dpsi;
-        momentum_rhs<R, R>(R(ux), R(uy), psi_inv, ExmByp, EypBxp, Ezp, Bxp, Byp, Bzp, cir, qmr, dux, duy, dpsi);
+        momentum_rhs(R(ux), R(uy), psi_inv, ExmByp, EypBxp, Ezp, Bxp, Byp, Bzp, cir, qmr, dux, duy, dpsi);
         const Dual<R> uxd{R(ux), dux}, uyd{R(uy), duy}, pid{psi_inv, -psi_inv * psi_inv * dpsi};
         Dual<R> ddux(R(0.0)), dduy(R(0.0)), ddpsi(R(0.0));
-        momentum_rhs<Dual<R>, R>(uxd, uyd, pid, ExmByp, EypBxp, Ezp, Bxp, Byp, Bzp, cir, qmr, ddux, dduy, ddpsi);
+        momentum_rhs(uxd, uyd, pid, ExmByp, EypBxp, Ezp, Bxp, Byp, Bzp, cir, qmr, ddux, dduy, ddpsi);
         ux += double(sdr * dux + R(0.5) * sdr * sdr * ddux.e);
         uy += double(sdr * duy + R(0.5) * sdr * sdr * dduy.e);
         psi += double(sdr * dpsi + R(0.5) * sdr * sdr * ddpsi.e);
@@ -168,7 +198,10 @@ __global__ __launch_bounds__(256) void k_push_plasma(Geom g, hpq_plasma p, const
 
 // AdvanceBeamParticlesSlice (BeamParticleAdvance.cpp:128-336; no radiation reaction, spin
 // or external fields) for particle ip; a particle that ends below the slice with sub-cycles
-// left is appended to slip_out (shiftSlippedParticles, SliceSort.cpp:13-70).
+// left is appended to slip_out (shiftSlippedParticles, SliceSort.cpp:13-70). Bound by latency: a
+// slice's few thousand particles take their sub-cycles one after the other. With a field's loads
+// issued together instead of under a test per cell, ten sub-cycles of a slice of a million-particle
+// beam take 25 us (44).
 template <int O>
 __device__ void push_beam_particle(const Geom& g, const hpq_beam_state& b, long ip, const double* __restrict__ store,
                                    int cPsi, int cEz, int cBx, int cBy, int cBz, double dt, int n_subcycles,
@@ -179,12 +212,6 @@ __device__ void push_beam_particle(const Geom& g, const hpq_beam_state& b, long 
     double xp = b.x[ip], yp = b.y[ip], zp = b.z[ip];
     double ux = b.ux[ip], uy = b.uy[ip], uz = b.uz[ip];
     int i = b.nsubcycles[ip];
-    const double* Psi = store + long(cPsi) * g.plane;
-    const double* Ez = store + long(cEz) * g.plane;
-    const double* Bx = store + long(cBx) * g.plane;
-    const double* By = store + long(cBy) * g.plane;
-    const double* Bz = store + long(cBz) * g.plane;
-    constexpr int W = O + 2;
     for (; i < n_subcycles; i++) {
         if (zp < min_z) break;
         const double gammap_inv = 1.0 / sqrt(1.0 + (ux * ux + uy * uy + uz * uz) * inv_c2);
@@ -195,28 +222,8 @@ __device__ void push_beam_particle(const Geom& g, const hpq_beam_state& b, long 
             b.valid[ip] = 0;
             return;
         }
-        double ExmByp = 0, EypBxp = 0, Ezp = 0, Bxp = 0, Byp = 0, Bzp = 0;
-        const double xm = (xp - g.xoff) * g.dxi, ym = (yp - g.yoff) * g.dyi;
-        Dsf sx[W], sy[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-            sx[k] = dshape<1, O>(xm, k);
-            sy[k] = dshape<1, O>(ym, k);
-        }
-#pragma unroll
-        for (int iy = 0; iy < W; ++iy)
-#pragma unroll
-            for (int ix = 0; ix < W; ++ix) {
-                const Dsf X = sx[ix], Y = sy[iy];
-                if (!in_store(g, X.cell, Y.cell)) continue;
-                const long k = g.idx(X.cell, Y.cell);
-                ExmByp += (X.ds * Y.s) * Psi[k] * g.dxi;
-                EypBxp += (X.s * Y.ds) * Psi[k] * g.dyi;
-                Ezp += (X.s * Y.s) * Ez[k];
-                Bxp += (X.s * Y.s) * Bx[k];
-                Byp += (X.s * Y.s) * By[k];
-                Bzp += (X.s * Y.s) * Bz[k];
-            }
+        const Gathered<double> G = gather_fields<O, double>(g, store, cPsi, cEz, cBx, cBy, cBz, xp, yp);
+        double ExmByp = G.ExmBy, EypBxp = G.EypBx, Ezp = G.Ez, Bxp = G.Bx, Byp = G.By, Bzp = G.Bz;
         if (b.use_external_fields) {
             // ApplyExternalField, src/particles/pusher/ExternalFields.H:43-55
             const double* e = b.external_fields;

@@ -7,7 +7,10 @@
 
 namespace hpq {
 
-// Forward-mode dual number for the second-order Taylor step (src/utils/DualNumbers.H:13-43)
+// Forward-mode dual number for the second-order Taylor step (src/utils/DualNumbers.H:13-43).
+// A factor or term that does not depend on the parameter stays a plain number instead of a dual
+// number with derivative zero: the products with that zero, which no compiler may drop, only
+// ever added a zero.
 template <class R>
 struct Dual {
     R v, e;
@@ -22,17 +25,24 @@ template <class R>
 __host__ __device__ __forceinline__ Dual<R> operator*(const Dual<R>& a, const Dual<R>& b) {
     return {a.v * b.v, a.e * b.v + a.v * b.e};
 }
+template <class R, class S>
+__host__ __device__ __forceinline__ Dual<R> operator+(const Dual<R>& a, const S& b) { return {a.v + b, a.e}; }
+template <class R, class S>
+__host__ __device__ __forceinline__ Dual<R> operator-(const Dual<R>& a, const S& b) { return {a.v - b, a.e}; }
+template <class R, class S>
+__host__ __device__ __forceinline__ Dual<R> operator*(const Dual<R>& a, const S& b) { return {a.v * b, a.e * b}; }
 
-// PlasmaMomentumPush, src/particles/pusher/PushPlasmaParticles.H:37-75 (no laser terms)
-template <class T, class R>
-__host__ __device__ __forceinline__ void momentum_rhs(const T& ux, const T& uy, const T& psi_inv, R ExmBy, R EypBx, R Ez,
-                                             R Bx_c, R By_c, R Bz, R ci, R qmc, T& dux, T& duy, T& dpsi) {
-    const R A = 0.0, ADx = 0.0, ADy = 0.0;
-    const T gamma_psi =
-        T(0.5) * psi_inv * psi_inv * (T(1.0) + T(A) + ux * ux * T(ci * ci) + uy * uy * T(ci * ci)) + T(0.5);
-    dux = (T(qmc) * (gamma_psi * T(ExmBy) + T(By_c) + (uy * T(Bz)) * psi_inv) - T(ADx) * psi_inv);
-    duy = (T(qmc) * (gamma_psi * T(EypBx) - T(Bx_c) - (ux * T(Bz)) * psi_inv) - T(ADy) * psi_inv);
-    dpsi = (T(qmc) * T(ci) * ((ux * T(ExmBy) + uy * T(EypBx)) * T(ci) * psi_inv - T(Ez)));
+// PlasmaMomentumPush, src/particles/pusher/PushPlasmaParticles.H:37-75 (no laser terms). T: the
+// number type of the particle, F of the fields at it, S of the constants.
+template <class T, class F, class S>
+__host__ __device__ __forceinline__ void momentum_rhs(const T& ux, const T& uy, const T& psi_inv, const F& ExmBy,
+                                                      const F& EypBx, const F& Ez, const F& Bx_c, const F& By_c,
+                                                      const F& Bz, S ci, S qmc, T& dux, T& duy, T& dpsi) {
+    const S half = S(0.5), cc = ci * ci, qc = qmc * ci;
+    const T gamma_psi = (psi_inv * half) * psi_inv * (ux * ux * cc + S(1.0) + uy * uy * cc) + half;
+    dux = (gamma_psi * ExmBy + By_c + (uy * Bz) * psi_inv) * qmc;
+    duy = (gamma_psi * EypBx - Bx_c - (ux * Bz) * psi_inv) * qmc;
+    dpsi = ((ux * ExmBy + uy * EypBx) * ci * psi_inv - Ez) * qc;
 }
 
 struct BC {
