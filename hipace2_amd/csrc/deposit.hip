@@ -585,13 +585,12 @@ void deposit_beam(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const
     deposit_beam_select(c, b, slice, store, comps, nullptr, 0);
 }
 
-// Builds a slice's ordered contributions once for repeated beam_sequences_add; false where there
+// Builds a slice's ordered contributions ahead of their use or for repeated use; null where there
 // is nothing to build (no particles, atomic deposition), and deposit_beam does it all.
-bool prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice) {
-    if (!b || slice < 0 || slice >= c->g.nz || !b->off || b->off[slice + 1] <= b->off[slice]) return false;
-    if (c->p.deposition != HPQ_DEPOSIT_ORDERED) return false;
-    beam_sequences(c, b, slice, nullptr, 0);
-    return true;
+const CellLists* prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice) {
+    if (!b || slice < 0 || slice >= c->g.nz || !b->off || b->off[slice + 1] <= b->off[slice]) return nullptr;
+    if (c->p.deposition != HPQ_DEPOSIT_ORDERED) return nullptr;
+    return &beam_sequences(c, b, slice, nullptr, 0);
 }
 
 // only the particles whose select entry equals select_value deposit (select NULL: all)
@@ -604,8 +603,7 @@ void deposit_beam_select(hpq_ctx* c, const hpq_beam* b, int slice, double* store
     if ((comps[0] >= 0) != (comps[1] >= 0))
         throw HpqError(HPQ_E_INVALID, "deposit_current_slice: jx and jy go together");
     if (c->p.deposition == HPQ_DEPOSIT_ORDERED) {
-        beam_sequences(c, b, slice, select, select_value);
-        beam_sequences_add(c, store, comps);
+        beam_sequences_add(c, beam_sequences(c, b, slice, select, select_value), store, comps);
         return;
     }
     TraceScope ts(c, HPQ_TRACE_BEAM_DEPOSIT);

@@ -23,7 +23,8 @@
 //           cell's sequence;
 //   sum     each cell adds its sequence in order to the plane's value. The sequences hold jx, jy
 //           and jz and depend on the beam alone: the predictor-corrector loop, which deposits
-//           the same slice's beam in every iteration, builds them once.
+//           the same slice's beam in every iteration, builds them once, and the slice after it
+//           uses them again.
 #include <climits>
 #include <cmath>
 
@@ -432,11 +433,19 @@ void cell_lists_free(CellLists& L) {
 }
 
 // The contribution sequences of ::DepositCurrentSlice in the CPU build's order (particles of
-// `slice` whose select entry equals select_value; select NULL: all), for beam_sequences_add
-// until the next call. The slice has particles.
-void beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value) {
+// `slice` whose select entry equals select_value; select NULL: all), for beam_sequences_add.
+// The slice has particles. Two slices' sequences are held: a slice deposits its own jz and the
+// next one's jx and jy, so each slice's beam is deposited in two slices in a row, and the
+// sequences that the first built serve the second. They are forgotten when the particles may have
+// changed: at every call from outside, and where the slice is pushed or its weights change.
+const CellLists& beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value) {
     const Geom& g = c->g;
-    CellLists& L = c->cl_beam;
+    for (const CellLists& L : c->cl_beam)
+        if (!select && L.slice == slice) return L;
+    // in the place of none or of the slice that is done with: slices go downwards
+    auto age = [](const CellLists& L) { return L.slice < 0 ? INT_MAX : L.slice; };
+    CellLists& L = c->cl_beam[age(c->cl_beam[1]) > age(c->cl_beam[0]) ? 1 : 0];
+    L.slice = -1;
     const long first = b->off[slice];
     const long count = b->off[slice + 1] - first;
     const int S = c->p.depos_order + 1;
@@ -466,12 +475,18 @@ void beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* sel
                            L.seg, L.contrib, m);
     });
     HPQ_HIP(hipGetLastError());
+    if (!select) L.slice = slice;
+    return L;
+}
+
+void beam_sequences_forget(hpq_ctx* c, int slice) {
+    for (CellLists& L : c->cl_beam)
+        if (slice < 0 || L.slice == slice) L.slice = -1;
 }
 
 // the sequences added to the planes comps (jx, jy, jz; -1: none)
-void beam_sequences_add(hpq_ctx* c, double* store, const int32_t* comps) {
+void beam_sequences_add(hpq_ctx* c, const CellLists& L, double* store, const int32_t* comps) {
     const Geom& g = c->g;
-    const CellLists& L = c->cl_beam;
     TraceScope ts(c, HPQ_TRACE_BEAM_DEPOSIT);
     const int nshort = int((g.plane + 255) / 256);
     hipLaunchKernelGGL(k_beam_sum, dim3(nshort + 512), dim3(256), 0, c->stream, g, L.seg, L.contrib, L.m, store,

@@ -71,7 +71,7 @@ void layout_init(hpq_ctx* c) {
 void side_init(hpq_ctx* c) {
     if (c->side) return;
     HPQ_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
-    for (hipEvent_t* e : {&c->ev_start, &c->ev_beam, &c->ev_fields, &c->ev_end})
+    for (hipEvent_t* e : {&c->ev_start, &c->ev_beam, &c->ev_fields, &c->ev_end, &c->ev_push})
         HPQ_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
 }
 
@@ -213,12 +213,17 @@ public:
     // end-of-slice pass run on the context's second stream (explicit solver, chained slices):
     //   side: [jz_beam of this slice, jx/jy_beam of the next]          after the planes are zeroed
     //   main: [plasma deposit, Poisson solves] wait(beam) [Sx/Sy, explicit deposit, MG, SALAME]
-    //   side: wait(fields) [diagnostics, ShiftSlices, next InitializeSlices]
-    //   main: [plasma push] wait(end)
-    // The push reads Psi, Ez, Bx, By, Bz, which the end-of-slice pass neither writes nor
-    // zeroes, so the two overlap; the next slice's deposits wait for the zeroing.
+    //   side: [the beam's contribution sequences that the next slice deposits]
+    //   side: wait(fields) [diagnostics, ShiftSlices, next InitializeSlices] [beam push]
+    //   main: [plasma push] wait(end)     next slice: [plasma deposit] wait(push) [Poisson solves]
+    // The pushes read Psi, Ez, Bx, By, Bz, which the end-of-slice pass neither writes nor
+    // zeroes, so they overlap with it; the next slice's deposits wait for the zeroing and its
+    // Poisson solves for the beam push. The beam push changes this slice's particles and those
+    // that slipped out of earlier ones, the next slice deposits the two below. The host
+    // launches the plasma deposit first: the beam's launches are hidden behind it.
     void SolveOneSlice(int islice, bool initialized = false, bool chain = false,
-                       const std::function<void()>& before_push = {}, bool two = false) {
+                       const std::function<void()>& before_push = {}, bool two = false,
+                       const std::function<void()>& beam_push = {}) {
         const hpq_params& P = c_->p;
         two = two && P.explicit_solver;
         insitu_plasma(c_, p_, islice);
@@ -244,23 +249,25 @@ public:
                 deposit_beam_select(c_, b_, islice - 1, s_, comps, c_->salame.mask, 0);
             }
         };
-        if (two) {
-            HPQ_HIP(hipEventRecord(c_->ev_start, c_->stream));
-            on_side([&] {
-                HPQ_HIP(hipStreamWaitEvent(c_->stream, c_->ev_start, 0));
-                beam_deposits();
-                HPQ_HIP(hipEventRecord(c_->ev_beam, c_->stream));
-            });
-        }
         if (P.explicit_solver) {
+            if (two) HPQ_HIP(hipEventRecord(c_->ev_start, c_->stream));
             DepositCurrent(c_, p_, s_, L_.jx, L_.jy, -1, L_.rho, L_.chi, L_.rhomjz);
-            if (!two) DepositCurrentSlice(c_, b_, islice, s_, -1, -1, L_.jz_beam);
+            if (two) {
+                on_side([&] {
+                    HPQ_HIP(hipStreamWaitEvent(c_->stream, c_->ev_start, 0));
+                    beam_deposits();
+                    HPQ_HIP(hipEventRecord(c_->ev_beam, c_->stream));
+                });
+            } else {
+                DepositCurrentSlice(c_, b_, islice, s_, -1, -1, L_.jz_beam);
+            }
         } else {
             DepositCurrent(c_, p_, s_, L_.jx, L_.jy, L_.jz, L_.rho, -1, L_.rhomjz);
             DepositCurrentSlice(c_, b_, islice, s_, P.do_beam_jx_jy ? L_.jx : -1, P.do_beam_jx_jy ? L_.jy : -1,
                                 L_.jz);
         }
         fields_.AddRhoIons();
+        JoinBeamPush();
         fields_.SolvePoissonPsiExmByEypBxEzBz();
         if (P.explicit_solver) {
             if (two) {
@@ -271,6 +278,9 @@ public:
             }
             InitializeSxSyWithBeam();
             explicit_deposition(c_, p_, s_);
+            // SALAME deposits the beam on the main stream, with the same scratch
+            if (two && chain && !c_->salame.mask)
+                on_side([&] { prepare_beam(c_, b_, islice - (P.do_beam_jx_jy ? 2 : 1)); });
             if (P.mg_guess == HPQ_MG_GUESS_LINEAR) mg_guess_linear(c_, s_ + long(L_.Bx) * c_->g.plane, islice);
             if (P.mg_guess == HPQ_MG_GUESS_DST) bxby_guess_dst(c_, s_, P.mg_guess_iters);
             ExplicitMGSolveBxBy();
@@ -285,6 +295,11 @@ public:
                 HPQ_HIP(hipStreamWaitEvent(c_->stream, c_->ev_fields, 0));
                 fields_.EndSlice(islice, chain);
                 HPQ_HIP(hipEventRecord(c_->ev_end, c_->stream));
+                if (beam_push) {
+                    beam_push();
+                    HPQ_HIP(hipEventRecord(c_->ev_push, c_->stream));
+                    pushing_ = true;
+                }
             });
         } else {
             fields_.EndSlice(islice, chain);
@@ -294,6 +309,13 @@ public:
         c_->stats[3] += double(p_->n);
         if (two) HPQ_HIP(hipStreamWaitEvent(c_->stream, c_->ev_end, 0));
         if (!chain) fields_.ShiftSlices();
+        if (beam_push && !two) beam_push();
+    }
+
+    // the main stream waits for a beam push on the second one
+    void JoinBeamPush() {
+        if (pushing_) HPQ_HIP(hipStreamWaitEvent(c_->stream, c_->ev_push, 0));
+        pushing_ = false;
     }
 
     // Hipace::InitializeSxSyWithBeam, :745-790
@@ -407,14 +429,14 @@ public:
         fields_.InitialBfieldGuess(err, P.pc_tol);
         // the next slice's beam deposits the same in every iteration
         const int32_t beam[3] = {L_.next_jx, L_.next_jy, -1};
-        const bool sequences = P.do_beam_jx_jy && prepare_beam(c_, b_, islice - 1);
+        const CellLists* sequences = P.do_beam_jx_jy ? prepare_beam(c_, b_, islice - 1) : nullptr;
         int it = 0;
         err = 1.0;
         while (err > P.pc_tol && it < P.pc_maxiter) {
             ++it;
             advance_plasma(c_, p_, s_, true);
             DepositCurrent(c_, p_, s_, L_.next_jx, L_.next_jy, -1, -1, -1, -1);
-            if (sequences) beam_sequences_add(c_, s_, beam);
+            if (sequences) beam_sequences_add(c_, *sequences, s_, beam);
             else if (P.do_beam_jx_jy) deposit_beam(c_, b_, islice - 1, s_, beam);
             fields_.SolvePoissonBxBy();
             err = fields_.MixAndShiftBfields(it, P.pc_mix);
@@ -429,6 +451,7 @@ private:
     double* s_;
     Fields fields_;
     const Layout& L_;
+    bool pushing_ = false;   // a beam push on the second stream has not been waited for
 };
 
 }  // namespace hpq
@@ -443,20 +466,31 @@ namespace {
 template <class F>
 int guarded(hpq_ctx* c, F&& f) {
     // the caller may have changed the particle arrays since the last call
-    if (c) c->ord_plasma.valid = false;
+    if (c) {
+        c->ord_plasma.valid = false;
+        beam_sequences_forget(c);
+    }
+    // what an abandoned pass has left on the second stream ends before the caller goes on
+    auto drain = [&] {
+        if (c && c->side) (void)hipStreamSynchronize(c->side);
+    };
     try {
         f();
         return HPQ_OK;
     } catch (const HpqError& e) {
+        drain();
         if (c) c->err = e.msg;
         return e.code;
     } catch (const HipError& e) {
+        drain();
         if (c) c->err = e.msg;
         return HPQ_E_HIP;
     } catch (const std::bad_alloc&) {
+        drain();
         if (c) c->err = "out of host memory";
         return HPQ_E_NOMEM;
     } catch (const std::exception& e) {
+        drain();
         if (c) c->err = e.what();
         return HPQ_E_INVALID;
     }
@@ -793,7 +827,7 @@ void hpq_destroy(hpq_ctx* c) {
     mg_free(c);
     bins_free(c);
     plasma_order_free(c->ord_plasma);
-    cell_lists_free(c->cl_beam);
+    for (CellLists& L : c->cl_beam) cell_lists_free(L);
     init_scratch_free(c);
     if (c->relb_rows) (void)hipFree(c->relb_rows);
     if (c->diag_partial) (void)hipFree(c->diag_partial);
@@ -806,7 +840,7 @@ void hpq_destroy(hpq_ctx* c) {
     beam_slip_free(c);
     insitu_free(c);
     salame_free(c);
-    for (hipEvent_t e : {c->ev_start, c->ev_beam, c->ev_fields, c->ev_end})
+    for (hipEvent_t e : {c->ev_start, c->ev_beam, c->ev_fields, c->ev_end, c->ev_push})
         if (e) (void)hipEventDestroy(e);
     if (c->side) (void)hipStreamDestroy(c->side);
     delete c;
@@ -979,11 +1013,14 @@ int hpq_run_step_with_beam(hpq_ctx* c, const hpq_plasma* p, hpq_beam_state* b, d
         const hpq_beam view{b->x, b->y, b->z, b->ux, b->uy, b->uz, b->w, b->valid, b->off, b->n, b->charge, b->mass};
         beam_begin_step(c, b);
         Hipace h(c, p, &view, store);
-        for (int isl = c->g.nz - 1; isl >= 0; --isl) {
-            h.SolveOneSlice(isl);
-            // AdvanceBeamParticlesSlice after the plasma push (src/Hipace.cpp:700-709)
-            advance_beam(c, b, isl, store, dt_step, n_subcycles, do_z_push != 0);
-        }
+        const int nz = c->g.nz;
+        const bool two = c->p.explicit_solver && nz > 1;
+        if (two) side_init(c);
+        // AdvanceBeamParticlesSlice with the plasma push (src/Hipace.cpp:700-709)
+        for (int isl = nz - 1; isl >= 0; --isl)
+            h.SolveOneSlice(isl, isl != nz - 1, isl != 0, {}, two,
+                            [&] { advance_beam(c, b, isl, store, dt_step, n_subcycles, do_z_push != 0); });
+        h.JoinBeamPush();
         diag_finalize(c);
     });
 }

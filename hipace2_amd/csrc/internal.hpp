@@ -212,6 +212,7 @@ struct CellLists {
     double* contrib = nullptr;
     long contrib_cap = 0;
     long m = 0;   // (particle, stencil offset) pairs: stride of the contribution arrays
+    int slice = -1;   // the slice all of whose particles' sequences are held; -1: none that may be reused
 };
 
 // Scratch of the plasma injection: per-cell particle counts and their exclusive scan.
@@ -273,7 +274,7 @@ struct hpq_ctx {
     hpq::MultiGrid mg;
     hpq::Bins bins;
     hpq::PlasmaOrder ord_plasma;     // ordered deposition of the plasma (main stream)
-    hpq::CellLists cl_beam;          // ordered deposition of the beam (either stream)
+    hpq::CellLists cl_beam[2];       // ordered deposition of the beam (either stream)
     hpq::InitScratch init;
     double* relb_rows = nullptr;     // row sums of ComputeRelBFieldError (2 * ny)
     long relb_cap = 0;
@@ -299,7 +300,7 @@ struct hpq_ctx {
     // second stream of the chained slice loop: beam deposition and the end-of-slice pass run
     // beside the plasma deposition / Poisson solves and the plasma push
     hipStream_t side = nullptr;
-    hipEvent_t ev_start = nullptr, ev_beam = nullptr, ev_fields = nullptr, ev_end = nullptr;
+    hipEvent_t ev_start = nullptr, ev_beam = nullptr, ev_fields = nullptr, ev_end = nullptr, ev_push = nullptr;
     double* insitu_partial = nullptr;  // per-workgroup in-situ sums of one slice
     long insitu_cap = 0;               // workgroups insitu_partial holds
     std::vector<hpq::Capture> captures;
@@ -336,7 +337,7 @@ int mg_solve1(hpq_ctx* c, double* sol, const double* rhs, const double* acf, lon
 void deposit_current(hpq_ctx* c, const hpq_plasma* p, double* store, const int32_t* comps, bool ions);
 void explicit_deposition(hpq_ctx* c, const hpq_plasma* p, double* store);
 void deposit_beam(hpq_ctx* c, const hpq_beam* b, int slice, double* store, const int32_t* comps);
-bool prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice);
+const CellLists* prepare_beam(hpq_ctx* c, const hpq_beam* b, int slice);
 void advance_plasma(hpq_ctx* c, const hpq_plasma* p, const double* store, bool temp_slice);
 void plane_fill(hpq_ctx* c, double* store, const int* comps, int ncomps, double v);
 void plane_copy(hpq_ctx* c, double* store, const int* dst, const int* src, int ncomps);
@@ -394,8 +395,9 @@ void scan_exclusive(hipStream_t s, int32_t* a, long n, int32_t* tmp);
 long scan_tmp_size(long n);
 void deposit_current_ordered(hpq_ctx* c, const hpq_plasma* p, double* store, const int32_t* comps, bool ions);
 void explicit_deposition_ordered(hpq_ctx* c, const hpq_plasma* p, double* store);
-void beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value);
-void beam_sequences_add(hpq_ctx* c, double* store, const int32_t* comps);
+const CellLists& beam_sequences(hpq_ctx* c, const hpq_beam* b, int slice, const int32_t* select, int select_value);
+void beam_sequences_add(hpq_ctx* c, const CellLists& L, double* store, const int32_t* comps);
+void beam_sequences_forget(hpq_ctx* c, int slice = -1);
 void plasma_order_free(PlasmaOrder& L);
 void cell_lists_free(CellLists& L);
 void sort_beam_slices(hpq_ctx* c, hpq_beam_state* b, int64_t* off_out);

@@ -369,6 +369,7 @@ void advance_beam(hpq_ctx* c, hpq_beam_state* b, int slice, const double* store,
     });
     HPQ_HIP(hipGetLastError());
     S.cur = out;
+    beam_sequences_forget(c, slice);
 }
 
 // ---------------------------------------------------------------------------------

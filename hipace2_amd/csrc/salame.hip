@@ -201,6 +201,7 @@ void salame_multiply(hpq_ctx* c, const hpq_beam* b, int slice, double W) {
     hipLaunchKernelGGL(k_sal_multiply, grid1d(n, 256), dim3(256), 0, c->stream, c->salame.mask, c->salame.w,
                        c->salame.valid, first, n, W);
     HPQ_HIP(hipGetLastError());
+    beam_sequences_forget(c);
 }
 
 }  // namespace hpq
