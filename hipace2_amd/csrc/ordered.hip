@@ -28,7 +28,7 @@
 // index elsewhere) and now:
 //                                 lists / records   current      explicit
 //   linear wake (near the lattice)   52 -> 37      115 -> 110   221 -> 183
-//   nonlinear wake (crossing)        55 -> 44      422 -> 185  1328 -> 282
+//   nonlinear wake (crossing)        55 -> 44      422 -> 138  1328 -> 275
 //
 // A particle's cell is the floor of the cell-scaled position the shape functions take theirs
 // from (floor(xmid) or floor(xmid + 1/2)); a stencil's start cell is that floor plus a
@@ -51,7 +51,6 @@ constexpr int SUPER = 256;       // particles per box of the second level
 constexpr int RUNS_PER_SUPER = SUPER / RUN;
 constexpr uint32_t NO_CELL = 0xffffffffu;
 constexpr int REC = 8;           // doubles per record
-constexpr int BW = 16, BH = 8;   // cells of a deposition wavefront's block
 constexpr int LIST = 128;        // runs listed per block
 constexpr int WIDE = 512;        // a run that meets more blocks than this goes to one list for all
 
@@ -62,7 +61,8 @@ struct OrdView {
     int bxlo, bylo, shift;
     int T, ntx, nty;   // deposition tiles: T cells (hipace.tile_size), ntx x nty over the guarded box
     int nrun, nsuper;
-    int nbx, nby;      // blocks of the gather
+    int lw, lh;        // log2 of a block's width and height
+    int nbx, nby;      // blocks
     int mlo, mhi;      // cells a block's window reaches below and above it
     long n;
     const double* __restrict__ rec;
@@ -157,8 +157,8 @@ __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView
     // the run into the list of every block whose window its box meets
     if (x0 <= x1) {
         const int c0 = v.bxlo + g.ng, r0 = v.bylo + g.ng;   // cell 0 counted from block 0's first
-        const int bx0 = max(x0 + c0 - v.mhi, 0) / BW, bx1 = min((x1 + c0 + v.mlo) / BW, v.nbx - 1);
-        const int by0 = max(y0 + r0 - v.mhi, 0) / BH, by1 = min((y1 + r0 + v.mlo) / BH, v.nby - 1);
+        const int bx0 = max(x0 + c0 - v.mhi, 0) >> v.lw, bx1 = min((x1 + c0 + v.mlo) >> v.lw, v.nbx - 1);
+        const int by0 = max(y0 + r0 - v.mhi, 0) >> v.lh, by1 = min((y1 + r0 + v.mlo) >> v.lh, v.nby - 1);
         const int nx = bx1 - bx0 + 1, nb = nx > 0 && by1 >= by0 ? nx * (by1 - by0 + 1) : 0;
         const int run = int(ip / RUN);
         if (nb > WIDE) {
@@ -181,8 +181,6 @@ __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView
 // ---- deposition -----------------------------------------------------------------------------
 constexpr int SUPER_BATCH = 64;     // second-level boxes tested at a time
 constexpr int BATCH = 16;           // runs tested at a time
-constexpr int SEQ = 1024;           // entries sequenced at a time
-constexpr int BS = BW + 4;          // LDS pitch of a block row: a stencil's rows on different banks
 
 __device__ __forceinline__ int lanes_before(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0));
@@ -223,6 +221,16 @@ struct Stencil {
     // S columns and of the S rows, (q w invvol, 1/psi), (vx/c, vy/c), (gamma/psi, target).
     // CURRENT: (charge density, target) of the N offsets, the two factors of every quantity.
     static constexpr int ENT = KIND == EXPLICIT ? 2 * S + 3 : N + 6;
+    // Entries sequenced at a time with blocks of `cells` cells, found in the place of the staged
+    // ones; where a window holds more, its colours are taken one after the other, each from all
+    // runs. The largest block's current deposition has room for 2048 without losing a wavefront
+    // per CU: 138 instead of 182 us for crossing orbits at 511 x 511, 2 x 2 particles per cell. The
+    // explicit one has not: with 1920 entries and 27 particles staged at a time it takes 243 instead
+    // of 275 us there, but 205 instead of 194 near the lattice.
+    static constexpr int seq(int cells) {
+        const int room = CHUNK * ENT * 8, want = KIND == CURRENT && cells == 128 ? 2048 : 1024;
+        return room < want ? room : want;
+    }
 };
 
 // One wavefront per block of BW x BH cells of the guarded plane. ::DepositCurrent's per-cell
@@ -241,14 +249,15 @@ struct Stencil {
 // 60 vector instructions (42 of them FP64) on each of four SIMDs. A 16 x 8 block keeps the
 // window of an order-2 derivative stencil at 1.9 times its cells and gives 511 x 511 cells
 // 2145 wavefronts; CHUNK, SEQ and BS are chosen so that nine of them fit a CU's LDS, one round
-// for that grid (eight in two rounds: 212 instead of 183 us).
+// for that grid (eight in two rounds: 212 instead of 183 us). Smaller grids have smaller blocks.
 // NSUM: the sums of a cell (CURRENT: components asked for, at most NSUM).
-template <int KIND, int T, int O, int NSUM>
+template <int KIND, int T, int O, int NSUM, int BW, int BH>
 __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, double* __restrict__ store, Comps cm,
                                                         double charge_mass_ratio) {
     using St = Stencil<KIND, T, O>;
-    constexpr int S = St::S, N = St::N, PP = St::PP, U = St::U, CHUNK = St::CHUNK, ENT = St::ENT;
+    constexpr int S = St::S, N = St::N, PP = St::PP, U = St::U, CHUNK = St::CHUNK, ENT = St::ENT, SEQ = St::seq(BW * BH);
     constexpr int NW = BW + S - 1, NH = BH + S - 1;   // window, in cells
+    constexpr int BS = BW + 4;   // LDS pitch of a block row: a stencil's rows on different banks
     constexpr int CELLS = BS * BH;
     static_assert(NW <= 64 && N <= 32, "window and offset masks");
     __shared__ double2 ent[CHUNK][ENT];
@@ -701,6 +710,25 @@ int bits(long v) {
     return b;
 }
 
+// The blocks of a grid: 16 x 8 cells, 8 x 8 or 8 x 4, the largest of which there are as many as
+// the CUs hold wavefronts at once, or the smallest. A larger block's window holds fewer
+// particles that other blocks take as well; too few blocks leave the chip idle, and a wavefront
+// takes its particles one after the other. Measured for a near-lattice plasma of one particle per
+// cell, order 2, current + explicit in us, with 16 x 8, 8 x 8 and 8 x 4 cells:
+//    63 x 63 52, 37, 31; 127 x 127 60, 47, 39; 255 x 255 71, 62, 54; 383 x 383 84, 74, 95;
+//   511 x 511 106, 126, 145 (2 x 2 particles per cell 310, 337, 370).
+constexpr long FILL = 8 * 256;
+void blocks(const Geom& g, OrdView& v) {
+    const int sizes[3][2] = {{4, 3}, {3, 3}, {3, 2}};
+    for (const auto& s : sizes) {
+        v.lw = s[0];
+        v.lh = s[1];
+        v.nbx = (g.ldx + (1 << v.lw) - 1) >> v.lw;
+        v.nby = (g.ldy + (1 << v.lh) - 1) >> v.lh;
+        if (long(v.nbx) * v.nby >= FILL) break;
+    }
+}
+
 // every start cell whose stencil (at most 6 wide, start at most 2 below the cell) reaches the
 // guarded plane has a cell in [bxlo, bxlo + wx) x [bylo, bylo + wy)
 OrdView view(const hpq_ctx* c, const PlasmaOrder& L, long n, int& wx, int& wy) {
@@ -718,8 +746,7 @@ OrdView view(const hpq_ctx* c, const PlasmaOrder& L, long n, int& wx, int& wy) {
     v.n = n;
     v.nrun = int((n + RUN - 1) / RUN);
     v.nsuper = int((n + SUPER - 1) / SUPER);
-    v.nbx = (g.ldx + BW - 1) / BW;
-    v.nby = (g.ldy + BH - 1) / BH;
+    blocks(g, v);
     // the current deposition's stencil starts at most 1 below the cell and ends at most 2 above,
     // the derivative ones' at most 2 below and 3 above
     v.mlo = 3;
@@ -744,7 +771,9 @@ OrdView make_records(hpq_ctx* c, const hpq_plasma* p, double charge_invvol) {
     grow(L.cell, L.cell_cap, n);
     grow(L.boxes, L.boxes_cap, 4 * ((n + RUN - 1) / RUN + (n + SUPER - 1) / SUPER));
     // two sets of run counts: every pass clears the next one's
-    const long nblk = long((g.ldx + BW - 1) / BW) * ((g.ldy + BH - 1) / BH);
+    OrdView size{};
+    blocks(g, size);
+    const long nblk = long(size.nbx) * size.nby;
     if (!L.count) {
         grow(L.list, L.list_cap, (nblk + 1) * LIST);
         grow(L.count, L.count_cap, 2 * (nblk + 1));
@@ -764,8 +793,12 @@ OrdView make_records(hpq_ctx* c, const hpq_plasma* p, double charge_invvol) {
 
 template <int KIND, int T, int O, int NSUM>
 void launch_deposit(hpq_ctx* c, const OrdView& v, double* store, const Comps& cm, double ratio) {
-    hipLaunchKernelGGL((k_deposit_ordered<KIND, T, O, NSUM>), dim3(unsigned(v.nbx * v.nby)), dim3(64), 0, c->stream,
-                       c->g, v, store, cm, ratio);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(v.nbx * v.nby)), dim3(64), 0, c->stream, c->g, v, store, cm, ratio);
+    };
+    if (v.lw == 4) launch(k_deposit_ordered<KIND, T, O, NSUM, 16, 8>);
+    else if (v.lh == 3) launch(k_deposit_ordered<KIND, T, O, NSUM, 8, 8>);
+    else launch(k_deposit_ordered<KIND, T, O, NSUM, 8, 4>);
     HPQ_HIP(hipGetLastError());
 }
 
