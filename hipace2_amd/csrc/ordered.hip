@@ -422,10 +422,7 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
             const uint32_t word = uint32_t(__double2loint(r3.y));
             // column and row of the stencil's first cell in the block, and its cells inside
             const int x = int(word & xmask) - X0 - (S - 1), y = int(word >> v.shift) - Y0 - (S - 1);
-            auto bits = [](int first, int last) {   // bits [first, last) of the stencil's S
-                return first < last ? ((1u << min(last, S)) - 1u) & ~((1u << max(first, 0)) - 1u) : 0u;
-            };
-            const uint32_t cols = bits(-x, ncol_in - x), rows = bits(-y, nrow_in - y);
+            const uint32_t cols = stencil_bits(-x, ncol_in - x, S), rows = stencil_bits(-y, nrow_in - y, S);
             uint32_t inside = 0u;
 #pragma unroll
             for (int r = 0; r < S; ++r) {
