@@ -186,9 +186,9 @@ struct PlasmaOrder {
     double* rec = nullptr;
     uint32_t* cell = nullptr;
     int32_t* boxes = nullptr;
-    int32_t *count = nullptr, *list = nullptr;   // runs of particles listed per gather block
+    int32_t *count = nullptr, *list = nullptr;   // runs of particles listed per deposition block
     long rec_cap = 0, cell_cap = 0, boxes_cap = 0, count_cap = 0, list_cap = 0;
-    int pick = 0;                                // the set of counts in use
+    bool unclear = true;                         // the counts have to be cleared before the next pass
     bool valid = false;
     int base = -1;
     const double* x = nullptr;

@@ -53,6 +53,7 @@ constexpr uint32_t NO_CELL = 0xffffffffu;
 constexpr int REC = 8;           // doubles per record
 constexpr int LIST = 128;        // runs listed per block
 constexpr int WIDE = 512;        // a run that meets more blocks than this goes to one list for all
+constexpr int NEXT = 0, MADE = 16, SET_WORDS = 32;   // words of OrdView::set, on lines of their own
 
 // Records, cells and boxes of one plasma state. Cells count from (bxlo, bylo): x in the low
 // `shift` bits of the word, y above them. A box is (xmin, xmax, ymin, ymax), empty when
@@ -69,7 +70,12 @@ struct OrdView {
     const uint32_t* __restrict__ cell;
     const int4* __restrict__ rbox;
     const int4* __restrict__ sbox;
-    const int32_t* __restrict__ count;   // runs listed per block, then the wide ones (may exceed LIST)
+    // Runs listed per block, then the wide ones (may exceed LIST): two sets. A records pass uses the
+    // set that set[NEXT] names, clears the other and notes its own in set[MADE]; the deposition that
+    // reads the set then names the other one. What is to be clear and what is not lives on the
+    // device alone, so that a captured pass may be replayed any number of times.
+    const int32_t* __restrict__ count;
+    const int32_t* __restrict__ set;
     const int32_t* __restrict__ list;    // LIST runs per block and of the wide ones, in any order
 };
 
@@ -104,12 +110,13 @@ template <int BASE, bool QSA>
 __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView v, int wx, int wy,
                                                    double charge_invvol, double max_qsa, double* __restrict__ rec,
                                                    uint32_t* __restrict__ cell, int4* __restrict__ rbox,
-                                                   int4* __restrict__ sbox, int32_t* __restrict__ count,
-                                                   int32_t* __restrict__ list, int32_t* __restrict__ next_count,
+                                                   int4* __restrict__ sbox, int32_t* __restrict__ counts,
+                                                   int32_t* __restrict__ list, int32_t* __restrict__ made,
                                                    int* __restrict__ qsa_count) {
     __shared__ int box[4];
     const int nblk = v.nbx * v.nby;
-    for (int t = int(blockIdx.x) * REC_T + int(threadIdx.x); t <= nblk; t += int(gridDim.x) * REC_T) next_count[t] = 0;
+    const int set = v.set[NEXT];
+    int32_t* const count = counts + long(set) * (nblk + 1);
     if (threadIdx.x < 4) box[threadIdx.x] = (threadIdx.x & 1) ? -1 : INT_MAX;
     __syncthreads();
     const long ip = long(blockIdx.x) * SUPER + threadIdx.x;
@@ -174,6 +181,9 @@ __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView
             }
         }
     }
+    int32_t* const next_count = counts + long(set ^ 1) * (nblk + 1);
+    for (int t = int(blockIdx.x) * REC_T + int(threadIdx.x); t <= nblk; t += int(gridDim.x) * REC_T) next_count[t] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *made = set;
     __syncthreads();
     if (threadIdx.x == 0) sbox[blockIdx.x] = make_int4(box[0], box[1], box[2], box[3]);
 }
@@ -253,7 +263,7 @@ struct Stencil {
 // NSUM: the sums of a cell (CURRENT: components asked for, at most NSUM).
 template <int KIND, int T, int O, int NSUM, int BW, int BH>
 __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, double* __restrict__ store, Comps cm,
-                                                        double charge_mass_ratio) {
+                                                        double charge_mass_ratio, int32_t* __restrict__ next) {
     using St = Stencil<KIND, T, O>;
     constexpr int S = St::S, N = St::N, PP = St::PP, U = St::U, CHUNK = St::CHUNK, ENT = St::ENT, SEQ = St::seq(BW * BH);
     constexpr int NW = BW + S - 1, NH = BH + S - 1;   // window, in cells
@@ -285,7 +295,11 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
     // the wide runs whose box meets the window, sorted, when they hold them all; otherwise
     // (listed == false) those whose box meets the window, found through the two levels of boxes,
     // LIST at most by one call; pos is where the next goes on.
-    const int own = v.count[b], wide = v.count[v.nbx * v.nby];
+    const int nblk = v.nbx * v.nby, set = v.set[MADE];
+    // both sets' loads in flight with that of the set's number
+    const int own2[2] = {v.count[b], v.count[nblk + 1 + b]}, wide2[2] = {v.count[nblk], v.count[2 * nblk + 1]};
+    const int own = set ? own2[1] : own2[0], wide = set ? wide2[1] : wide2[0];
+    if (blockIdx.x == 0 && lane == 0) *next = set ^ 1;
     const bool listed = own <= LIST && wide <= LIST && own + wide <= LIST;
     struct Pos {
         int s0 = 0;            // next second-level box
@@ -752,8 +766,8 @@ OrdView view(const hpq_ctx* c, const PlasmaOrder& L, long n, int& wx, int& wy) {
     v.cell = L.cell;
     v.rbox = reinterpret_cast<const int4*>(L.boxes);
     v.sbox = v.rbox + v.nrun;
-    const long nblk = long(v.nbx) * v.nby;
-    v.count = L.count + (L.pick ? nblk + 1 : 0);
+    v.count = L.count + SET_WORDS;
+    v.set = L.count;
     v.list = L.list;
     return v;
 }
@@ -767,23 +781,21 @@ OrdView make_records(hpq_ctx* c, const hpq_plasma* p, double charge_invvol) {
     grow(L.rec, L.rec_cap, n * REC);
     grow(L.cell, L.cell_cap, n);
     grow(L.boxes, L.boxes_cap, 4 * ((n + RUN - 1) / RUN + (n + SUPER - 1) / SUPER));
-    // two sets of run counts: every pass clears the next one's
     OrdView size{};
     blocks(g, size);
     const long nblk = long(size.nbx) * size.nby;
-    if (!L.count) {
-        grow(L.list, L.list_cap, (nblk + 1) * LIST);
-        grow(L.count, L.count_cap, 2 * (nblk + 1));
-        hipLaunchKernelGGL(k_clear_counts, grid1d(2 * (nblk + 1), 256), dim3(256), 0, c->stream, L.count, 2 * (nblk + 1));
-    }
-    L.pick ^= 1;
+    const long words = SET_WORDS + 2 * (nblk + 1);
+    grow(L.list, L.list_cap, (nblk + 1) * LIST);
+    grow(L.count, L.count_cap, words);
     int wx, wy;
     const OrdView v = view(c, L, n, wx, wy);
-    int32_t* count = L.count + (L.pick ? nblk + 1 : 0);
-    int32_t* next_count = L.count + (L.pick ? 0 : nblk + 1);
+    // the first pass, and the one after a pass whose deposition was not launched
+    if (L.unclear) hipLaunchKernelGGL(k_clear_counts, grid1d(words, 256), dim3(256), 0, c->stream, L.count, words);
+    L.unclear = true;
     hipLaunchKernelGGL((k_records<BASE, QSA>), dim3(unsigned(v.nsuper)), dim3(REC_T), 0, c->stream, g, *p, v, wx, wy,
                        charge_invvol, c->p.max_qsa, L.rec, L.cell, reinterpret_cast<int4*>(L.boxes),
-                       reinterpret_cast<int4*>(L.boxes) + v.nrun, count, L.list, next_count, c->d_count);
+                       reinterpret_cast<int4*>(L.boxes) + v.nrun, L.count + SET_WORDS, L.list, L.count + MADE,
+                       c->d_count);
     HPQ_HIP(hipGetLastError());
     return v;
 }
@@ -791,12 +803,14 @@ OrdView make_records(hpq_ctx* c, const hpq_plasma* p, double charge_invvol) {
 template <int KIND, int T, int O, int NSUM>
 void launch_deposit(hpq_ctx* c, const OrdView& v, double* store, const Comps& cm, double ratio) {
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(unsigned(v.nbx * v.nby)), dim3(64), 0, c->stream, c->g, v, store, cm, ratio);
+        hipLaunchKernelGGL(kernel, dim3(unsigned(v.nbx * v.nby)), dim3(64), 0, c->stream, c->g, v, store, cm, ratio,
+                           c->ord_plasma.count + NEXT);
     };
     if (v.lw == 4) launch(k_deposit_ordered<KIND, T, O, NSUM, 16, 8>);
     else if (v.lh == 3) launch(k_deposit_ordered<KIND, T, O, NSUM, 8, 8>);
     else launch(k_deposit_ordered<KIND, T, O, NSUM, 8, 4>);
     HPQ_HIP(hipGetLastError());
+    c->ord_plasma.unclear = false;
 }
 
 void check_count(const hpq_plasma* p) {
