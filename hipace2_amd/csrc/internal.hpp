@@ -184,7 +184,7 @@ struct Bins {
 // the current deposition on the same state.
 struct PlasmaOrder {
     double* rec = nullptr;
-    uint32_t* cell = nullptr;
+    uint32_t* cell = nullptr;                    // and, after those of all particles, their links
     int32_t* boxes = nullptr;
     int32_t *count = nullptr, *list = nullptr;   // runs of particles listed per deposition block
     long rec_cap = 0, cell_cap = 0, boxes_cap = 0, count_cap = 0, list_cap = 0;

@@ -18,17 +18,19 @@
 //            record, its cell as one word, and the bounding boxes of the cells of every RUN
 //            and every SUPER consecutive particles (the QSA removal of the deposit functor
 //            happens here); every run is listed at the blocks whose window (the cells a particle
-//            reaching the block can start in) its box meets;
+//            reaching the block can start in) its box meets, or, where these are many, its
+//            particles are linked into lists by cell;
 //   deposit  a wavefront sorts its list, takes the window's particles from the listed runs by
-//            index, sequences them by colour, and adds them to its block's sums in LDS.
-// The work depends on the number of particles in a window, not on their order, so crossing
-// orbits cost nothing extra. Measured at 511 x 511, 2 x 2 particles per cell, order 2, in us of
-// kernels, with per-cell lists (built by counting, scanning and scattering; walked cell by
-// cell, block by block in raster order where the plasma is near its lattice and merged by
-// index elsewhere) and now:
-//                                 lists / records   current      explicit
-//   linear wake (near the lattice)   52 -> 37      115 -> 110   221 -> 183
-//   nonlinear wake (crossing)        55 -> 44      422 -> 138  1328 -> 275
+//            index and the linked ones with them, sequences them by colour, and adds them to its
+//            block's sums in LDS.
+// What a window's particles cost to add does not depend on the order of the arrays; what they cost
+// to find does. Measured at 511 x 511, 2 x 2 particles per cell, order 2, in us of kernels, with
+// per-cell lists (built by counting, scanning and scattering; walked cell by cell, block by block
+// in raster order where the plasma is near its lattice and merged by index elsewhere) and now:
+//                                        lists / records   current      explicit
+//   linear wake (near the lattice)          51 -> 36      123 -> 111   229 -> 191
+//   nonlinear wake (crossing)               57 -> 39      402 -> 131  1313 -> 249
+//   arrays in random order (linked)        222 -> 58      342 -> 231  1034 -> 319
 //
 // A particle's cell is the floor of the cell-scaled position the shape functions take theirs
 // from (floor(xmid) or floor(xmid + 1/2)); a stencil's start cell is that floor plus a
@@ -52,8 +54,9 @@ constexpr int RUNS_PER_SUPER = SUPER / RUN;
 constexpr uint32_t NO_CELL = 0xffffffffu;
 constexpr int REC = 8;           // doubles per record
 constexpr int LIST = 128;        // runs listed per block
-constexpr int WIDE = 512;        // a run that meets more blocks than this goes to one list for all
-constexpr int NEXT = 0, MADE = 16, SET_WORDS = 32;   // words of OrdView::set, on lines of their own
+constexpr int NEXT = 0, MADE = 16, PASS_WORDS = 32;   // words of OrdView::pass, on lines of their own
+constexpr int BIN = 2;           // log2 of the width and height of a bin of linked particles
+constexpr int HEADS = 8;         // linked lists per bin
 
 // Records, cells and boxes of one plasma state. Cells count from (bxlo, bylo): x in the low
 // `shift` bits of the word, y above them. A box is (xmin, xmax, ymin, ymax), empty when
@@ -65,18 +68,33 @@ struct OrdView {
     int lw, lh;        // log2 of a block's width and height
     int nbx, nby;      // blocks
     int mlo, mhi;      // cells a block's window reaches below and above it
+    int narrow;        // blocks that a listed run meets, at most
     long n;
     const double* __restrict__ rec;
     const uint32_t* __restrict__ cell;
     const int4* __restrict__ rbox;
     const int4* __restrict__ sbox;
-    // Runs listed per block, then the wide ones (may exceed LIST): two sets. A records pass uses the
-    // set that set[NEXT] names, clears the other and notes its own in set[MADE]; the deposition that
-    // reads the set then names the other one. What is to be clear and what is not lives on the
-    // device alone, so that a captured pass may be replayed any number of times.
+    // Runs listed per block (may exceed LIST), then whether particles are linked: two sets, those of
+    // even and of odd passes, each cleared by the pass before.
     const int32_t* __restrict__ count;
-    const int32_t* __restrict__ set;
-    const int32_t* __restrict__ list;    // LIST runs per block and of the wide ones, in any order
+    const int32_t* __restrict__ list;    // LIST runs per block, in any order
+    // Kept beside these arrays, and found from them by the few that need it, since a kernel argument
+    // takes a register all along:
+    // Passes are numbered on the device. A records pass takes the number in pass()[NEXT] and notes it
+    // in pass()[MADE], the deposition that reads it sets pass()[NEXT] to the one after. Nothing that a
+    // pass depends on is kept by the host, so that a recorded pass may be replayed any number of times.
+    __host__ __device__ const int32_t* pass() const { return count - PASS_WORDS; }
+    // The particles of runs that meet too many blocks, linked by the bin of their cell in HEADS
+    // lists each: the pass that made the list in the high word, particle + 1 in the low one, and the
+    // next of a particle's list + 1 (0: none) in link().
+    __host__ __device__ const unsigned long long* head() const {
+        return reinterpret_cast<const unsigned long long*>(count + 2 * (nbx * nby + 1));
+    }
+    __host__ __device__ const uint32_t* link() const { return cell + n; }
+    __host__ __device__ static int bins(int cells, int ng) { return (cells_found(cells, ng) + (1 << BIN) - 1) >> BIN; }
+    // cells counted in one direction: every start cell whose stencil (at most 6 wide, start at most 2
+    // below the cell) reaches the guarded plane has its cell among them
+    __host__ __device__ static int cells_found(int cells, int ng) { return cells + 2 * ng + 9; }
 };
 
 // The deposit functor's per-particle values of the current and explicit deposition
@@ -104,19 +122,21 @@ __device__ __forceinline__ PlasmaVals plasma_vals(const Geom& g, const hpq_plasm
 // Records of SUPER consecutive particles per workgroup, RUN of them per wavefront. QSA: the
 // removal of the current deposit functor (PlasmaDepositCurrent.cpp:182-198).
 // wx, wy: particles whose cell lies outside [0, wx) x [0, wy) reach no cell of the plane.
-// Bound by HBM: 52 bytes read and 68 written per particle.
+// Bound by HBM: 52 bytes read and 68 written per particle. Where all particles are linked (random
+// order), by one atomic exchange for each, 22 us more at a million particles.
 constexpr int REC_T = SUPER;
 template <int BASE, bool QSA>
 __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView v, int wx, int wy,
                                                    double charge_invvol, double max_qsa, double* __restrict__ rec,
                                                    uint32_t* __restrict__ cell, int4* __restrict__ rbox,
                                                    int4* __restrict__ sbox, int32_t* __restrict__ counts,
-                                                   int32_t* __restrict__ list, int32_t* __restrict__ made,
+                                                   int32_t* __restrict__ list, unsigned long long* __restrict__ head,
+                                                   uint32_t* __restrict__ link, int32_t* __restrict__ made,
                                                    int* __restrict__ qsa_count) {
     __shared__ int box[4];
     const int nblk = v.nbx * v.nby;
-    const int set = v.set[NEXT];
-    int32_t* const count = counts + long(set) * (nblk + 1);
+    const unsigned pass = unsigned(v.pass()[NEXT]);
+    int32_t* const count = counts + long(pass & 1) * (nblk + 1);
     if (threadIdx.x < 4) box[threadIdx.x] = (threadIdx.x & 1) ? -1 : INT_MAX;
     __syncthreads();
     const long ip = long(blockIdx.x) * SUPER + threadIdx.x;
@@ -146,44 +166,109 @@ __global__ __launch_bounds__(REC_T) void k_records(Geom g, hpq_plasma p, OrdView
         }
         cell[ip] = w;
     }
-    int x0 = bx >= 0 ? bx : INT_MAX, x1 = bx, y0 = by >= 0 ? by : INT_MAX, y1 = by;
+    // the bounding box of the cells of the wavefront's particles that `of` selects
+    auto bounds = [&](bool of) -> int4 {
+        int4 q = make_int4(of ? bx : INT_MAX, of ? bx : -1, of ? by : INT_MAX, of ? by : -1);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        x0 = min(x0, __shfl_xor(x0, o));
-        x1 = max(x1, __shfl_xor(x1, o));
-        y0 = min(y0, __shfl_xor(y0, o));
-        y1 = max(y1, __shfl_xor(y1, o));
-    }
-    if ((threadIdx.x & 63) == 0 && ip < p.n) {
-        rbox[ip / RUN] = make_int4(x0, x1, y0, y1);
-        atomicMin(&box[0], x0);
-        atomicMax(&box[1], x1);
-        atomicMin(&box[2], y0);
-        atomicMax(&box[3], y1);
-    }
-    // the run into the list of every block whose window its box meets
-    if (x0 <= x1) {
+        for (int o = 32; o > 0; o >>= 1) {
+            q.x = min(q.x, __shfl_xor(q.x, o));
+            q.y = max(q.y, __shfl_xor(q.y, o));
+            q.z = min(q.z, __shfl_xor(q.z, o));
+            q.w = max(q.w, __shfl_xor(q.w, o));
+        }
+        return q;
+    };
+    // the blocks whose window a box meets
+    struct Met {
+        int bx0, bx1, by0, by1, nx, n;
+    };
+    auto met = [&](const int4& q) -> Met {
         const int c0 = v.bxlo + g.ng, r0 = v.bylo + g.ng;   // cell 0 counted from block 0's first
-        const int bx0 = max(x0 + c0 - v.mhi, 0) >> v.lw, bx1 = min((x1 + c0 + v.mlo) >> v.lw, v.nbx - 1);
-        const int by0 = max(y0 + r0 - v.mhi, 0) >> v.lh, by1 = min((y1 + r0 + v.mlo) >> v.lh, v.nby - 1);
-        const int nx = bx1 - bx0 + 1, nb = nx > 0 && by1 >= by0 ? nx * (by1 - by0 + 1) : 0;
-        const int run = int(ip / RUN);
-        if (nb > WIDE) {
-            if ((threadIdx.x & 63) == 0) {
-                const int at = atomicAdd(&count[nblk], 1);
-                if (at < LIST) list[long(nblk) * LIST + at] = run;
-            }
+        Met m;
+        m.bx0 = max(q.x + c0 - v.mhi, 0) >> v.lw;
+        m.bx1 = min((q.y + c0 + v.mlo) >> v.lw, v.nbx - 1);
+        m.by0 = max(q.z + r0 - v.mhi, 0) >> v.lh;
+        m.by1 = min((q.w + r0 + v.mlo) >> v.lh, v.nby - 1);
+        m.nx = m.bx1 - m.bx0 + 1;
+        m.n = m.nx > 0 && m.by1 >= m.by0 ? m.nx * (m.by1 - m.by0 + 1) : 0;
+        return m;
+    };
+    // the run into the lists of blocks
+    const int lane = int(threadIdx.x & 63);
+    auto into_lists = [&](const Met& m) {
+        for (int t = lane; t < m.n; t += 64) {
+            const int blk = (m.by0 + t / m.nx) * v.nbx + m.bx0 + t % m.nx;
+            const int at = atomicAdd(&count[blk], 1);
+            if (at < LIST) list[long(blk) * LIST + at] = int(ip / RUN);
+        }
+    };
+    int4 q = bounds(bx >= 0);
+    if (q.x <= q.y) {
+        const Met m = met(q);
+        if (m.n <= v.narrow) {
+            into_lists(m);
         } else {
-            for (int t = int(threadIdx.x & 63); t < nb; t += 64) {
-                const int blk = (by0 + t / nx) * v.nbx + bx0 + t % nx;
-                const int at = atomicAdd(&count[blk], 1);
-                if (at < LIST) list[long(blk) * LIST + at] = run;
+            // Up to four pieces, split along the longer side: the end of one lattice row and the start
+            // of the next, particles on either side of a periodic boundary, a stray one. Where these
+            // meet too many blocks as well, or one block twice, the particles go by themselves.
+            auto halve = [&](bool of, const int4& r, bool& low) {   // true: along x
+                const bool along = r.y - r.x >= r.w - r.z;
+                low = of && (along ? bx <= (r.x + r.y) >> 1 : by <= (r.z + r.w) >> 1);
+                return along;
+            };
+            auto apart = [&](bool along, const Met& a, const Met& b) {
+                return a.n == 0 || b.n == 0 || (along ? a.bx1 < b.bx0 : a.by1 < b.by0);
+            };
+            bool of[2], low;
+            const bool along = halve(bx >= 0, q, of[0]);
+            of[1] = bx >= 0 && !of[0];
+            int4 half[2];
+            Met m[4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                half[h] = bounds(of[h]);
+                m[2 * h] = met(half[h]);
+                m[2 * h + 1] = Met{};
+            }
+            bool pieces = apart(along, m[0], m[2]);
+            if (pieces && m[0].n + m[2].n > v.narrow) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool al = halve(of[h], half[h], low);
+                    const Met a = met(bounds(low)), b = met(bounds(of[h] && !low));
+                    if (apart(al, a, b)) {
+                        m[2 * h] = a;
+                        m[2 * h + 1] = b;
+                    }
+                }
+                pieces = m[0].n + m[1].n + m[2].n + m[3].n <= v.narrow;
+            }
+            if (pieces) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) into_lists(m[k]);
+            } else {
+                if (bx >= 0) {
+                    const long k = (long(by >> BIN) * OrdView::bins(g.nx, g.ng) + (bx >> BIN)) * HEADS + ip % HEADS;
+                    const unsigned long long mine = (unsigned long long)pass << 32 | unsigned(ip + 1);
+                    const unsigned long long old = atomicExch(&head[k], mine);
+                    link[ip] = unsigned(old >> 32) == pass ? uint32_t(old) : 0u;
+                }
+                // read by later launches only, so that each L2 may gather the stores
+                if (lane == 0) __hip_atomic_store(&count[nblk], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                q = make_int4(INT_MAX, -1, INT_MAX, -1);   // found through the bins, not the boxes
             }
         }
     }
-    int32_t* const next_count = counts + long(set ^ 1) * (nblk + 1);
+    if (lane == 0 && ip < p.n) {
+        rbox[ip / RUN] = q;
+        atomicMin(&box[0], q.x);
+        atomicMax(&box[1], q.y);
+        atomicMin(&box[2], q.z);
+        atomicMax(&box[3], q.w);
+    }
+    int32_t* const next_count = counts + long(~pass & 1) * (nblk + 1);
     for (int t = int(blockIdx.x) * REC_T + int(threadIdx.x); t <= nblk; t += int(gridDim.x) * REC_T) next_count[t] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *made = set;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *made = int(pass);
     __syncthreads();
     if (threadIdx.x == 0) sbox[blockIdx.x] = make_int4(box[0], box[1], box[2], box[3]);
 }
@@ -234,9 +319,9 @@ struct Stencil {
     // Entries sequenced at a time with blocks of `cells` cells, found in the place of the staged
     // ones; where a window holds more, its colours are taken one after the other, each from all
     // runs. The largest block's current deposition has room for 2048 without losing a wavefront
-    // per CU: 138 instead of 182 us for crossing orbits at 511 x 511, 2 x 2 particles per cell. The
-    // explicit one has not: with 1920 entries and 27 particles staged at a time it takes 243 instead
-    // of 275 us there, but 205 instead of 194 near the lattice.
+    // per CU: 131 instead of 156 us for crossing orbits at 511 x 511, 2 x 2 particles per cell, the
+    // same near the lattice. The explicit one has not: with 1920 entries and 27 particles staged at a
+    // time it takes 233 instead of 249 us there, but 201 instead of 191 near the lattice.
     static constexpr int seq(int cells) {
         const int room = CHUNK * ENT * 8, want = KIND == CURRENT && cells == 128 ? 2048 : 1024;
         return room < want ? room : want;
@@ -259,7 +344,7 @@ struct Stencil {
 // 60 vector instructions (42 of them FP64) on each of four SIMDs. A 16 x 8 block keeps the
 // window of an order-2 derivative stencil at 1.9 times its cells and gives 511 x 511 cells
 // 2145 wavefronts; CHUNK, SEQ and BS are chosen so that nine of them fit a CU's LDS, one round
-// for that grid (eight in two rounds: 212 instead of 183 us). Smaller grids have smaller blocks.
+// for that grid (eight in two rounds: 211 instead of 191 us). Smaller grids have smaller blocks.
 // NSUM: the sums of a cell (CURRENT: components asked for, at most NSUM).
 template <int KIND, int T, int O, int NSUM, int BW, int BH>
 __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, double* __restrict__ store, Comps cm,
@@ -275,8 +360,15 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
     __shared__ double sum[NSUM][CELLS];
     // entries: colour << 13 | listed run << 6 | particle of the run, first by index (found, in the
     // place of the staged entries), then by colour
-    __shared__ uint16_t seq[SEQ];
+    __shared__ alignas(8) uint16_t seq[SEQ];
     uint16_t* const found = reinterpret_cast<uint16_t*>(&ent[0][0]);
+    // with linked particles the sequence holds particle indices, sorted in the place of the staged
+    // entries (see below)
+    uint32_t* const seq_ip = reinterpret_cast<uint32_t*>(seq);
+    uint32_t* const key = reinterpret_cast<uint32_t*>(&ent[0][0]);
+    constexpr int KEYS = sizeof(ent) >= 4096 ? 1024 : 512;
+    constexpr int KEEP = KEYS / 2 < SEQ / 2 ? KEYS / 2 : SEQ / 2;
+    static_assert(sizeof(ent) >= KEYS * sizeof(uint32_t) && KEYS - KEEP >= 2 * RUN, "room for the keys");
     static_assert(sizeof(ent) >= SEQ * sizeof(uint16_t), "the found entries fit");
     __shared__ int runs[LIST];
     __shared__ uint16_t supers[SUPER_BATCH];
@@ -291,16 +383,29 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
 
     auto meets = [&](const int4& q) { return q.y >= X0 && q.x < X0 + NW && q.w >= Y0 && q.z < Y0 + NH; };
 
-    // Runs of particles that may hold some of the window, by index. The block's own list and
-    // the wide runs whose box meets the window, sorted, when they hold them all; otherwise
-    // (listed == false) those whose box meets the window, found through the two levels of boxes,
-    // LIST at most by one call; pos is where the next goes on.
-    const int nblk = v.nbx * v.nby, set = v.set[MADE];
-    // both sets' loads in flight with that of the set's number
-    const int own2[2] = {v.count[b], v.count[nblk + 1 + b]}, wide2[2] = {v.count[nblk], v.count[2 * nblk + 1]};
-    const int own = set ? own2[1] : own2[0], wide = set ? wide2[1] : wide2[0];
-    if (blockIdx.x == 0 && lane == 0) *next = set ^ 1;
-    const bool listed = own <= LIST && wide <= LIST && own + wide <= LIST;
+    // Runs of particles that may hold some of the window, by index. The block's own list, sorted,
+    // when it holds them all; otherwise (listed == false) those whose box meets the window, found
+    // through the two levels of boxes, LIST at most by one call; pos is where the next goes on.
+    const int nblk = v.nbx * v.nby, pass = v.pass()[MADE];
+    // both sets' loads in flight with that of the pass
+    const int own2[2] = {v.count[b], v.count[nblk + 1 + b]}, any2[2] = {v.count[nblk], v.count[2 * nblk + 1]};
+    const int own = pass & 1 ? own2[1] : own2[0], any_linked = pass & 1 ? any2[1] : any2[0];
+    if (blockIdx.x == 0 && lane == 0) *next = pass + 1;
+    const bool listed = own <= LIST;
+    // the lists of the bins that the window meets, and whether they hold any particle
+    const int binx = X0 >> BIN, biny = Y0 >> BIN;
+    const int nbinx = OrdView::bins(g.nx, g.ng), nbinw = min((X0 + NW - 1) >> BIN, nbinx - 1) - binx + 1;
+    const int nlinks = nbinw * (min((Y0 + NH - 1) >> BIN, OrdView::bins(g.ny, g.ng) - 1) - biny + 1) * HEADS;
+    auto first_linked = [&](int t) -> uint32_t {
+        const int bin = t / HEADS, r = bin / nbinw;
+        const unsigned long long h = v.head()[(long(biny + r) * nbinx + binx + bin - r * nbinw) * HEADS + t % HEADS];
+        return unsigned(h >> 32) == unsigned(pass) ? uint32_t(h) : 0u;
+    };
+    bool linked = false;
+    if (any_linked) {
+        for (int t = lane; t < nlinks; t += 64) linked |= first_linked(t) != 0u;
+        linked = __ballot(linked) != 0ull;
+    }
     struct Pos {
         int s0 = 0;            // next second-level box
         int first = 0;         // first box of the current batch
@@ -375,19 +480,14 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
         for (int q = 0; q < 2; ++q) {
             const int t = lane + 64 * q;
             mine[q] = INT_MAX;
-            if (t < own) {
-                mine[q] = v.list[long(b) * LIST + t];
-            } else if (t < own + wide) {
-                mine[q] = v.list[long(v.nbx) * v.nby * LIST + t - own];
-                if (!meets(v.rbox[mine[q]])) mine[q] = INT_MAX;
-            }
+            if (t < own) mine[q] = v.list[long(b) * LIST + t];
             reinterpret_cast<int*>(unsorted)[t] = mine[q];
-            nruns += __popcll(__ballot(mine[q] != INT_MAX));
         }
+        nruns = own;
         __syncthreads();
         int rank[2] = {0, 0};
 #pragma unroll 4
-        for (int t = 0; 4 * t < own + wide; ++t) {
+        for (int t = 0; 4 * t < own; ++t) {
             const int4 r = unsorted[t];
 #pragma unroll
             for (int q = 0; q < 2; ++q)
@@ -399,7 +499,7 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
             if (mine[q] != INT_MAX) runs[rank[q]] = mine[q];
         __syncthreads();
         pos.end = true;
-    } else {
+    } else if (!linked) {
         nruns = find_runs();
     }
 
@@ -418,8 +518,13 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
     auto fetch = [&](int e) -> Record {
         Record r;
         if (lane < CHUNK && e < n) {
-            const int id = seq[e];
-            const long ip = long(runs[(id >> 6) & 127]) * RUN + (id & 63);
+            long ip;
+            if (linked) {
+                ip = long(seq_ip[e]);
+            } else {
+                const int id = seq[e];
+                ip = long(runs[(id >> 6) & 127]) * RUN + (id & 63);
+            }
             const double2* p = reinterpret_cast<const double2*>(v.rec + ip * REC);
 #pragma unroll
             for (int f = 0; f < 4; ++f) r.d[f] = p[f];
@@ -652,18 +757,138 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
         }
         __syncthreads();
     };
+    // With linked particles in the window: colour by colour, KEEP particles at a time. Of those from
+    // index `lo` on the lowest are taken, from the linked lists, whose order is that of chance, and from
+    // the runs, which go by index; sorted, they are the sequence, and the next one starts where it
+    // ends (`hi`). Every round walks the lists again: a lane follows one of HEADS lists of a bin, so
+    // that a walk is as long as a bin has particles / HEADS, 8 loads after one another at 2 x 2 particles
+    // per cell, three times for the window's bins (of 4 lists, 16 and twice: 300 and 308 us for all of
+    // the current deposition at 511 x 511, but 534 and 408 us with 2000 particles more in one spot of
+    // 127 x 127). Walks, sorts and records read out of order make the current deposition of a
+    // plasma in random order take 231 instead of 111 us (511 x 511, 2 x 2 particles per cell). When
+    // such a plasma's runs were all tested by every block, it took 15 ms.
+    auto window_colour = [&](uint32_t w) -> int {
+        const unsigned x = unsigned(int(w & xmask) - X0), y = unsigned(int(w >> v.shift) - Y0);
+        if (w == NO_CELL || x >= unsigned(NW) || y >= unsigned(NH)) return 4;
+        return int((PX >> (x & 63)) & 1ull) * 2 + int((PY >> (y & 63)) & 1ull);
+    };
+    // the first cnt keys sorted (bitonic, the next power of two of them)
+    auto sort_keys = [&](int cnt) {
+        int P = 64;
+        while (P < cnt) P <<= 1;
+        for (int t = cnt + lane; t < P; t += 64) key[t] = ~0u;
+        __syncthreads();
+        for (int k = 2; k <= P; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+#pragma unroll 4
+                for (int t = lane; t < P / 2; t += 64) {
+                    const int i = 2 * (t & ~(j - 1)) | (t & (j - 1));
+                    const uint32_t a = key[i], c = key[i | j];
+                    const bool up = (i & k) == 0;
+                    key[i] = up == (a < c) ? a : c;
+                    key[i | j] = up == (a < c) ? c : a;
+                }
+                __syncthreads();
+            }
+    };
+    auto collect_linked = [&](int colour, uint32_t lo) -> uint32_t {
+        constexpr int AHEAD = 8;
+        uint32_t hi = ~0u;
+        int cnt = 0;
+        // the KEEP lowest of the keys so far
+        auto cut = [&] {
+            sort_keys(cnt);
+            hi = uint32_t(__builtin_amdgcn_readfirstlane(int(key[KEEP])));
+            cnt = KEEP;
+            __syncthreads();
+        };
+        __syncthreads();
+        for (int t0 = 0;; t0 += 64) {
+            const bool last = t0 >= nlinks;   // room for the runs, too
+            uint32_t p = t0 + lane < nlinks ? first_linked(t0 + lane) : 0u;
+            do {
+                uint32_t w = NO_CELL, after = 0u;
+                if (p) {
+                    w = v.cell[p - 1];
+                    after = v.link()[p - 1];
+                }
+                if (cnt > (last ? KEEP : KEYS - 64)) cut();
+                const bool hit = window_colour(w) == colour && p - 1 >= lo && p - 1 < hi;
+                const unsigned long long h = __ballot(hit);
+                if (hit) key[cnt + lanes_before(h)] = p - 1;
+                cnt += __popcll(h);
+                p = after;
+            } while (__ballot(p != 0u) != 0ull);
+            if (last) break;
+        }
+        __syncthreads();
+        if (!listed) {
+            pos = Pos{};
+            pos.s0 = int(lo / SUPER);
+            nruns = 0;
+        }
+        for (int t = 0;; t += AHEAD) {
+            if (t >= nruns) {
+                if (pos.end) break;
+                nruns = find_runs();
+                t = 0;
+            }
+            uint32_t w[AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q) {
+                const long ip = t + q < nruns ? long(runs[t + q]) * RUN + lane : v.n;
+                w[q] = ip < v.n && ip >= long(lo) && ip < long(hi) ? v.cell[ip] : NO_CELL;
+            }
+            bool full = false;
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q) {
+                if (full || t + q >= nruns) continue;
+                const uint32_t first = uint32_t(__builtin_amdgcn_readfirstlane(runs[t + q])) * RUN;
+                if (first >= hi || cnt > KEYS - RUN) {
+                    hi = min(hi, first);
+                    full = true;
+                    continue;
+                }
+                const bool hit = window_colour(w[q]) == colour;
+                const unsigned long long h = __ballot(hit);
+                if (hit) key[cnt + lanes_before(h)] = first + unsigned(lane);
+                cnt += __popcll(h);
+            }
+            if (full) break;
+        }
+        __syncthreads();
+        sort_keys(cnt);
+        // those below hi, KEEP at most
+        int m = 0;
+        for (int t0 = 0; t0 < cnt; t0 += 64) m += __popcll(__ballot(t0 + lane < cnt && key[t0 + lane] < hi));
+        if (m > KEEP) {
+            m = KEEP;
+            hi = uint32_t(__builtin_amdgcn_readfirstlane(int(key[KEEP])));
+        }
+        for (int t = lane; t < m; t += 64) seq_ip[t] = key[t];
+        n = m;
+        __syncthreads();
+        return hi;
+    };
     // All colours at once when their entries fit, otherwise colour by colour; `all`: one list
     // holds every run of the window.
     const bool all = pos.end;
+    bool together = all && !linked;   // for the first sequence
     unsigned mask = present;
-    int t = all ? collect(present, 0) : 0;
-    const bool fits = all && t >= nruns;
-    if (!fits) t = 0;
-    int colour = 0;
+    int t = 0, colour = 0;
+    uint32_t lo = 0u;   // linked: where the next sequence starts, all ones after a colour's last
     while (true) {
-        if (!fits) {
+        if (linked) {
+            if (lo == ~0u) {
+                ++colour;
+                lo = 0u;
+            }
+            while (colour < 4 && !((present >> colour) & 1u)) ++colour;
+            if (colour > 3) break;
+            lo = collect_linked(colour, lo);
+        } else {
             // the next entries of this colour
-            while (colour < 4) {
+            while (!together && colour < 4) {
                 mask = present & (1u << colour);
                 if (mask && t < nruns) break;
                 if (mask && !pos.end) {
@@ -673,16 +898,21 @@ __global__ __launch_bounds__(64) void k_deposit_ordered(Geom g, OrdView v, doubl
                 }
                 ++colour;
                 t = 0;
-                if (!all && colour < 4) {
+                if (!all) {
                     pos = Pos{};
-                    nruns = find_runs();
+                    nruns = 0;
                 }
             }
             if (colour > 3) break;
             t = collect(mask, t);
+            if (together && t < nruns) {   // too many: colour by colour from the first run
+                together = false;
+                t = 0;
+                continue;
+            }
         }
         run_sequence();
-        if (fits) break;
+        if (together) break;
     }
     __syncthreads();
     for (int t = lane; t < BW * BH; t += 64) {
@@ -724,10 +954,13 @@ int bits(long v) {
 // The blocks of a grid: 16 x 8 cells, 8 x 8 or 8 x 4, the largest of which there are as many as
 // the CUs hold wavefronts at once, or the smallest. A larger block's window holds fewer
 // particles that other blocks take as well; too few blocks leave the chip idle, and a wavefront
-// takes its particles one after the other. Measured for a near-lattice plasma of one particle per
-// cell, order 2, current + explicit in us, with 16 x 8, 8 x 8 and 8 x 4 cells:
-//    63 x 63 52, 37, 31; 127 x 127 60, 47, 39; 255 x 255 71, 62, 54; 383 x 383 84, 74, 95;
-//   511 x 511 106, 126, 145 (2 x 2 particles per cell 310, 337, 370).
+// takes its particles one after the other. Measured at order 2, current + explicit in us, with
+// 16 x 8, 8 x 8 and 8 x 4 cells:
+//   near the lattice, one particle per cell: 63 x 63 53, 39, 32; 127 x 127 62, 48, 41;
+//     255 x 255 72, 64, 56; 383 x 383 87, 76, 96; 511 x 511 102, 117, 144 (2 x 2 per cell 300, 316, 347);
+//   crossing orbits, 2 x 2 per cell: 255 x 255 274, 201, 176; 383 x 383 321, 272, 260;
+//     511 x 511 383, 370, 387, where the next smaller blocks would be 4 % faster: the line stays
+//     where the lattice, the usual state, puts it.
 constexpr long FILL = 8 * 256;
 void blocks(const Geom& g, OrdView& v) {
     const int sizes[3][2] = {{4, 3}, {3, 3}, {3, 2}};
@@ -740,15 +973,24 @@ void blocks(const Geom& g, OrdView& v) {
     }
 }
 
-// every start cell whose stencil (at most 6 wide, start at most 2 below the cell) reaches the
-// guarded plane has a cell in [bxlo, bxlo + wx) x [bylo, bylo + wy)
+// Blocks that a listed run meets, at most; a run that meets more has its particles linked. When
+// all runs met LIST * blocks / runs of them, the lists would be full on average, and full lists
+// make a block look for its runs among all boxes, which costs more than links do: the line lies an
+// eighth below, and not below 20, for a run of a lattice meets up to 9 and one of crossing orbits
+// up to 20 whatever their number. Measured with runs spread by random displacements (511 x 511,
+// 2 x 2 particles per cell, current + explicit in us; listed unless they meet 512 blocks, with this
+// line, with one at 16): 7 cells 540, 510, 630; 10 cells 930, 720, 790; 14 cells 1060, 1250, 720;
+// 20 cells 1290, 730, 670; 40 cells 2260, 710, 700.
+constexpr long NARROW = 20;
+
+// cells are counted in [bxlo, bxlo + wx) x [bylo, bylo + wy)
 OrdView view(const hpq_ctx* c, const PlasmaOrder& L, long n, int& wx, int& wy) {
     const Geom& g = c->g;
     OrdView v{};
     v.bxlo = -g.ng - 6;
     v.bylo = -g.ng - 6;
-    wx = g.nx + 2 * g.ng + 9;
-    wy = g.ny + 2 * g.ng + 9;
+    wx = OrdView::cells_found(g.nx, g.ng);
+    wy = OrdView::cells_found(g.ny, g.ng);
     v.shift = bits(wx);
     if (v.shift + bits(wy) > 31) throw HpqError(HPQ_E_UNSUPPORTED, "ordered deposition: more than 2^31 cells");
     v.T = c->p.tile_size > 0 ? c->p.tile_size : 32;
@@ -766,8 +1008,9 @@ OrdView view(const hpq_ctx* c, const PlasmaOrder& L, long n, int& wx, int& wy) {
     v.cell = L.cell;
     v.rbox = reinterpret_cast<const int4*>(L.boxes);
     v.sbox = v.rbox + v.nrun;
-    v.count = L.count + SET_WORDS;
-    v.set = L.count;
+    const long nblk = long(v.nbx) * v.nby;
+    v.narrow = int(std::min<long>(std::max(NARROW, 7 * LIST * nblk / (8 * long(std::max(v.nrun, 1)))), INT_MAX));
+    v.count = L.count + PASS_WORDS;
     v.list = L.list;
     return v;
 }
@@ -779,23 +1022,22 @@ OrdView make_records(hpq_ctx* c, const hpq_plasma* p, double charge_invvol) {
     const Geom& g = c->g;
     const long n = p->n;
     grow(L.rec, L.rec_cap, n * REC);
-    grow(L.cell, L.cell_cap, n);
+    grow(L.cell, L.cell_cap, 2 * n);
     grow(L.boxes, L.boxes_cap, 4 * ((n + RUN - 1) / RUN + (n + SUPER - 1) / SUPER));
-    OrdView size{};
-    blocks(g, size);
-    const long nblk = long(size.nbx) * size.nby;
-    const long words = SET_WORDS + 2 * (nblk + 1);
-    grow(L.list, L.list_cap, (nblk + 1) * LIST);
-    grow(L.count, L.count_cap, words);
     int wx, wy;
-    const OrdView v = view(c, L, n, wx, wy);
+    OrdView v = view(c, L, n, wx, wy);
+    const long nblk = long(v.nbx) * v.nby;
+    const long words = PASS_WORDS + 2 * (nblk + 1) + 2L * HEADS * OrdView::bins(g.nx, g.ng) * OrdView::bins(g.ny, g.ng);
+    grow(L.list, L.list_cap, nblk * LIST);
+    grow(L.count, L.count_cap, words);
+    v = view(c, L, n, wx, wy);
     // the first pass, and the one after a pass whose deposition was not launched
     if (L.unclear) hipLaunchKernelGGL(k_clear_counts, grid1d(words, 256), dim3(256), 0, c->stream, L.count, words);
     L.unclear = true;
     hipLaunchKernelGGL((k_records<BASE, QSA>), dim3(unsigned(v.nsuper)), dim3(REC_T), 0, c->stream, g, *p, v, wx, wy,
                        charge_invvol, c->p.max_qsa, L.rec, L.cell, reinterpret_cast<int4*>(L.boxes),
-                       reinterpret_cast<int4*>(L.boxes) + v.nrun, L.count + SET_WORDS, L.list, L.count + MADE,
-                       c->d_count);
+                       reinterpret_cast<int4*>(L.boxes) + v.nrun, L.count + PASS_WORDS, L.list,
+                       const_cast<unsigned long long*>(v.head()), L.cell + n, L.count + MADE, c->d_count);
     HPQ_HIP(hipGetLastError());
     return v;
 }

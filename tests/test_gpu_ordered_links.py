@@ -1,0 +1,104 @@
+"""The ordered plasma depositions of plasmas whose array order does not follow space, whose particles
+are linked by cell instead of listed by runs: against the oracle, bit for bit, for random order, a
+lattice in pieces of random order, lattice rows that end in the middle of a run (runs listed in two
+pieces), order by columns, scattered particles among listed runs, more particles in a window than
+are sequenced or sorted at a time, and full lists beside links, on grids of all three block sizes.
+And their time beside that of the same plasma in lattice order.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from helpers import PLASMA_REALS, random_store  # noqa: E402
+from test_gpu_ordered import COMPS, _config, _lattice  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def _ordered(d, cfg, order, rng):
+    n = d["x"].size
+    if order == "random":
+        p = rng.permutation(n)
+    elif order == "pieces":   # of 16 particles
+        m = n // 16 * 16
+        p = np.concatenate([(rng.permutation(m // 16)[:, None] * 16 + np.arange(16)).ravel(), np.arange(m, n)])
+    elif order == "columns":
+        p = np.lexsort((np.floor((d["y"] - cfg.ylo) / cfg.dy), np.floor((d["x"] - cfg.xlo) / cfg.dx)))
+    else:
+        return d
+    return {k: np.ascontiguousarray(v[p]) for k, v in d.items()}
+
+
+def _set(sim, d):
+    """A plasma of any number of particles."""
+    from hipace2_amd import _abi
+    sim.np = d["x"].size
+    for k in PLASMA_REALS:
+        sim.plasma[k] = torch.as_tensor(d[k], dtype=torch.float64).to(sim.device)
+    sim.plasma["valid"] = torch.as_tensor(d["valid"]).to(sim.device)
+    sim._pdesc = _abi.Plasma(*[sim.plasma[k].data_ptr() for k in PLASMA_REALS + ["valid"]], sim.np)
+
+
+# nx, ny, ppc, amp (cells), scattered, spot (particles moved to a spot of two cells), order, tile
+CASES = [(127, 129, 2, 0.5, 0, 0, "random", 32), (127, 129, 2, 0.5, 0, 0, "pieces", 9), (255, 31, 2, 0.5, 0, 0, "rows", 32),
+         (31, 255, 2, 0.5, 0, 0, "columns", 32), (97, 127, 3, 1.0, 200, 0, "rows", 24), (33, 31, 7, 1.0, 0, 0, "random", 8),
+         (33, 31, 7, 1.0, 40, 0, "rows", 32), (127, 65, 2, 0.1, 0, 3000, "random", 32), (365, 373, 1, 0.5, 0, 0, "random", 32),
+         (511, 525, 1, 0.5, 60, 0, "rows", 24), (525, 509, 1, 0.5, 0, 0, "random", 32)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(v) for v in c))
+@pytest.mark.parametrize("order,dtype", [(0, 1), (1, 2), (2, 1), (2, 2), (3, 0), (3, 2)])
+def test_linked_particles(case, order, dtype):
+    from hipace2_amd.simulation import Simulation
+    from oracle.oracle import OracleSim
+    nx, ny, ppc, amp, scattered, spot, arrays, tile = case
+    cfg = _config(nx, ny, order, dtype, tile)
+    rng = np.random.default_rng(nx)
+    d = _lattice(cfg, ppc, amp, scattered, seed=ny)
+    if spot:
+        w = rng.choice(d["x"].size, size=spot, replace=False)
+        for k, n in (("x", cfg.dx), ("y", cfg.dy)):
+            d[k][w] = n * rng.normal(0.3, 1.5, spot)
+            d[k + "_prev"] = d[k].copy()
+    d = _ordered(d, cfg, arrays, rng)
+    sim, orc = Simulation(cfg), OracleSim(cfg)
+    st = random_store(sim.ncomp, sim.ldy, sim.ldx, seed=2)
+    sim.store.copy_(torch.as_tensor(st))
+    orc.set_store(st)
+    orc.set_plasma(d)
+    _set(sim, d)
+    comps = [c if sim.layout[c] >= 0 else -1 for c in COMPS]
+    for cs in (comps, ["jx", "jy", -1, -1, "chi", "rhomjz"]):
+        assert sim.deposit_current(cs) == orc.deposit_plasma(cs)
+    sim.explicit_deposition()
+    orc.explicit_deposit()
+    g, o = sim.store_host(), orc.store()
+    for name in ("jx", "jy", "rho", "chi", "rhomjz", "Sx", "Sy"):
+        assert np.array_equal(g[sim.layout[name]], o[orc.layout[name]]), name
+
+
+@pytest.mark.parametrize("arrays", ["random", "pieces"])
+def test_time_does_not_depend_on_the_order_of_the_arrays(arrays):
+    """Both depositions of a plasma in another order take less than eight times what they take in
+    lattice order (measured: below two; with every block testing every run, 70 to 90)."""
+    from hipace2_amd.simulation import Simulation
+    cfg = _config(511, 511, 2, 2, 32)
+    lattice = _lattice(cfg, 2, 0.1, 0, seed=1)
+    other = _ordered(lattice, cfg, arrays, np.random.default_rng(3))
+    sim = Simulation(cfg)
+
+    def best(d):
+        _set(sim, d)
+        t = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            sim.deposit_current(["jx", "jy", -1, -1, "chi", "rhomjz"])
+            sim.explicit_deposition()
+            b.record()
+            b.synchronize()
+            t.append(a.elapsed_time(b))
+        return min(t)
+
+    assert best(other) < 8 * best(lattice)
