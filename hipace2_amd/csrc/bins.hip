@@ -220,15 +220,6 @@ __global__ void k_bin_offsets(const int32_t* __restrict__ first, int nbins, int 
     if (b == nbins) offsets[b] = int32_t(n);
 }
 
-template <class T>
-void grow(T*& p, long& cap, long need) {
-    if (need <= cap) return;
-    if (p) HPQ_HIP(hipFree(p));
-    p = nullptr;
-    HPQ_HIP(hipMalloc(&p, sizeof(T) * size_t(need)));
-    cap = need;
-}
-
 }  // namespace
 
 // exclusive scan of a[0..n) in place; tmp holds the block sums of every level

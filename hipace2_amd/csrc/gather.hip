@@ -372,15 +372,6 @@ __global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restr
     }
 }
 
-template <class T>
-void grow(T*& p, long& cap, long need) {
-    if (need <= cap) return;
-    if (p) HPQ_HIP(hipFree(p));
-    p = nullptr;
-    HPQ_HIP(hipMalloc(&p, sizeof(T) * size_t(std::max(need, 1L))));
-    cap = need;
-}
-
 // base-cell grid of a context: every start cell whose stencil (at most 6 wide, start at most 2
 // below the base cell) reaches the guarded plane; the deposition tiles
 void lists_geometry(const hpq_ctx* c, CellLists& L) {

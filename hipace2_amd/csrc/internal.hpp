@@ -30,6 +30,19 @@ struct HpqError : std::exception {
     const char* what() const noexcept override { return msg.c_str(); }
 };
 
+// scratch of at least `need` entries; where there is no memory for it, none at all, so that the next
+// call starts anew
+template <class T>
+void grow(T*& p, long& cap, long need) {
+    if (need <= cap) return;
+    cap = 0;
+    T* const old = p;
+    p = nullptr;
+    if (old) HPQ_HIP(hipFree(old));
+    HPQ_HIP(hipMalloc(&p, sizeof(T) * size_t(need)));
+    cap = need;
+}
+
 // Slice geometry. Positions follow GetPosOffset (src/fields/Fields.H:72-77).
 struct Geom {
     int nx = 0, ny = 0, nz = 0, ng = 2;

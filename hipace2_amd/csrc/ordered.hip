@@ -935,16 +935,6 @@ __global__ __launch_bounds__(256) void k_clear_counts(int32_t* __restrict__ a, l
     if (t < n) a[t] = 0;
 }
 
-template <class T>
-void grow(T*& p, long& cap, long need) {
-    if (need <= cap) return;
-    if (p) HPQ_HIP(hipFree(p));
-    p = nullptr;
-    cap = 0;
-    HPQ_HIP(hipMalloc(&p, sizeof(T) * size_t(std::max(need, 1L))));
-    cap = need;
-}
-
 int bits(long v) {
     int b = 0;
     while ((1L << b) <= v) ++b;
