@@ -278,18 +278,24 @@ __global__ __launch_bounds__(256) void k_beam_pairs(Geom g, CLView cl, const int
 }
 
 // Every cell's sum, added to the plane's value in sequence order; jx and jy go together, as in
-// the deposit functor. Workgroups below nshort: a thread per cell with a short sequence. The
-// rest: a wavefront per cell of longc; chunks of 64 contributions per component are read by the
-// whole wavefront into LDS (LCH chunks in flight), and lanes 0-2 add the jx, jy and jz chunks.
-// One launch for both: the predictor-corrector loop runs it in every iteration, where a launch
-// more costs 4 us of some 70.
+// the deposit functor. The first workgroups take a wavefront per cell of longc: chunks of 64
+// contributions per component are read by the whole wavefront into LDS (LCH chunks in flight), and
+// lanes 0-2 add the jx, jy and jz chunks. The last nshort take a thread per cell with a short
+// sequence. One launch for both: the predictor-corrector loop runs it in every iteration, where a
+// launch more costs 4 us of some 60. Bound by the chain of adds of the longest sequences, so these
+// start first, and the wavefronts of a workgroup take cells far apart in the list, whose neighbours
+// are neighbours in the beam's core. Measured for the densest slice of a beam of two million particles
+// at 255 x 255 (hundreds of long sequences, the longest of some 30000) 2.00 ms, of four million at
+// 511 x 511, order 3, 205 us; with two launches, the long ones in workgroups of one wavefront,
+// 2.13 ms and 221 us; with neighbours in one workgroup, after the short ones, 2.52 ms and 289 us.
 __global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restrict__ seg,
                                                   const double* __restrict__ contrib, long m,
                                                   double* __restrict__ store, int cjx, int cjy, int cjz,
                                                   const int32_t* __restrict__ longc, int nshort) {
     const long ps = g.plane;
-    if (int(blockIdx.x) < nshort) {
-        const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int nlong = int(gridDim.x) - nshort;
+    if (int(blockIdx.x) >= nlong) {
+        const long t = long(int(blockIdx.x) - nlong) * blockDim.x + threadIdx.x;
         if (t >= g.plane) return;
         const int a = seg[t], e = seg[t + 1];
         if (a == e || e - a > BEAM_LONG) return;
@@ -320,7 +326,7 @@ __global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restr
     };
     const int comp = lane == 0 ? cjx : lane == 1 ? (cjx >= 0 ? cjy : -1) : lane == 2 ? cjz : -1;
     const int nl = longc[0];
-    for (int w = (int(blockIdx.x) - nshort) * 4 + wave; w < nl; w += (int(gridDim.x) - nshort) * 4) {
+    for (int w = wave * nlong + int(blockIdx.x); w < nl; w += 4 * nlong) {
         const long t = longc[1 + w];
         const int a = seg[t], e = seg[t + 1];
         double acc = comp >= 0 ? store[comp * ps + t] : 0.0;
@@ -352,19 +358,34 @@ __global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restr
                     v[d][2] = contrib[2 * m + hn];
                 }
                 if (comp >= 0) {
-                    // in sequence order; sixteen LDS reads in flight ahead of the adds
+                    // in sequence order; eight LDS reads in flight while the eight before are added
                     const int cnt = min(64, e - hc);
                     const double* row = buf[lane];
-                    int u = 0;
-                    for (; u + 16 <= cnt; u += 16) {
-                        double q[16];
+                    if (cnt == 64) {
+                        double q[2][8];
 #pragma unroll
-                        for (int k = 0; k < 16; ++k) q[k] = row[u + k];
-                        asm volatile("" ::: "memory");
+                        for (int k = 0; k < 8; ++k) q[0][k] = row[k];
 #pragma unroll
-                        for (int k = 0; k < 16; ++k) acc += q[k];
+                        for (int u = 8; u <= 64; u += 8) {
+#pragma unroll
+                            for (int k = 0; k < 8; ++k)
+                                if (u < 64) q[(u / 8) & 1][k] = row[u + k];
+                            asm volatile("" ::: "memory");
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) acc += q[(u / 8 + 1) & 1][k];
+                        }
+                    } else {
+                        int u = 0;
+                        for (; u + 8 <= cnt; u += 8) {
+                            double q[8];
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) q[k] = row[u + k];
+                            asm volatile("" ::: "memory");
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) acc += q[k];
+                        }
+                        for (; u < cnt; ++u) acc += row[u];
                     }
-                    for (; u < cnt; ++u) acc += row[u];
                 }
             }
         }
