@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void k_beam_pairs(Geom g, CLView cl, const int
 // launch more costs 4 us of some 60. Bound by the chain of adds of the longest sequences, so these
 // start first, and the wavefronts of a workgroup take cells far apart in the list, whose neighbours
 // are neighbours in the beam's core. Measured for the densest slice of a beam of two million particles
-// at 255 x 255 (hundreds of long sequences, the longest of some 30000) 2.00 ms, of four million at
+// at 255 x 255 (the longest sequences hold some 300000) 2.00 ms, of four million at
 // 511 x 511, order 3, 205 us; with two launches, the long ones in workgroups of one wavefront,
 // 2.13 ms and 221 us; with neighbours in one workgroup, after the short ones, 2.52 ms and 289 us.
 __global__ __launch_bounds__(256) void k_beam_sum(Geom g, const int32_t* __restrict__ seg,
