@@ -508,7 +508,7 @@ void explicit_deposit_f32(hpq_ctx* c, const hpq_plasma* p, const int32_t* order,
                           double qmr);
 
 #ifndef HPQ_F32_TU
-// the FP64 path in the reference CPU build's summation order (gather.hip)
+// the FP64 path in the reference CPU build's summation order (plasma: ordered.hip, beam: gather.hip)
 static bool ordered(const hpq_ctx* c) {
     return c->p.deposition == HPQ_DEPOSIT_ORDERED && c->p.precision == HPQ_PREC_FP64;
 }

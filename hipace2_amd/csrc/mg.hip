@@ -1593,7 +1593,7 @@ int mg_solve1(hpq_ctx* c, double* sol, const double* rhs, const double* acf, lon
     }
     M.ctl_dirty = true;   // until the solve ends normally
     // average_down_acoef (:1641-1661): level 1 in the initial smoothing, levels 2..cb in the
-    // first V-cycle's down-sweep, the coarse ones inside k_coarse
+    // first V-cycle's down-sweep, the coarse ones inside k_coarse_lds
     // initial smoothing from the guess (buf[1]) into buf[0], the iterate after zero cycles;
     // k_target then sets the convergence target from its residual and rhs max norms
     S.nblk = smooth<4, false, true, false, true, true, true>(c, S.L0, L1, S.buf[0], S.rhs0, S.rcs, S.L0.acf, S.buf[1],
