@@ -41,9 +41,10 @@ def _set(sim, d):
 
 
 # nx, ny, ppc, amp (cells), scattered, spot (particles moved to a spot of two cells), order, tile
-CASES = [(127, 129, 2, 0.5, 0, 0, "random", 32), (127, 129, 2, 0.5, 0, 0, "pieces", 9), (255, 31, 2, 0.5, 0, 0, "rows", 32),
-         (31, 255, 2, 0.5, 0, 0, "columns", 32), (97, 127, 3, 1.0, 200, 0, "rows", 24), (33, 31, 7, 1.0, 0, 0, "random", 8),
-         (33, 31, 7, 1.0, 40, 0, "rows", 32), (127, 65, 2, 0.1, 0, 3000, "random", 32), (365, 373, 1, 0.5, 0, 0, "random", 32),
+CASES = [(127, 129, 2, 0.5, 0, 0, "random", 32), (127, 129, 2, 0.5, 0, 0, "pieces", 9),
+         (255, 31, 2, 0.5, 0, 0, "rows", 32), (31, 255, 2, 0.5, 0, 0, "columns", 32),
+         (97, 127, 3, 1.0, 200, 0, "rows", 24), (33, 31, 7, 1.0, 0, 0, "random", 8), (33, 31, 7, 1.0, 40, 0, "rows", 32),
+         (127, 65, 2, 0.1, 0, 3000, "random", 32), (365, 373, 1, 0.5, 0, 0, "random", 32),
          (511, 525, 1, 0.5, 60, 0, "rows", 24), (525, 509, 1, 0.5, 0, 0, "random", 32)]
 
 

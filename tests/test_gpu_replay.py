@@ -16,7 +16,8 @@ from test_gpu_ordered import COMPS, _config, _lattice  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny,order,dtype,shuffled", [(63, 47, 2, 2, False), (61, 63, 1, 2, True), (127, 129, 3, 0, True)])
+@pytest.mark.parametrize("nx,ny,order,dtype,shuffled", [
+    (63, 47, 2, 2, False), (61, 63, 1, 2, True), (127, 129, 3, 0, True)])
 def test_depositions_replayed(nx, ny, order, dtype, shuffled):
     from hipace2_amd.simulation import Simulation
     from oracle.oracle import OracleSim
